@@ -574,8 +574,8 @@ __device__ __forceinline__ int circle(int pos, int r, int N) {
 // division by the runtime size.
 // Sweeps until a sweep's rotations pass the loose stop of rotation() (the
 // outputs are fp32: eigenvalues good to ~1e-8 relative, eigenvectors of
-// separated eigenvalues to ~1e-8).
-__device__ void lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_flag) {
+// separated eigenvalues to ~1e-8).  Returns the power of two H was scaled by.
+__device__ double lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_flag) {
   __shared__ double rc[kL / 2], rs[kL / 2];
   __shared__ int pp[kL / 2], qq[kL / 2];
   const int tid = threadIdx.x;
@@ -583,20 +583,26 @@ __device__ void lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_
   double (*Hc)[kLP] = H;
   for (int e = tid; e < np * np; e += 256) J[e / np][e % np] = (e / np == e % np) ? 1.0 : 0.0;
   __syncthreads();
-  // H is positive semidefinite (a Gram matrix): ||H||_F <= trace(H)
+  // H is positive semidefinite (a Gram matrix): ||H||_F <= trace(H); scaled to
+  // a trace of order one (rotation() relies on it)
   double tr = 0.0;
   for (int i = 0; i < np; ++i) tr += fabs(Hc[i][i]);
-  const double flo = 4.0 * 2.220446049250313e-16 * tr;
+  const double sc = unit_scale(tr);
+  const float flo = (float)(4.0 * 2.220446049250313e-16 * tr * sc);
+  const RotStop stop = rot_stop(true);
+  __syncthreads();
+  for (int e = tid; e < np * np; e += 256) Hc[e / np][e % np] *= sc;
+  __syncthreads();
   for (int sweep = 0; sweep < 40; ++sweep) {
     if (tid == 0) *sig_flag = 0;
     __syncthreads();
-    int sig = 0;
+    bool sig = false;
     for (int t = 0; t < np - 1; ++t) {
       if (tid < half) {
         const int p = circle(tid, t, np), q = circle(np - 1 - tid, t, np);
         double c, sn;
-        int sg;
-        rotation(Hc[p][p], Hc[q][q], Hc[p][q], flo, &c, &sn, &sg);
+        bool sg;
+        rotation(Hc[p][p], Hc[q][q], Hc[p][q], flo, stop, &c, &sn, &sg);
         rc[tid] = c;
         rs[tid] = sn;
         pp[tid] = p;
@@ -614,9 +620,10 @@ __device__ void lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_
         const double h00 = Hc[pi][pj], h01 = Hc[pi][qj], h10 = Hc[qi][pj], h11 = Hc[qi][qj];
         const double x00 = cj * h00 - sj * h01, x01 = sj * h00 + cj * h01;
         const double x10 = cj * h10 - sj * h11, x11 = sj * h10 + cj * h11;
-        double y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
-        double y10 = si * x00 + ci * x10, y11 = si * x01 + ci * x11;
-        if (bi == bj && si != 0.0) y01 = y10 = 0.0;
+        const double y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
+        double y10 = si * x00 + ci * x10;
+        const double y11 = si * x01 + ci * x11;
+        if (bi == bj) y10 = y01;  // the diagonal blocks stay exactly symmetric
         Hc[pi][pj] = y00;
         Hc[pi][qj] = y01;
         Hc[qi][pj] = y10;
@@ -634,13 +641,14 @@ __device__ void lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_
       }
       __syncthreads();
     }
-    if (sig & 2) atomicOr(sig_flag, 1);
+    if (sig) *sig_flag = 1;
     __syncthreads();
     const int any = *sig_flag;
     __syncthreads();
     if (!any) break;
   }
   __syncthreads();
+  return sc;
 }
 
 __global__ void __launch_bounds__(256, 3)
@@ -665,7 +673,7 @@ bfinal_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
     for (int e = tid; e < np; e += 256) H[l][e] = H[e][l] = 0.0;
   }
   __syncthreads();
-  lds_jacobi(H, J, np, &flag);
+  const double sc = lds_jacobi(H, J, np, &flag);  // H: sc times the eigenvalues
   // ascending order of the l real eigenvalues: rank by counting
   if (tid < l) {
     // NaN ranks as +Inf, ties by index: the ranks are a permutation
@@ -681,7 +689,8 @@ bfinal_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
   // the last k in ascending order: output j <- eigenpair order[l - k + j]
   if (tid < k) {
     const int e = order[l - k + tid];
-    const double s = H[e][e] < 0.0 ? 0.0 : sqrt(H[e][e]);  // NaN stays NaN
+    const double lam = H[e][e] / sc;
+    const double s = lam < 0.0 ? 0.0 : sqrt(lam);  // NaN stays NaN
     sig[tid] = s;
     S[d.s + tid] = s;
   }

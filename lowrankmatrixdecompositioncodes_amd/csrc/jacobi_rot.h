@@ -31,8 +31,7 @@ constexpr double kStopTol = 1e-10;
 constexpr double kLooseStopTol = 1e-4;
 constexpr double kLooseRatioTol = 1e-8;
 
-// 1/x and 1/sqrt(x) from the hardware estimates plus two Newton steps
-// (error a few ulp; a rotation only needs c^2 + s^2 = 1 to rounding).
+// 1/x from the hardware estimate plus two Newton steps (error a few ulp).
 static __device__ __forceinline__ double rcp_nr(double x) {
   double y = __builtin_amdgcn_rcp(x);
   double e = fma(-x, y, 1.0);
@@ -40,47 +39,65 @@ static __device__ __forceinline__ double rcp_nr(double x) {
   e = fma(-x, y, 1.0);
   return fma(y, e, y);
 }
-static __device__ __forceinline__ double rsq_nr(double x) {
-  double y = __builtin_amdgcn_rsq(x);
-  const double h = 0.5 * x;
-  double e = fma(-h * y, y, 0.5);
-  y = fma(y, e, y);
-  e = fma(-h * y, y, 0.5);
-  return fma(y, e, y);
+// The power of two that brings x > 0 to [1/2, 1); 1 for zero, NaN and Inf.
+static __device__ __forceinline__ double unit_scale(double x) {
+  if (!(x > 0.0) || isinf(x)) return 1.0;
+  int e;
+  (void)frexp(x, &e);
+  // a power of two beyond the largest double is not needed: 2^-1022 times
+  // 2^1022 is of order one already
+  return ldexp(1.0, -e > 1022 ? 1022 : -e);
+}
+
+// The same from a squared Frobenius norm, and 0 when the square left the range
+// in which it tells (the caller then scales by the largest entry).
+static __device__ __forceinline__ double norm_scale(double fro2) {
+  return (fro2 > 1e-280 && fro2 < 1e280) ? unit_scale(sqrt(fro2)) : 0.0;
+}
+
+// Which rotations keep the iteration going (see kStopTol, kLooseStopTol): those
+// with |g| > ratio sqrt|ab| and |t| > angle.
+struct RotStop {
+  float ratio2, angle;
+};
+static __host__ __device__ __forceinline__ RotStop rot_stop(bool loose) {
+  return loose ? RotStop{(float)(kLooseRatioTol * kLooseRatioTol), (float)kLooseStopTol}
+               : RotStop{(float)(kStopTol * kStopTol), -1.0f};
 }
 
 // Rotation (c, s) with [x' y'] = [x y] [[c, s], [-s, c]] zeroing the (p, q)
-// entry of a symmetric 2x2 [[a, g], [g, b]]: t = tan theta is the root of
-// g t^2 + (b - a) t - g = 0 of smaller modulus, t = sgn(d) 2g / (|d| + r),
-// d = b - a, r = sqrt(d^2 + 4g^2) (Rutishauser's choice).  With den = |d| + r,
-// 1 + t^2 = 2r / den, so c = 1 / sqrt(1 + t^2) = den / sqrt(2 r den) and
-// s = c t = sgn(d) 2g / sqrt(2 r den): two reciprocal square roots on the
-// serial path and c^2 + s^2 = (den^2 + 4g^2) / (2 r den) = 1 identically.
-// Evaluated on the entries scaled by a power of two so that the squares stay
-// in range.  Branch-free.  No rotation when |g| <= flo or |g| <= kRotTol
-// sqrt|ab|; *sig bit 0 reports |g| > kStopTol sqrt|ab|, bit 1 a rotation
-// with |s| > kLooseStopTol and |g| > kLooseRatioTol sqrt|ab| (bit 1 implies
-// bit 0).
-static __device__ __forceinline__ void rotation(double a, double b, double g, double flo, double* cs,
-                                         double* sn, int* sig) {
-  const double ag = fabs(g);
-  int e;
-  (void)frexp(fmax(fmax(fabs(a), fabs(b)), ag), &e);
-  const double sa = ldexp(a, -e), sb = ldexp(b, -e), sg = ldexp(g, -e);
-  const double ab = fabs(sa * sb), g2 = sg * sg;
-  const bool big = ag > flo;
-  const bool rot = big & (g2 > kRotTol * kRotTol * ab);
-  const double d = sb - sa;
-  const double r2 = rot ? fma(d, d, 4.0 * g2) : 1.0;
-  const double r = r2 * rsq_nr(r2);
-  const double den = fabs(d) + r;
-  const double q = rsq_nr(2.0 * r * den);
-  const double t2g = (d < 0.0) ? -2.0 * sg : 2.0 * sg;
-  *cs = rot ? den * q : 1.0;
-  *sn = rot ? t2g * q : 0.0;
-  *sig = ((big & (g2 > kStopTol * kStopTol * ab)) ? 1 : 0) |
-         ((rot & (fabs(*sn) > kLooseStopTol) & (g2 > kLooseRatioTol * kLooseRatioTol * ab)) ? 2
-                                                                                           : 0);
+// entry of a symmetric 2x2 [[a, g], [g, b]] of a matrix scaled to norm 1
+// (unit_scale): t = tan theta is the root of g t^2 + (b - a) t - g = 0 of
+// smaller modulus, t = sgn(d) 2g / (|d| + r), d = b - a, r = sqrt(d^2 + 4g^2)
+// (Rutishauser's choice).  The angle only has to be close: t is formed in
+// single precision (relative error below 1e-6, so a rotation leaves less than
+// 1e-6 of its off-diagonal, which the caller's update computes like any other
+// entry); everything above flo (1e-15 of the norm) keeps its square in range.
+// That (c, s) is a rotation to rounding is what orthogonality rests on:
+// c = 1 / sqrt(1 + t^2) in double precision from the single precision estimate
+// and one third-order step (error below 1e-20 before rounding), s = c t.
+// Branch-free.  No rotation when |g| <= flo or |g| <= kRotTol sqrt|ab|; *sig
+// tells whether the rotation counts for `stop`.
+// What bounds a rotation step is the issue of its instructions (a wave issues
+// one every four cycles and has its SIMD to itself): this form has 35, two
+// reciprocal square roots in double precision with two Newton steps each, the
+// scaling of each triple and the tests in double precision had about 80.
+static __device__ __forceinline__ void rotation(double a, double b, double g, float flo,
+                                                RotStop stop, double* cs, double* sn, bool* sig) {
+  const double d = b - a;
+  const float af = (float)a, bf = (float)b, gf = (float)g, df = (float)d;
+  const float ab = fabsf(af * bf), g2 = gf * gf;
+  const float r = __builtin_amdgcn_sqrtf(fmaf(df, df, 4.0f * g2));
+  const float q = (gf + gf) * __builtin_amdgcn_rcpf(fabsf(df) + r);
+  const bool rot = (fabsf(gf) > flo) & (g2 > (float)(kRotTol * kRotTol) * ab);
+  const float t = rot ? copysignf(1.0f, df) * q : 0.0f;
+  const double td = (double)t, x = fma(td, td, 1.0);
+  const double y = (double)__builtin_amdgcn_rsqf(fmaf(t, t, 1.0f));
+  const double e = fma(-x * y, y, 1.0);
+  const double c = fma(y * e, fma(0.375, e, 0.5), y);
+  *cs = c;
+  *sn = c * td;
+  *sig = rot & (g2 > stop.ratio2 * ab) & (fabsf(t) > stop.angle);
 }
 
 }  // namespace rsvd

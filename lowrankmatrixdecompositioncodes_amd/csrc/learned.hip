@@ -312,8 +312,7 @@ int sketch_features(Context* c, const double* A, const float* A32, int64_t m, in
   RSVD_TRY(gemm_f64(c, 'T', 'N', k, n, m, 1.0, Y64.p, m, A, lda, 0.0, B.p, k));
   RSVD_TRY(gemm_f64(c, 'N', 'T', k, k, n, 1.0, B.p, k, B.p, k, 0.0, G.p, k));
   RSVD_TRY(symmetrize_upper_f64(c, k, G.p));
-  int sw = 0;
-  RSVD_TRY(symeig_jacobi_f64(c, k, G.p, k, nullptr, k, lam.p, 60, &sw, 1));
+  RSVD_TRY(symeig_jacobi_f64(c, k, G.p, k, nullptr, k, lam.p, 60, nullptr, 1));
   RSVD_TRY(sort_pairs_f64(c, k, lam.p, 1, nullptr, 0, 0, nullptr, 0, 0));
   RSVD_TRY(sumsq_f64(c, m, n, A, lda, a2.p));
   hipLaunchKernelGGL(sketch_features_kernel, dim3(1), dim3(64), 0, c->stream,

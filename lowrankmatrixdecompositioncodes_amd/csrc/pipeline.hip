@@ -109,7 +109,7 @@ int svd_from_Q_f64(Context* c, const double* A, int64_t m, int64_t n, int64_t ld
   hipLaunchKernelGGL(symmetrize_upper_kernel, dim3(grid1(l * l)), dim3(256), 0, c->stream, l, G.p);
   RSVD_LAUNCH_CHECK();
   int sw = 0;
-  RSVD_TRY(symeig_jacobi_f64(c, l, G.p, l, Uh.p, l, lam.p, 60, &sw));
+  RSVD_TRY(symeig_jacobi_f64(c, l, G.p, l, Uh.p, l, lam.p, 60, info ? &sw : nullptr));
   RSVD_TRY(sort_pairs_f64(c, l, lam.p, 0, Uh.p, l, l, nullptr, 0, 0));
   hipLaunchKernelGGL(sqrt_kernel, dim3(grid1(l)), dim3(256), 0, c->stream, l,
                      (const double*)lam.p, sig.p);

@@ -341,9 +341,9 @@ int mlp_train(Context* c, float* theta, const float* X, const int* q, const floa
 int sketch_features(Context* c, const double* A, const float* A32, int64_t m, int64_t n,
                     int64_t lda, uint64_t seed, float* feat);
 // Symmetric eigensolver (two-sided block Jacobi).  G (n x n, ld ldg, both
-// triangles, symmetric) is diagonalised in place: on return G ~ diag(lambda)
-// and V (optional, n x n) holds the eigenvectors (V^T G_in V = diag);
-// evals (optional) = diag(G), unsorted.  *sweeps_out = sweeps used.  The
+// triangles, symmetric) is used up; V (optional, n x n) holds the eigenvectors
+// (V^T G V = diag) and evals (optional) the eigenvalues, both unsorted.
+// *sweeps_out (optional; reading it waits for the solve) = sweeps used.  The
 // iteration ends after the first sweep whose rotations were all below 1e-10
 // of sqrt(g_pp g_qq), or 1e-4 with loose = 1 (eigenvectors to fp32 level).
 int symeig_jacobi_f64(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t ldv,

@@ -35,7 +35,9 @@ namespace {
 
 
 __device__ __forceinline__ int player(int pos, int r, int N) {
-  return pos == 0 ? 0 : 1 + ((pos - 1 + r) % (N - 1));
+  int x = pos - 1 + r;  // 0 <= r < N - 1
+  x = x >= N - 1 ? x - (N - 1) : x;
+  return pos == 0 ? 0 : 1 + x;
 }
 
 // The columns of block pair w in round r: slot s (0..2B-1) is column
@@ -61,50 +63,60 @@ __device__ __forceinline__ int64_t pair_col(int w, int s, int r, int N, int nblo
   return PairCols<B>(w, r, N, nblocks, n).col(s);
 }
 
-// Local pairing of step t of the inner sweep.  Round 0 of a sweep runs the
-// full cyclic sweep of the 2B columns (S - 1 steps, every pair once, within
-// and across the two blocks); the other rounds only meet the B x B cross pairs
-// (B steps: local column k of block a with B + (k + t) mod B of block b) --
-// the pairs inside one block were already met in round 0.  Every pair of
-// columns still meets once per sweep, and the inner steps per sweep fall from
-// about 2n to about n.
-template <int B>
-__device__ __forceinline__ void local_pair(int k, int t, bool cross, int* p, int* q) {
-  constexpr int S = 2 * B;
-  if (cross) {
-    *p = k;
-    *q = B + (k + t) % B;
-  } else {
-    *p = player(k, t, S);
-    *q = player(S - 1 - k, t, S);
-  }
-}
+// The inner sweep.  Round 0 of a sweep meets every pair of its 2B columns: first
+// the pairs inside each of the two blocks (B - 1 steps, jac_within), then the
+// B x B cross pairs (B steps, jac_cross); the other rounds only the cross pairs.
+// Every pair of columns meets once per sweep, and the inner steps per sweep are
+// about n instead of 2n.
 
-// The inner sweep of one block pair on its S x S tile (S = 2B), in LDS: H in
-// Ha (double-buffered with Hb), J accumulated in Jl (row-major, padded HP).
-// A step: thread t = (bi, bj) (bi = t / B, bj = t % B) computes the rotation
-// of local pair bj (the 16 lanes of each row of a wave compute the 16
-// rotations), takes that of pair bi from the lane of its row that computed it
-// (a cross-lane read, no LDS round trip and no extra barrier), applies
-// R_bi^T . R_bj to the 2 x 2 block of H at (pair bi rows, pair bj columns) --
-// the blocks partition H -- and R_bi to rows 2 bj, 2 bj + 1 of J's columns of
-// pair bi.  One barrier per step.  Returns the buffer holding the final H.
-template <int B, bool CROSS>
-__device__ double* jac_inner_t(double* Ha, double* Hb, double* Jl, double flo, int* any_sig) {
+// A 64-bit value moved inside each 16-lane row of the wave (a data-parallel
+// move, no trip through the LDS crossbar): CTRL 0x150 (row_newbcast:0) gives
+// every lane lane 0's, 0x12f (row_ror:15) the next lane's, 0x121 (row_ror:1) the
+// previous lane's, both cyclically.
+template <int CTRL>
+__device__ __forceinline__ double row_move(double v) {
+  union {
+    double d;
+    int i[2];
+  } u = {v};
+  u.i[0] = __builtin_amdgcn_mov_dpp(u.i[0], CTRL, 0xf, 0xf, true);
+  u.i[1] = __builtin_amdgcn_mov_dpp(u.i[1], CTRL, 0xf, 0xf, true);
+  return u.d;
+}
+__device__ __forceinline__ double row_first(double v) { return row_move<0x150>(v); }
+__device__ __forceinline__ double row_next(double v) { return row_move<0x12f>(v); }
+__device__ __forceinline__ double row_prev(double v) { return row_move<0x121>(v); }
+
+// The pairs inside the two blocks of the S x S tile (S = 2B) in LDS, H in Ha
+// (double-buffered with Hb), J accumulated in Jl (row-major, padded HP): step m
+// rotates column i against i xor m in both blocks.  Thread (bi, x) (bi = t / B,
+// x = t % B) computes the rotation of pair bj = (bi + x) mod B -- the 16 lanes of
+// a row of a wave compute the 16 rotations, its lane 0 that of pair bi, which
+// the row takes from there -- applies R_bi^T . R_bj to the 2 x 2 block of H at
+// (pair bi rows, pair bj columns) -- the blocks partition H -- and R_bi to rows
+// 2 x, 2 x + 1 of J's columns of pair bi.  One barrier per step.  Returns the
+// buffer holding the final H; *any_sig |= a rotation of the lane's counted.
+template <int B>
+__device__ double* jac_within(double* Ha, double* Hb, double* Jl, float flo, RotStop stop,
+                              bool* any_sig) {
   constexpr int S = 2 * B, HP = S + 1;
-  static_assert(B == 16, "a row of 16 lanes holds the B rotations of a step");
   const int tid = threadIdx.x;
-  const int bi = tid / B, bj = tid % B;
-  const int src = (tid & 48) | bi;  // lane of this row that owns pair bi
+  const int bi = tid / B, x = tid % B, bj = (bi + x) % B;
   double* Hc = Ha;
   double* Hn = Hb;
-  int sig = 0;
-  constexpr int steps = CROSS ? B : S - 1;
-  for (int t = 0; t < steps; ++t) {
+  // pair k of step m: the (k mod B/2)-th i without m's top bit, in block k / (B/2)
+  auto pair = [](int k, int m, int top, int* p, int* q) {
+    const int h = k & (B / 2 - 1), lo = h & (top - 1);
+    const int i = 2 * (h - lo) + lo, base = (k / (B / 2)) * B;
+    *p = base + i;
+    *q = base + (i ^ m);
+  };
+  for (int m = 1; m < B; ++m) {
+    const int top = 1 << (31 - __builtin_clz(m));
     int pi, qi, pj, qj;
-    local_pair<B>(bi, t, CROSS, &pi, &qi);
-    local_pair<B>(bj, t, CROSS, &pj, &qj);
-    const int x0 = 2 * bj;
+    pair(bi, m, top, &pi, &qi);
+    pair(bj, m, top, &pj, &qj);
+    const int x0 = 2 * x;
     // every LDS read of the step first, so that one latency covers them
     const double aj = Hc[pj * HP + pj], bbj = Hc[qj * HP + qj], gj = Hc[pj * HP + qj];
     const double h00 = Hc[pi * HP + pj], h01 = Hc[pi * HP + qj];
@@ -112,20 +124,20 @@ __device__ double* jac_inner_t(double* Ha, double* Hb, double* Jl, double flo, i
     const double j00 = Jl[x0 * HP + pi], j01 = Jl[x0 * HP + qi];
     const double j10 = Jl[(x0 + 1) * HP + pi], j11 = Jl[(x0 + 1) * HP + qi];
     double cj, sj;
-    int sgj;
-    rotation(aj, bbj, gj, flo, &cj, &sj, &sgj);
-    sig |= sgj;
-    const double ci = __shfl(cj, src, 64), si = __shfl(sj, src, 64);
+    bool sgj;
+    rotation(aj, bbj, gj, flo, stop, &cj, &sj, &sgj);
+    *any_sig |= sgj;
+    const double ci = row_first(cj), si = row_first(sj);
     // X = H_blk R_j, then R_i^T X
     const double x00 = cj * h00 - sj * h01, x01 = sj * h00 + cj * h01;
     const double x10 = cj * h10 - sj * h11, x11 = sj * h10 + cj * h11;
-    double y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
-    double y10 = si * x00 + ci * x10, y11 = si * x01 + ci * x11;
-    if (bi == bj && si != 0.0) y01 = y10 = 0.0;  // the annihilated pair
-    Hn[pi * HP + pj] = y00;
+    const double y01 = ci * x01 - si * x11;
+    double y10 = si * x00 + ci * x10;
+    if (x == 0) y10 = y01;  // a diagonal block stays exactly symmetric
+    Hn[pi * HP + pj] = ci * x00 - si * x10;
     Hn[pi * HP + qj] = y01;
     Hn[qi * HP + pj] = y10;
-    Hn[qi * HP + qj] = y11;
+    Hn[qi * HP + qj] = si * x01 + ci * x11;
     Jl[x0 * HP + pi] = ci * j00 - si * j01;
     Jl[x0 * HP + qi] = si * j00 + ci * j01;
     Jl[(x0 + 1) * HP + pi] = ci * j10 - si * j11;
@@ -135,46 +147,107 @@ __device__ double* jac_inner_t(double* Ha, double* Hb, double* Jl, double flo, i
     Hc = Hn;
     Hn = tmp;
   }
-  *any_sig = sig;
   return Hc;
 }
 
-template <int B>
-__device__ double* jac_inner(double* Ha, double* Hb, double* Jl, bool cross, double flo,
-                             int* any_sig) {
-  return cross ? jac_inner_t<B, true>(Ha, Hb, Jl, flo, any_sig)
-               : jac_inner_t<B, false>(Ha, Hb, Jl, flo, any_sig);
-}
+// The cross pairs: step t rotates column p_k = k of block a against column
+// q_k = (k + t) mod B of block b.  Thread (bi, x) keeps the 2 x 2 block of H at
+// (pair bi rows, pair bj columns), bj = (bi + x) mod B, and rows 2 bi, 2 bi + 1 of
+// J's columns of pair bj in registers.  From a step to the next p stays and q
+// moves by one pair, so H(p, p) and J(p) stay, H(p, q) and J(q) come from the next
+// lane of the row (a data-parallel move), and only H(q, p) and H(q, q) cross rows:
+// they go through LDS (E), with the entries of the next rotations (R and E's
+// diagonal).  One barrier per step (E and R double-buffered).  After B steps every
+// entry is back where it started.  E: 2 B B pairs, R: 2 B pairs (LDS).
+// What bounds a step is LDS traffic and latency: with H and J in LDS (19
+// accesses a thread and step instead of 5) a step took 1195 cycles, here 800.
+typedef double d2_t __attribute__((ext_vector_type(2)));
 
-// J and the final tile H of pair w out (column-major S x S each); the flag
-// collects the rotation-size bits of rotation() (bit 0: above kStopTol, bit
-// 1: a rotation the loose stop counts).
 template <int B>
-__device__ void jac_out(const double* Hf, const double* Jl, int w, double* __restrict__ Jout,
-                        double* __restrict__ Hout, int any_sig,
-                        unsigned long long* __restrict__ flag) {
+__device__ void jac_cross(const double* H, const double* Jl, d2_t* E, d2_t* R, float flo,
+                          RotStop stop, bool* any_sig, double* __restrict__ Jw,
+                          double* __restrict__ Hw) {
+  static_assert(B == 16, "a row of 16 lanes holds the B rotations of a step");
   constexpr int S = 2 * B, HP = S + 1;
   const int tid = threadIdx.x;
-  double* __restrict__ Jw = Jout + (size_t)w * S * S;
-  double* __restrict__ Hw = Hout + (size_t)w * S * S;
-  for (int e = tid; e < S * S; e += 256) {
-    const int i = e % S, j = e / S;
-    Jw[i + j * S] = Jl[i * HP + j];
-    Hw[i + j * S] = Hf[i * HP + j];
+  const int bi = tid / B, x = tid % B, bj = (bi + x) % B, r0 = 2 * bi;
+  double h00 = H[bi * HP + bj], h01 = H[bi * HP + B + bj];
+  double h10 = H[(B + bi) * HP + bj], h11 = H[(B + bi) * HP + B + bj];
+  double a = H[bj * HP + bj], b = H[(B + bj) * HP + B + bj], g = H[bj * HP + B + bj];
+  double jp0 = Jl[r0 * HP + bj], jq0 = Jl[r0 * HP + B + bj];
+  double jp1 = Jl[(r0 + 1) * HP + bj], jq1 = Jl[(r0 + 1) * HP + B + bj];
+  const int up = (tid + B) % (B * B);              // the same lane of pair bi + 1's row
+  const int dj = ((bj + 1) % B) * B;               // lane 0 of pair bj + 1's row
+  bool sig = false;
+#pragma unroll 2
+  for (int t = 0; t < B; ++t) {
+    d2_t* Et = E + (t & 1) * B * B;
+    d2_t* Rt = R + (t & 1) * B;
+    double c, s;
+    bool sg;
+    rotation(a, b, g, flo, stop, &c, &s, &sg);
+    sig |= sg;
+    const double ci = row_first(c), si = row_first(s);
+    // X = H_blk R_j, then R_i^T X
+    const double x00 = c * h00 - s * h01, x01 = s * h00 + c * h01;
+    const double x10 = c * h10 - s * h11, x11 = s * h10 + c * h11;
+    const double y01 = ci * x01 - si * x11, y11 = si * x01 + ci * x11;
+    double y10 = si * x00 + ci * x10;
+    if (x == 0) y10 = y01;  // a diagonal block stays exactly symmetric
+    h00 = ci * x00 - si * x10;
+    h01 = row_next(y01);
+    Et[tid] = d2_t{row_prev(y10), y11};
+    if (x == 0) Rt[bi] = d2_t{h00, h01};
+    const double n0 = s * jp0 + c * jq0, n1 = s * jp1 + c * jq1;
+    jp0 = c * jp0 - s * jq0;
+    jp1 = c * jp1 - s * jq1;
+    jq0 = row_next(n0);
+    jq1 = row_next(n1);
+    __syncthreads();
+    const d2_t e = Et[up], r = Rt[bj];
+    b = Et[dj][1];
+    h10 = e[0];
+    h11 = e[1];
+    a = r[0];
+    g = r[1];
   }
-  const unsigned long long m =
-      (__any(any_sig & 1) ? 1ULL : 0ULL) | (__any(any_sig & 2) ? 2ULL : 0ULL);
-  if (m && (tid & 63) == 0) atomicOr(flag, m);
+  *any_sig |= sig;
+  Jw[r0 * S + bj] = jp0;
+  Jw[r0 * S + B + bj] = jq0;
+  Jw[(r0 + 1) * S + bj] = jp1;
+  Jw[(r0 + 1) * S + B + bj] = jq1;
+  Hw[bi * S + bj] = h00;
+  Hw[bi * S + B + bj] = h01;
+  Hw[(B + bi) * S + bj] = h10;
+  Hw[(B + bi) * S + B + bj] = h11;
+}
+
+// The whole inner sweep of pair w; J and the final tile out (row-major S x S
+// each).  Ha holds the tile, Jl the identity; Hb is scratch.  The flag is set
+// when a rotation counted for the stop.
+template <int B>
+__device__ void jac_solve(double* Ha, double* Hb, double* Jl, d2_t* R, bool cross, float flo,
+                          RotStop stop, int w, double* __restrict__ Jout,
+                          double* __restrict__ Hout, unsigned long long* __restrict__ flag) {
+  constexpr int S = 2 * B, HP = S + 1;
+  static_assert(2 * B * B * sizeof(d2_t) <= S * HP * sizeof(double), "E fits a tile's region");
+  bool sig = false;
+  double* Hc = cross ? Ha : jac_within<B>(Ha, Hb, Jl, flo, stop, &sig);
+  d2_t* E = reinterpret_cast<d2_t*>(Hc == Ha ? Hb : Ha);
+  jac_cross<B>(Hc, Jl, E, R, flo, stop, &sig, Jout + (size_t)w * S * S, Hout + (size_t)w * S * S);
+  if (__any(sig) && (threadIdx.x & 63) == 0) atomicOr(flag, 1ULL);
 }
 
 // First round of the iteration: the pair tiles are read from G.
 template <int B>
 __global__ void __launch_bounds__(256)
 symj_solve_kernel(int64_t n, const double* __restrict__ G, int64_t ldg, int nblocks, int N,
-                  int round, const double* __restrict__ fro2, double* __restrict__ Jout,
-                  double* __restrict__ Hout, unsigned long long* __restrict__ flag) {
+                  int round, const double* __restrict__ scal, RotStop stop,
+                  double* __restrict__ Jout, double* __restrict__ Hout,
+                  unsigned long long* __restrict__ flag) {
   constexpr int S = 2 * B, HP = S + 1;
-  __shared__ double Ha[S * HP], Hb[S * HP], Jl[S * HP];
+  __shared__ __align__(16) double Ha[S * HP], Hb[S * HP], Jl[S * HP];
+  __shared__ d2_t R[2 * B];
   __shared__ int64_t cols[S];
   const int w = blockIdx.x;
   const int tid = threadIdx.x;
@@ -186,11 +259,9 @@ symj_solve_kernel(int64_t n, const double* __restrict__ G, int64_t ldg, int nblo
     Ha[i * HP + j] = (ci >= 0 && cj >= 0) ? G[ci + cj * ldg] : 0.0;
     Jl[i * HP + j] = (i == j) ? 1.0 : 0.0;
   }
-  const double flo = 4.0 * 2.220446049250313e-16 * sqrt(*fro2);
+  const float flo = (float)scal[0];
   __syncthreads();
-  int sig = 0;
-  const double* Hf = jac_inner<B>(Ha, Hb, Jl, round > 0, flo, &sig);
-  jac_out<B>(Hf, Jl, w, Jout, Hout, sig, flag);
+  jac_solve<B>(Ha, Hb, Jl, R, round > 0, flo, stop, w, Jout, Hout, flag);
 }
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
@@ -266,7 +337,8 @@ __device__ void jac_apply(int bid, int64_t n, const double* __restrict__ Gin,
     const PairCols<B> pa(w1, round, N, nblocks, n), pb(w2, round, N, nblocks, n);
     const double* J1 = Jall + (size_t)w1 * S * S;
     const double* J2 = Jall + (size_t)w2 * S * S;
-    // thread: row r of the tile, columns c0 + 8 it
+    // thread: row r of the tile, columns c0 + 8 it; column r of the J, rows
+    // c0 + 8 it
     const int r = tid % S, c0 = tid / S;
     const int64_t gr = pa.col(r);
     double tv[4], av[4], bv[4];
@@ -276,15 +348,15 @@ __device__ void jac_apply(int bid, int64_t n, const double* __restrict__ Gin,
       const int64_t gc = pb.col(c);
       const double g = Gin[(gr < 0 ? 0 : gr) + (gc < 0 ? 0 : gc) * ldg];
       tv[it] = (gr >= 0 && gc >= 0) ? g : 0.0;
-      av[it] = J1[r + c * S];
-      bv[it] = J2[r + c * S];
+      av[it] = J1[c * S + r];
+      bv[it] = J2[c * S + r];
     }
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int c = c0 + 8 * it;
       T[r * HP + c] = tv[it];
-      Ja[r * HP + c] = av[it];
-      Jb[r * HP + c] = bv[it];
+      Ja[c * HP + r] = av[it];
+      Jb[c * HP + r] = bv[it];
     }
     if (skip) return;
     __syncthreads();
@@ -318,7 +390,7 @@ __device__ void jac_apply(int bid, int64_t n, const double* __restrict__ Gin,
   if (V == nullptr) return;
   // V strip: rows [r0, r0 + 2S) of the pair's columns, in two S-row halves
   // (T and X).  Thread: row r of the strip, columns cq + 4 it; J_w element
-  // (tid % S, tid / S + 8 it).
+  // (tid / S + 8 it, tid % S).
   bid -= ntg;
   const int w = bid % pairs;
   const int64_t r0 = (int64_t)(bid / pairs) * (2 * S);
@@ -335,12 +407,12 @@ __device__ void jac_apply(int bid, int64_t n, const double* __restrict__ Gin,
   }
   const int jr = tid % S, jc0 = tid / S;
 #pragma unroll
-  for (int it = 0; it < 4; ++it) jv[it] = Jw[jr + (jc0 + 8 * it) * S];
+  for (int it = 0; it < 4; ++it) jv[it] = Jw[(jc0 + 8 * it) * S + jr];
   double* Vh = r < S ? T + r * HP : X + (r - S) * HP;  // this thread's row of the strip
 #pragma unroll
   for (int it = 0; it < 8; ++it) Vh[cq + 4 * it] = vv[it];
 #pragma unroll
-  for (int it = 0; it < 4; ++it) Jb[jr * HP + jc0 + 8 * it] = jv[it];
+  for (int it = 0; it < 4; ++it) Jb[(jc0 + 8 * it) * HP + jr] = jv[it];
   if (skip) return;
   __syncthreads();
   const d4_t o1 = tile_mfma<false>(T, Jb), o2 = tile_mfma<false>(X, Jb);
@@ -369,11 +441,11 @@ template <int B>
 __global__ void __launch_bounds__(256)
 symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__ Gout,
                  int64_t ldg, double* __restrict__ V, int64_t ldv, int nblocks, int N, int round,
-                 int round1, int nsolve, const double* __restrict__ fro2,
+                 int round1, int nsolve, const double* __restrict__ scal, RotStop stop,
                  const double* __restrict__ Jin, const double* __restrict__ Hin,
                  double* __restrict__ Jout, double* __restrict__ Hout, int ntg,
                  unsigned long long* __restrict__ flag,
-                 const unsigned long long* __restrict__ prev, unsigned long long mask) {
+                 const unsigned long long* __restrict__ prev) {
   constexpr int S = 2 * B, HP = S + 1, BP = B + 1;
   // Device-side stop: every launch of a sweep reads the previous sweep's
   // rotation flags (complete: that sweep's launches have finished) and does
@@ -381,14 +453,14 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
   // it has read the last one's flags.  Read here and tested after the other
   // global reads are issued (before any global write), so one memory latency
   // covers them all.
-  const unsigned long long pv = prev ? *prev : mask;
-  const bool skip = (pv & mask) == 0;
+  const bool skip = prev && *prev == 0;
   // Apply role: four S x HP regions T, Ja, Jb, X.  Solve role: Ha, Jl and
   // Tab (later Hb) S x HP each, then JBq, X3 and JAq S x BP each; no region
   // changes tenant before the inner sweep.  Both footprints let four
   // workgroups share a CU.
   constexpr int kSm = (4 * S * HP > 3 * S * HP + 3 * S * BP) ? 4 * S * HP : 3 * S * HP + 3 * S * BP;
-  __shared__ double sm[kSm];
+  __shared__ __align__(16) double sm[kSm];
+  __shared__ d2_t R[2 * B];
   const int tid = threadIdx.x;
   if ((int)blockIdx.x >= nsolve) {
     jac_apply<B>((int)blockIdx.x - nsolve, n, Gin, Gout, ldg, V, ldv, nblocks, N, round, Jin, ntg,
@@ -406,7 +478,8 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
   // the blocks of pair w in round1 and where they sat in round r
   const int xa = player(w, round1, N), xb = player(N - 1 - w, round1, N);
   auto locate = [&](int x, int* wp, int* h) {
-    const int pos = (x == 0) ? 0 : 1 + (((x - 1 - round) % (N - 1)) + (N - 1)) % (N - 1);
+    const int y = x - 1 - round;
+    const int pos = (x == 0) ? 0 : 1 + (y < 0 ? y + N - 1 : y);
     if (pos < N / 2) {
       *wp = pos;
       *h = 0;
@@ -423,8 +496,9 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
   const double* JB = Jin + (size_t)wb * S * S;
   const double* HA = Hin + (size_t)wa * S * S;
   const double* HB = Hin + (size_t)wb * S * S;
-  // every global read first: thread row i of Tab (columns j0 + 8 it), of JAq
-  // and JBq (columns j0 + 8 it), and entry (dc, dd) of the two diagonal blocks
+  // every global read first: thread row i of Tab (columns j0 + 8 it), rows
+  // dd + B it of JAq and JBq (column dc), and entry (dd, dc) of the two diagonal
+  // blocks
   const int i = tid % S, j0 = tid / S;
   const int dc = tid % B, dd = tid / B;
   const int64_t gi = pa.col(i);
@@ -438,15 +512,15 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
   }
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
-    av[it] = JA[i + (ha * B + j0 + 8 * it) * S];
-    bv[it] = JB[i + (hb * B + j0 + 8 * it) * S];
+    av[it] = JA[(dd + B * it) * S + ha * B + dc];
+    bv[it] = JB[(dd + B * it) * S + hb * B + dc];
   }
-  const double hav = HA[(ha * B + dc) + (ha * B + dd) * S];
-  const double hbv = HB[(hb * B + dc) + (hb * B + dd) * S];
+  const double hav = HA[(ha * B + dd) * S + ha * B + dc];
+  const double hbv = HB[(hb * B + dd) * S + hb * B + dc];
   // the rotation floor goes through LDS: its load then completes with the
   // others instead of being deferred to its first use in the inner sweep
-  __shared__ double flo_s;
-  if (tid == 0) flo_s = 4.0 * 2.220446049250313e-16 * sqrt(*fro2);
+  __shared__ float flo_s;
+  if (tid == 0) flo_s = (float)scal[0];
   // J starts as the identity (its region has no other tenant)
 #pragma unroll
   for (int it = 0; it < 4; ++it) Jl[i * HP + j0 + 8 * it] = (i == j0 + 8 * it) ? 1.0 : 0.0;
@@ -454,12 +528,12 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
   for (int it = 0; it < 4; ++it) Tab[i * HP + j0 + 8 * it] = tv[it];
 #pragma unroll
   for (int it = 0; it < 2; ++it) {
-    JAq[i * BP + j0 + 8 * it] = av[it];
-    JBq[i * BP + j0 + 8 * it] = bv[it];
+    JAq[(dd + B * it) * BP + dc] = av[it];
+    JBq[(dd + B * it) * BP + dc] = bv[it];
   }
   // diagonal blocks of the new tile from round r's final tiles
-  Ha[dc * HP + dd] = hav;
-  Ha[(B + dc) * HP + B + dd] = hbv;
+  Ha[dd * HP + dc] = hav;
+  Ha[(B + dd) * HP + B + dc] = hbv;
   // the skip test after the LDS stores, so that no global read waits for it
   if (skip) return;
   __syncthreads();
@@ -479,48 +553,223 @@ symj_step_kernel(int64_t n, const double* __restrict__ Gin, double* __restrict__
     }
   }
   __syncthreads();
-  const double flo = flo_s;
-  int sig = 0;
-  const double* Hf = jac_inner<B>(Ha, Hb, Jl, round1 > 0, flo, &sig);
-  jac_out<B>(Hf, Jl, w, Jout, Hout, sig, flag);
+  jac_solve<B>(Ha, Hb, Jl, R, round1 > 0, flo_s, stop, w, Jout, Hout, flag);
 }
 
-__global__ void symj_identity_kernel(int64_t n, double* __restrict__ V, int64_t ldv) {
+// Gs = sc G with sc the power of two of unit_scale (so that no rotation has to
+// scale its entries), V = I, the sweeps' flags cleared, scal = {rotation floor,
+// 1 / sc}.  fro2: ||G||_F^2; where that over- or underflowed every workgroup
+// finds the largest entry for itself.
+__global__ void __launch_bounds__(256)
+symj_prep_kernel(int64_t n, const double* __restrict__ G, int64_t ldg, double* __restrict__ Gs,
+                 double* __restrict__ V, int64_t ldv, const double* __restrict__ fro2,
+                 double* __restrict__ scal, unsigned long long* __restrict__ flags, int nflags) {
+  __shared__ double red[256];
   const int64_t total = n * n;
-  for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
+  double sc = norm_scale(*fro2), fro = sqrt(*fro2) * sc;
+  if (sc == 0.0) {
+    double mx = 0.0;
+    for (int64_t idx = threadIdx.x; idx < total; idx += 256)
+      mx = fmax(mx, fabs(G[idx % n + (idx / n) * ldg]));
+    red[threadIdx.x] = mx;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if ((int)threadIdx.x < w) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + w]);
+      __syncthreads();
+    }
+    sc = unit_scale(red[0]);
+    fro = 1.0;
+  }
+  for (int64_t idx = blockIdx.x * (int64_t)256 + threadIdx.x; idx < total;
+       idx += (int64_t)gridDim.x * 256) {
     const int64_t i = idx % n, j = idx / n;
-    V[i + j * ldv] = (i == j) ? 1.0 : 0.0;
+    Gs[i + j * ldg] = sc * G[i + j * ldg];
+    if (V) V[i + j * ldv] = (i == j) ? 1.0 : 0.0;
+  }
+  if (blockIdx.x == 0) {
+    for (int e = threadIdx.x; e < nflags; e += 256) flags[e] = 0;
+    if (threadIdx.x == 0) {
+      scal[0] = 4.0 * 2.220446049250313e-16 * fro;
+      scal[1] = 1.0 / sc;
+    }
   }
 }
 
 __global__ void symj_diag_kernel(int64_t n, const double* __restrict__ G, int64_t ldg,
-                                 double* __restrict__ d) {
+                                 const double* __restrict__ scal, double* __restrict__ d) {
   const int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (j < n) d[j] = G[j + j * ldg];
+  if (j < n) d[j] = G[j + j * ldg] * scal[1];
+}
+
+// The whole iteration for n <= kSmallN in one workgroup: G (upper triangle) and
+// V live in LDS, a step is one rotation of every pair of the round-robin order.
+// The block solver is launch- and latency-bound at these sizes (a round of one
+// block pair takes as long as one of seventeen): a whole call at n = 26 took
+// 0.39 ms with it and 0.19 ms here, at n = 40 0.66 and 0.32 ms.  A step's LDS
+// traffic, all of H and V, grows as n^2 and there are n steps: at n = 64 this
+// kernel takes 0.72 ms, more than the block solver's three rounds a sweep.
+// Per step: wave 0 computes the rotations while the other waves apply the
+// previous step's to V; after a barrier every thread applies the step's to its
+// 2 x 2 block of H (pairs bi <= bj; entry (i, j) is kept at row min, column max).
+constexpr int kSmallN = 48, kSmallThreads = 1024, kSmallLd = kSmallN + 1;
+
+__device__ __forceinline__ double& upper(double* H, int i, int j) {
+  return i < j ? H[i * kSmallLd + j] : H[j * kSmallLd + i];
+}
+
+__global__ void __launch_bounds__(kSmallThreads)
+symj_small_kernel(int n, const double* __restrict__ G, int64_t ldg, double* __restrict__ V, int64_t ldv,
+                  double* __restrict__ evals, int max_sweeps, RotStop stop,
+                  int* __restrict__ sweeps) {
+  __shared__ double H[kSmallN * kSmallLd], J[kSmallN * kSmallLd];
+  __shared__ double rc[2][kSmallN / 2], rs[2][kSmallN / 2];
+  __shared__ int pp[2][kSmallN / 2], qq[2][kSmallN / 2];
+  __shared__ double red[kSmallThreads / 64];
+  __shared__ int sig_s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int np = n + (n & 1), half = np / 2;
+  double ss = 0.0;
+  for (int e = tid; e < np * kSmallN; e += kSmallThreads) {
+    const int i = e % kSmallN, j = e / kSmallN;
+    const double v = (i < n && j < n) ? G[i + j * ldg] : 0.0;
+    if (i >= np) continue;
+    if (i <= j) H[i * kSmallLd + j] = v;
+    J[i * kSmallLd + j] = (i == j) ? 1.0 : 0.0;
+    if (i <= j) ss += (i < j ? 2.0 : 1.0) * v * v;
+  }
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  if (lane == 0) red[wave] = ss;
+  __syncthreads();
+  double fro2 = 0.0;
+  for (int w = 0; w < kSmallThreads / 64; ++w) fro2 += red[w];
+  double sc = norm_scale(fro2), fro = sqrt(fro2) * sc;
+  if (sc == 0.0) {  // the squares over- or underflowed: scale by the largest entry
+    double mx = 0.0;
+    for (int e = lane; e < np * np; e += 64) mx = fmax(mx, fabs(upper(H, e % np, e / np)));
+    for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 64));
+    sc = unit_scale(mx);
+    fro = 1.0;
+    __syncthreads();  // every wave has read the unscaled entries
+  }
+  const float flo = (float)(4.0 * 2.220446049250313e-16 * fro);
+  for (int e = tid; e < np * kSmallN; e += kSmallThreads) {
+    const int i = e % kSmallN, j = e / kSmallN;
+    if (i <= j) H[i * kSmallLd + j] *= sc;
+  }
+  __syncthreads();
+  // this thread's block (bi, bj) of the upper triangle of pairs, row by row
+  const int nblk = half * (half + 1) / 2;
+  int bi = 0, bj = tid;
+  if (tid < nblk) {
+    while (bj >= half - bi) {
+      bj -= half - bi;
+      ++bi;
+    }
+    bj += bi;
+  }
+  auto rotate_v = [&](int buf, int first, int stride) {
+    if (lane >= np) return;
+    for (int k = first; k < half; k += stride) {
+      const double c = rc[buf][k], s = rs[buf][k];
+      const int p = pp[buf][k], q = qq[buf][k];
+      const double x = J[lane * kSmallLd + p], y = J[lane * kSmallLd + q];
+      J[lane * kSmallLd + p] = c * x - s * y;
+      J[lane * kSmallLd + q] = s * x + c * y;
+    }
+  };
+  int buf = 0, sweep = 0;
+  bool pending = false;  // the previous step's rotations are not in V yet
+  while (sweep < max_sweeps && np > 1) {
+    bool sig = false;
+    for (int t = 0; t < np - 1; ++t) {
+      if (wave == 0) {
+        if (lane < half) {
+          auto pos = [&](int x) {
+            int y = x - 1 + t;
+            y = y >= np - 1 ? y - (np - 1) : y;
+            return x == 0 ? 0 : 1 + y;
+          };
+          const int p = pos(lane), q = pos(np - 1 - lane);
+          double c, s;
+          bool sg;
+          rotation(H[p * kSmallLd + p], H[q * kSmallLd + q], upper(H, p, q), flo, stop, &c, &s,
+                   &sg);
+          rc[buf][lane] = c;
+          rs[buf][lane] = s;
+          pp[buf][lane] = p;
+          qq[buf][lane] = q;
+          sig |= sg;
+        }
+      } else if (V && pending) {
+        rotate_v(buf ^ 1, wave - 1, kSmallThreads / 64 - 1);
+      }
+      __syncthreads();
+      if (tid < nblk) {
+        const int pi = pp[buf][bi], qi = qq[buf][bi], pj = pp[buf][bj], qj = qq[buf][bj];
+        const double ci = rc[buf][bi], si = rs[buf][bi], cj = rc[buf][bj], sj = rs[buf][bj];
+        double &e00 = upper(H, pi, pj), &e01 = upper(H, pi, qj), &e10 = upper(H, qi, pj),
+               &e11 = upper(H, qi, qj);
+        const double h00 = e00, h01 = e01, h10 = e10, h11 = e11;
+        const double x00 = cj * h00 - sj * h01, x01 = sj * h00 + cj * h01;
+        const double x10 = cj * h10 - sj * h11, x11 = sj * h10 + cj * h11;
+        e00 = ci * x00 - si * x10;
+        e01 = ci * x01 - si * x11;  // a diagonal block: the same entry as e10
+        if (bi != bj) e10 = si * x00 + ci * x10;
+        e11 = si * x01 + ci * x11;
+      }
+      __syncthreads();
+      buf ^= 1;
+      pending = true;
+    }
+    if (tid == 0) sig_s = 0;
+    __syncthreads();
+    if (sig) sig_s = 1;
+    __syncthreads();
+    ++sweep;
+    if (sig_s == 0) break;
+    __syncthreads();
+  }
+  if (V && pending) rotate_v(buf ^ 1, wave, kSmallThreads / 64);
+  __syncthreads();
+  for (int e = tid; e < n * kSmallN; e += kSmallThreads) {
+    const int i = e % kSmallN, j = e / kSmallN;
+    if (i >= n) continue;
+    if (V) V[i + j * ldv] = J[i * kSmallLd + j];
+    if (evals && i == j) evals[i] = H[i * kSmallLd + i] / sc;
+  }
+  if (tid == 0 && sweeps) *sweeps = sweep;
 }
 
 template <int B>
 int run_sweeps(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t ldv,
-               int max_sweeps, int loose, int* sweep_out) {
+               double* evals, int max_sweeps, int loose, int* sweep_out) {
   constexpr int S = 2 * B;
   const int nblocks = (int)((n + B - 1) / B);
   const int N = nblocks + (nblocks & 1);
   const int pairs = N / 2;
   const int ntg = pairs * (pairs + 1) / 2;
   const int ntv = V ? pairs * (int)((n + 2 * S - 1) / (2 * S)) : 0;
-  DBuf<double> G2, Jb, Hb, fro2;
+  const RotStop stop = rot_stop(loose);
+  DBuf<double> G2, Jb, Hb, fro2, scal;
   DBuf<unsigned long long> flags;
   const size_t js = (size_t)pairs * S * S;
   RSVD_TRY(G2.alloc((size_t)(ldg * n)));
   RSVD_TRY(Jb.alloc(2 * js));
   RSVD_TRY(Hb.alloc(2 * js));
   RSVD_TRY(fro2.alloc(1));
+  RSVD_TRY(scal.alloc(2));
   RSVD_TRY(flags.alloc((size_t)max_sweeps + 2));
   RSVD_TRY(sumsq_f64(c, n, n, G, ldg, fro2.p));
-  RSVD_HIP(hipMemsetAsync(flags.p, 0, sizeof(unsigned long long) * (max_sweeps + 2), c->stream));
-  double* cur = G;
-  double* nxt = G2.p;
+  {
+    int blocks = (int)((n * n + 255) / 256);
+    if (blocks > 2048) blocks = 2048;
+    hipLaunchKernelGGL(symj_prep_kernel, dim3(blocks), dim3(256), 0, c->stream, n,
+                       (const double*)G, ldg, G2.p, V, ldv, (const double*)fro2.p, scal.p, flags.p,
+                       max_sweeps + 2);
+    RSVD_LAUNCH_CHECK();
+  }
+  double* cur = G2.p;
+  double* nxt = G;
   int jc = 0;
   int sweep = 0;
   KTimer kt(c, "symeig");
@@ -528,15 +777,14 @@ int run_sweeps(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t
     // round 0 of sweep 0 from G itself; afterwards every launch applies
     // round r and solves the next round
     hipLaunchKernelGGL(symj_solve_kernel<B>, dim3(pairs), dim3(256), 0, c->stream, n,
-                       (const double*)G, ldg, nblocks, N, 0, (const double*)fro2.p, Jb.p, Hb.p,
-                       flags.p);
+                       (const double*)cur, ldg, nblocks, N, 0, (const double*)scal.p, stop, Jb.p,
+                       Hb.p, flags.p);
     RSVD_LAUNCH_CHECK();
     // The first launches of sweep s are queued before the host looks at
     // sweep s - 1's flags (copied to pinned memory behind sweep s - 1 and
     // waited for while those launches run); when s - 1 converged they return
     // at once (the device-side stop above), the rest of the sweep is never
     // queued, and the state is the one sweep s started from.
-    const unsigned long long mask = loose ? 2ULL : 1ULL;
     constexpr int kAhead = 4;  // launches of sweep s queued before the wait
     volatile unsigned long long* slot = static_cast<unsigned long long*>(c->pinned);
     hipEvent_t ev[2] = {nullptr, nullptr};
@@ -554,9 +802,9 @@ int run_sweeps(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t
         unsigned long long* fl = flags.p + (wrap ? sweep + 1 : sweep);
         hipLaunchKernelGGL(symj_step_kernel<B>, dim3(pairs + ntg + ntv), dim3(256), 0, c->stream,
                            n, (const double*)cur, nxt, ldg, V, ldv, nblocks, N, r, r1, pairs,
-                           (const double*)fro2.p, (const double*)(Jb.p + jc * js),
+                           (const double*)scal.p, stop, (const double*)(Jb.p + jc * js),
                            (const double*)(Hb.p + jc * js), Jb.p + (1 - jc) * js,
-                           Hb.p + (1 - jc) * js, ntg, fl, prev, mask);
+                           Hb.p + (1 - jc) * js, ntg, fl, prev);
         if (hipGetLastError() != hipSuccess) {
           rc = set_error("symeig: step launch failed");
           break;
@@ -572,9 +820,9 @@ int run_sweeps(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t
             rc = set_error("symeig: flag wait failed");
             break;
           }
-          // no pair met in sweep - 1 was above kStopTol (or counted by the
-          // loose stop): this sweep's launches did nothing
-          if ((slot[(sweep - 1) & 1] & mask) == 0) {
+          // no rotation of sweep - 1 counted for the stop: this sweep's
+          // launches did nothing
+          if (slot[(sweep - 1) & 1] == 0) {
             cur = cur0;
             jc = jc0;
             done = true;
@@ -594,9 +842,11 @@ int run_sweeps(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t
     (void)hipEventDestroy(ev[1]);
     if (rc) return rc;
   }
-  if (cur != G)
-    RSVD_HIP(hipMemcpy2DAsync(G, ldg * sizeof(double), cur, ldg * sizeof(double),
-                              n * sizeof(double), n, hipMemcpyDeviceToDevice, c->stream));
+  if (evals) {
+    hipLaunchKernelGGL(symj_diag_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+                       c->stream, n, (const double*)cur, ldg, (const double*)scal.p, evals);
+    RSVD_LAUNCH_CHECK();
+  }
   *sweep_out = sweep;
   return 0;
 }
@@ -608,22 +858,22 @@ int symeig_jacobi_f64(Context* c, int64_t n, double* G, int64_t ldg, double* V, 
   if (sweeps_out) *sweeps_out = 0;
   if (n <= 0) return 0;
   if (ldg < n || (V && ldv < n)) return set_error("symeig: leading dimension < n");
-  if (V) {
-    int blocks = (int)((n * n + 255) / 256);
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(symj_identity_kernel, dim3(blocks), dim3(256), 0, c->stream, n, V, ldv);
-    RSVD_LAUNCH_CHECK();
+  if (n <= kSmallN) {
+    DBuf<int> sw;
+    if (sweeps_out) RSVD_TRY(sw.alloc(1));
+    {
+      KTimer kt(c, "symeig");
+      hipLaunchKernelGGL(symj_small_kernel, dim3(1), dim3(kSmallThreads), 0, c->stream, (int)n, 
+                         (const double*)G, ldg, V, ldv, evals, max_sweeps, rot_stop(loose), sw.p);
+      RSVD_LAUNCH_CHECK();
+    }
+    if (sweeps_out) RSVD_TRY(read_small(c, sweeps_out, sw.p, sizeof(int)));
+    return 0;
   }
   int sweep = 0;
-  // B = 16: each thread owns one 2x2 block and computes two rotations per
+  // B = 16: each thread owns one 2x2 block and computes one rotation per
   // step; a larger B trades launches for a slower, LDS-bound inner sweep
-  const int rc = run_sweeps<16>(c, n, G, ldg, V, ldv, max_sweeps, loose, &sweep);
-  if (rc) return rc;
-  if (evals) {
-    hipLaunchKernelGGL(symj_diag_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       c->stream, n, (const double*)G, ldg, evals);
-    RSVD_LAUNCH_CHECK();
-  }
+  RSVD_TRY(run_sweeps<16>(c, n, G, ldg, V, ldv, evals, max_sweeps, loose, &sweep));
   if (sweeps_out) *sweeps_out = sweep;
   return 0;
 }
