@@ -348,6 +348,9 @@ int sketch_features(Context* c, const double* A, const float* A32, int64_t m, in
 // of sqrt(g_pp g_qq), or 1e-4 with loose = 1 (eigenvectors to fp32 level).
 int symeig_jacobi_f64(Context* c, int64_t n, double* G, int64_t ldg, double* V, int64_t ldv,
                       double* evals, int max_sweeps, int* sweeps_out, int loose = 0);
+// The eigenvalues alone of a symmetric G (n x n, n <= 64, upper triangle
+// used), descending.
+int symeig_values_f64(Context* c, int64_t n, const double* G, int64_t ldg, double* evals);
 // Column norms of W into nrm[n]; optional normalisation of the columns.
 int colnorms_f64(Context* c, int64_t L, int64_t n, double* W, int64_t ldw, double* nrm,
                  int normalise);
