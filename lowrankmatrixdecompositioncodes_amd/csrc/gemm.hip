@@ -3,23 +3,38 @@
 // deflation A -= Qp*Bp, U = Q*Uhat, ...), replacing the cblas_dgemm calls of
 // MKL/mvf.c:538-561.
 //
-// Tiling: a 256-thread workgroup (4 waves, 2x2) owns a BM x BN tile of C and
-// walks K in BK slices staged through LDS.  Each wave owns a (BM/2) x (BN/2)
-// sub-tile built from 16x16 MFMA blocks (v_mfma_f64_16x16x4f64 or
-// v_mfma_f32_16x16x4f32).  The MFMA "A" operand is fed from op(B) and the "B"
-// operand from op(A), so the accumulator lanes run along M: 16 consecutive
-// lanes hold 16 consecutive rows of one column of C and the epilogue writes
-// whole 128-byte (f64) segments of column-major C.
-//
+// A 16x16x4 FP64 MFMA holds its SIMD for 64 cycles and needs 1 KB of operands,
+// so no two waves need to share them: every wave runs on its own, without a
+// barrier in the k loop, with the next k block's loads in flight behind the
+// current block's products.  A k block is one 128-byte line of a k-contiguous
+// row (16 FP64 or 32 FP32 elements).  The k index inside a block is permuted so
+// that a lane's loads are 16 bytes wide: MFMA step s multiplies the elements
+// kmap(g, s) of the lane groups g = lane / 16 (any order of k serves, as long as
+// both operands use it).
+//  * An operand stored row-contiguous is loaded into registers in MFMA lane
+//    order, 16 lanes covering 32 rows of one k; its rows are dealt to the 16-row
+//    blocks in pairs (row 2 (lane % 16) + (b & 1) of a 32-row group belongs to
+//    block b), the same for both operands and the stores of C.
+//  * An operand stored k-contiguous is loaded eight full lines a time and
+//    transposed to lane order through a region of LDS of the wave's own
+//    (loaded in lane order it would take 16 half lines a load: 50 TF against
+//    61 TF for A^T B at 6000 x 288 x 16384).
+// Measured (FP64, best cut; the former kernel staged 128 x 64 tiles through one
+// LDS buffer with two barriers a slice): 16384 x 288 x 6000 N N 49 -> 67 TF,
+// A^T B as above 35 -> 61 TF, 2000 x 110 x 1000 39 -> 15 us, a 110 x 110 Gram of
+// 2000 rows 40 -> 9 us.  The large ones are bound by the MFMAs (71 TF at the
+// clock a large product reaches), the small ones by latency.
 // Operand lane layout of the 16x16x4 MFMAs (per 64-lane wave):
 //   srcA: lane l holds X[i = l%16][k = l/16]
 //   srcB: lane l holds Y[k = l/16][j = l%16]
 //   dst : lane l, register r holds D[i][j = l%16] with
 //         i = 4*(l/16) + r   for v_mfma_f32_16x16x4f32
 //         i = 4*r + l/16     for v_mfma_f64_16x16x4f64
-// Long-K products with few output tiles are split along K into a workspace
-// and summed in a fixed order by a second kernel (deterministic).
+// srcA is fed from op(B) and srcB from op(A), so accumulator lanes run along M
+// and the epilogue writes contiguous segments of column-major C.
+#include <algorithm>
 #include <climits>
+#include <type_traits>
 
 #include <rocblas/rocblas.h>
 
@@ -35,6 +50,12 @@ struct Mfma;
 template <>
 struct Mfma<double> {
   typedef d4_t acc_t;
+  // two elements, and the k-contiguous elements of one load (16 bytes), at
+  // their natural alignment (the hardware's wide global accesses need four
+  // bytes)
+  typedef double v2_t __attribute__((ext_vector_type(2), aligned(8)));
+  typedef v2_t vk_t;
+  typedef double vl_t __attribute__((ext_vector_type(2)));  // the same in LDS
   static __device__ __forceinline__ acc_t mma(double a, double b, acc_t c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
@@ -44,6 +65,9 @@ struct Mfma<double> {
 template <>
 struct Mfma<float> {
   typedef f4_t acc_t;
+  typedef float v2_t __attribute__((ext_vector_type(2), aligned(4)));
+  typedef float vk_t __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float vl_t __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ acc_t mma(float a, float b, acc_t c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
   }
@@ -51,30 +75,172 @@ struct Mfma<float> {
 };
 
 constexpr int kThreads = 256;
+// Depth of a k block, MFMA steps of a block, elements of a 16-byte load.
+template <typename T>
+struct KBlock {
+  static constexpr int kDepth = 128 / sizeof(T);
+  static constexpr int kSteps = kDepth / 4;
+  static constexpr int kVec = 16 / sizeof(T);
+  // element of the k block that lane group g multiplies in MFMA step s
+  static __device__ __forceinline__ int kmap(int g, int s) {
+    return kVec * (g + 4 * (s / kVec)) + s % kVec;
+  }
+};
 
-// C[z] = alpha * op(A)[:, kslice z] * op(B)[kslice z, :] + beta * C
-// When sumsq != nullptr, each workgroup writes the sum of squares of the values
-// it stored into sumsq[tm + gridDim.x*tn] for its tile (tm, tn) (double).
-template <typename T, bool TA, bool TB, int BM, int BN, int BK>
-__global__ void __launch_bounds__(kThreads)
-gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk, T alpha, const T* __restrict__ A,
-            int64_t lda, const T* __restrict__ B, int64_t ldb, T beta, T* __restrict__ C,
-            int64_t ldc, int64_t zstride, double* __restrict__ sumsq, int sym) {
-  constexpr int PAD = 4;
-  constexpr int WM = BM / 2, WN = BN / 2;
-  constexpr int TM = WM / 16, TN = WN / 16;
-  constexpr int EA = BM * BK / kThreads;
-  constexpr int EB = BN * BK / kThreads;
-  static_assert(EA * kThreads == BM * BK && EB * kThreads == BN * BK, "tile/threads");
-  __shared__ T As[BK][BM + PAD];
-  __shared__ T Bs[BK][BN + PAD];
+// row of a wave's 16-row block b held by index x (0..15)
+__device__ __forceinline__ int block_row(int b, int x) { return 32 * (b >> 1) + 2 * x + (b & 1); }
 
+// One operand of a wave: TT 16-row blocks of op(X) from row r0, `lim` rows in
+// all (rows past the end read the last row; their products are not stored).
+// KC: element (row, k) at X[k + row ld] (k-contiguous), else X[row + k ld].
+// A block is loaded into raw registers (load) and read from them in lane order
+// (frags).
+template <typename T, bool KC, int TT>
+struct Operand;
+
+template <typename T, int TT>
+struct Operand<T, false, TT> {
+  typedef typename Mfma<T>::v2_t v2_t;
+  static constexpr int SS = KBlock<T>::kSteps;
+  static constexpr int kLds = 0;
+  struct Raw {
+    T f[TT][SS];
+  };
+  const T* X;
+  int64_t ld, r0, last;
+  bool full;  // every row of the wave's blocks is valid
+  __device__ __forceinline__ Operand(const T* X_, int64_t ld_, int64_t r, int64_t lim, char*)
+      : X(X_), ld(ld_), r0(r), last(lim - 1), full(r + 16 * TT <= lim) {}
+  // FULL: every row valid; TAIL: zero where k >= kend
+  template <bool FULL, bool TAIL>
+  __device__ __forceinline__ void load(int64_t k0, int64_t kend, Raw& w) const {
+    const int li = threadIdx.x & 15, lk = (threadIdx.x & 63) >> 4;
+#pragma unroll
+    for (int s = 0; s < SS; ++s) {
+      const int64_t k = k0 + KBlock<T>::kmap(lk, s);
+      const bool ok = !TAIL || k < kend;
+      const T* p = X + (ok ? k : kend - 1) * ld;
+#pragma unroll
+      for (int b = 0; b < TT; b += 2) {
+        const int64_t r = r0 + block_row(b, li);
+        if constexpr (FULL) {
+          const v2_t v = *reinterpret_cast<const v2_t*>(p + r);
+          w.f[b][s] = ok ? v[0] : T(0);
+          w.f[b + 1][s] = ok ? v[1] : T(0);
+        } else {
+          const T v0 = p[r < last ? r : last], v1 = p[r + 1 < last ? r + 1 : last];
+          w.f[b][s] = ok ? v0 : T(0);
+          w.f[b + 1][s] = ok ? v1 : T(0);
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ void frags(const Raw& w, T (&f)[TT][SS]) const {
+#pragma unroll
+    for (int b = 0; b < TT; ++b)
+#pragma unroll
+      for (int s = 0; s < SS; ++s) f[b][s] = w.f[b][s];
+  }
+};
+
+// Load j takes rows 8 j + lane / 8, 16-byte chunk lane % 8 of each row's line.
+// In LDS row r keeps its chunk c at position c ^ ((r / 2) % 8): the sixteen
+// rows 2 x (or 2 x + 1) that a frag read takes at equal c spread over the banks.
+template <typename T, int TT>
+struct Operand<T, true, TT> {
+  static constexpr int SS = KBlock<T>::kSteps, VK = KBlock<T>::kVec;
+  static constexpr int kLds = TT * 16 * 128;  // bytes of the wave's region
+  typedef typename Mfma<T>::vk_t vk_t;
+  struct Raw {
+    vk_t v[2 * TT];
+  };
+  const T* X;
+  int64_t ld, r0, last;
+  bool full;
+  char* lds;
+  __device__ __forceinline__ Operand(const T* X_, int64_t ld_, int64_t r, int64_t lim, char* lds_)
+      : X(X_), ld(ld_), r0(r), last(lim - 1), full(r + 16 * TT <= lim), lds(lds_) {}
+  template <bool FULL, bool TAIL>
+  __device__ __forceinline__ void load(int64_t k0, int64_t kend, Raw& w) const {
+    const int lane = threadIdx.x & 63;
+    const int64_t k = k0 + VK * (lane & 7);
+#pragma unroll
+    for (int j = 0; j < 2 * TT; ++j) {
+      const int64_t r = r0 + 8 * j + (lane >> 3);
+      const T* p = X + (FULL || r < last ? r : last) * ld + k;
+      if constexpr (!TAIL) {
+        w.v[j] = *reinterpret_cast<const vk_t*>(p);
+      } else {
+#pragma unroll
+        for (int e = 0; e < VK; ++e) w.v[j][e] = (k + e < kend) ? p[e] : T(0);
+      }
+    }
+  }
+  __device__ __forceinline__ void frags(const Raw& w, T (&f)[TT][SS]) const {
+    const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+    // one wave's LDS operations complete in order; the fences keep the
+    // compiler from moving the reads over the writes or the next block's
+    // writes over these reads
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int j = 0; j < 2 * TT; ++j) {
+      const int r = 8 * j + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+      *reinterpret_cast<typename Mfma<T>::vl_t*>(lds + r * 128 + 16 * c) = w.v[j];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int b = 0; b < TT; ++b) {
+      const int r = block_row(b, li);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int c = (lk + 4 * q) ^ ((r >> 1) & 7);
+        const auto v = *reinterpret_cast<const typename Mfma<T>::vl_t*>(lds + r * 128 + 16 * c);
+#pragma unroll
+        for (int e = 0; e < VK; ++e) f[b][VK * q + e] = v[e];
+      }
+    }
+  }
+};
+
+// Arguments of a launch: C = alpha op(A) op(B) + beta C, M x N, inner K in
+// slices of kchunk (a multiple of the k block), slice z into C + z zstride.
+template <typename T>
+struct GemmArgs {
+  int64_t M, N, K, kchunk;
+  T alpha;
+  const T* A;
+  int64_t lda;
+  const T* B;
+  int64_t ldb;
+  T beta;
+  T* C;
+  int64_t ldc, zstride;
+  double* sumsq;  // optional: per-workgroup sums of squares of the stored C
+  int sym;        // Gram: form the entries on and above the diagonal only
+  int mirror;     // sym: store each also below the diagonal
+  int gx, gy;     // tiles
+};
+
+// Row tiles of column tile tn with an entry on or above the diagonal.
+__host__ __device__ __forceinline__ int64_t sym_tiles(int64_t tn, int64_t gx, int64_t bm,
+                                                      int64_t bn) {
+  const int64_t up = ((tn + 1) * bn + bm - 1) / bm;
+  return up < gx ? up : gx;
+}
+
+// A workgroup (four waves) owns a (16 TM WM) x (16 TN WN) tile of C; KS = 4 /
+// (WM WN) waves share a wave tile and deal its k blocks among them, their
+// partial tiles added in wave order through LDS at the end.
+template <typename T, bool TA, bool TB, int TM, int TN, int WM, int WN>
+__global__ void __launch_bounds__(kThreads, 2)
+gemm_kernel(const GemmArgs<T> g) {
+  constexpr int KS = 4 / (WM * WN);
+  constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
   typedef typename Mfma<T>::acc_t acc_t;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm0 = (wave & 1) * WM;
-  const int wn0 = (wave >> 1) * WN;
+  typedef typename Mfma<T>::v2_t v2_t;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  const int ks = wave / (WM * WN), wt = wave % (WM * WN);
   // Tile order.  Workgroups are handed to the 8 XCDs round-robin by
   // dispatch order (b % 8), each XCD with its own L2: XCD x takes a
   // contiguous run of tiles, walked with the dimension that has fewer tiles
@@ -83,11 +249,15 @@ gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk, T alpha, const T* _
   // side and A leaves HBM once instead of once per column tile).
   int64_t tm, tn;
   {
-    const int64_t gx = gridDim.x, gy = gridDim.y, nt = gx * gy;
-    const int64_t b = blockIdx.x + gx * (int64_t)blockIdx.y;
+    const int64_t gx = g.gx, gy = g.gy, nt = gridDim.x;
+    const int64_t b = blockIdx.x;
     const int64_t xcd = b & 7, j = b >> 3, q = nt >> 3, r = nt & 7;
     const int64_t t = xcd * q + (xcd < r ? xcd : r) + j;
-    if (gy <= gx) {
+    if (g.sym) {
+      // a Gram: the tiles of column tn that reach the diagonal, column by column
+      tm = t;
+      for (tn = 0; tm >= sym_tiles(tn, gx, BM, BN); ++tn) tm -= sym_tiles(tn, gx, BM, BN);
+    } else if (gy <= gx) {
       tn = t % gy;
       tm = t / gy;
     } else {
@@ -95,13 +265,11 @@ gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk, T alpha, const T* _
       tn = t / gx;
     }
   }
-  const int64_t m0 = tm * BM;
-  const int64_t n0 = tn * BN;
-  // a Gram (sym): tiles wholly below the diagonal are mirrored afterwards
-  if (sym && m0 >= n0 + BN) return;
-  const int64_t kbeg = (int64_t)blockIdx.z * kchunk;
-  const int64_t kend = (kbeg + kchunk < K) ? kbeg + kchunk : K;
-  T* Cz = C + (int64_t)blockIdx.z * zstride;
+  const int64_t m0 = tm * BM + (wt % WM) * 16 * TM;
+  const int64_t n0 = tn * BN + (wt / WM) * 16 * TN;
+  const int64_t kbeg = (int64_t)blockIdx.y * g.kchunk;
+  const int64_t kend = (kbeg + g.kchunk < g.K) ? kbeg + g.kchunk : g.K;
+  T* __restrict__ C = g.C + (int64_t)blockIdx.y * g.zstride;
 
   acc_t acc[TN][TM];
 #pragma unroll
@@ -109,93 +277,137 @@ gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk, T alpha, const T* _
 #pragma unroll
     for (int b = 0; b < TM; ++b) acc[a][b] = acc_t{0, 0, 0, 0};
 
-  T ra[EA], rb[EB];
-  auto load_tiles = [&](int64_t k0) {
-#pragma unroll
-    for (int e = 0; e < EA; ++e) {
-      int idx = tid + kThreads * e;
-      int mm, kk;
-      if (!TA) { mm = idx % BM; kk = idx / BM; }
-      else { kk = idx % BK; mm = idx / BK; }
-      int64_t gm = m0 + mm, gk = k0 + kk;
-      T v = T(0);
-      if (gm < M && gk < kend) v = TA ? A[gk + gm * lda] : A[gm + gk * lda];
-      ra[e] = v;
-    }
-#pragma unroll
-    for (int e = 0; e < EB; ++e) {
-      int idx = tid + kThreads * e;
-      int nn, kk;
-      if (!TB) { kk = idx % BK; nn = idx / BK; }
-      else { nn = idx % BN; kk = idx / BN; }
-      int64_t gn = n0 + nn, gk = k0 + kk;
-      T v = T(0);
-      if (gn < N && gk < kend) v = TB ? B[gn + gk * ldb] : B[gk + gn * ldb];
-      rb[e] = v;
-    }
-  };
-  auto store_tiles = [&]() {
-#pragma unroll
-    for (int e = 0; e < EA; ++e) {
-      int idx = tid + kThreads * e;
-      int mm, kk;
-      if (!TA) { mm = idx % BM; kk = idx / BM; }
-      else { kk = idx % BK; mm = idx / BK; }
-      As[kk][mm] = ra[e];
-    }
-#pragma unroll
-    for (int e = 0; e < EB; ++e) {
-      int idx = tid + kThreads * e;
-      int nn, kk;
-      if (!TB) { kk = idx % BK; nn = idx / BK; }
-      else { nn = idx % BN; kk = idx / BN; }
-      Bs[kk][nn] = rb[e];
-    }
-  };
+  // the waves' transposition regions, then their partial tiles
+  typedef Operand<T, TA, TM> OpA;
+  typedef Operand<T, !TB, TN> OpB;
+  constexpr int kStage = 4 * (OpA::kLds + OpB::kLds);
+  constexpr int kPart = KS > 1 ? KS * TN * TM * 4 * 64 * (int)sizeof(T) : 0;
+  constexpr int kSm = kStage > kPart ? kStage : kPart;
+  __shared__ __align__(16) char sm[kSm > 0 ? kSm : 16];
 
-  const int li = lane & 15;
-  const int lk = lane >> 4;
-  if (kbeg < kend) load_tiles(kbeg);
-  for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
-    __syncthreads();
-    store_tiles();
-    __syncthreads();
-    if (k0 + BK < kend) load_tiles(k0 + BK);
+  const bool live = m0 < g.M && n0 < g.N;
+  if (live) {
+    constexpr int KD = KBlock<T>::kDepth, SS = KBlock<T>::kSteps;
+    char* ws = sm + wave * (OpA::kLds + OpB::kLds);
+    const OpA oa(g.A, g.lda, m0, g.M, ws);
+    const OpB ob(g.B, g.ldb, n0, g.N, ws + OpA::kLds);
+    typename OpA::Raw a0, a1;
+    typename OpB::Raw b0, b1;
+    T fa[TM][SS], fb[TN][SS];
+    auto mma = [&]() {
 #pragma unroll
-    for (int ks = 0; ks < BK / 4; ++ks) {
-      const int kr = ks * 4 + lk;
-      T av[TN], bv[TM];
+      for (int s = 0; s < SS; ++s)
 #pragma unroll
-      for (int a = 0; a < TN; ++a) av[a] = Bs[kr][wn0 + a * 16 + li];
+        for (int a = 0; a < TN; ++a)
 #pragma unroll
-      for (int b = 0; b < TM; ++b) bv[b] = As[kr][wm0 + b * 16 + li];
-#pragma unroll
-      for (int a = 0; a < TN; ++a)
-#pragma unroll
-        for (int b = 0; b < TM; ++b) acc[a][b] = Mfma<T>::mma(av[a], bv[b], acc[a][b]);
+          for (int b = 0; b < TM; ++b) acc[a][b] = Mfma<T>::mma(fb[a][s], fa[b][s], acc[a][b]);
+    };
+    const int64_t full = (kend - kbeg) / KD;
+    // two register buffers, unrolled by two so that they swap by name
+    auto loop = [&](auto ft) {
+      constexpr bool F = decltype(ft)::value;
+      auto load = [&](int64_t kb, typename OpA::Raw& ra, typename OpB::Raw& rb) {
+        oa.template load<F, false>(kbeg + kb * KD, kend, ra);
+        ob.template load<F, false>(kbeg + kb * KD, kend, rb);
+      };
+      int64_t kb = ks;
+      if (kb < full) load(kb, a0, b0);
+      for (; kb + KS < full; kb += 2 * KS) {
+        oa.frags(a0, fa);
+        ob.frags(b0, fb);
+        load(kb + KS, a1, b1);
+        mma();
+        oa.frags(a1, fa);
+        ob.frags(b1, fb);
+        if (kb + 2 * KS < full) load(kb + 2 * KS, a0, b0);
+        mma();
+      }
+      if (kb < full) {
+        oa.frags(a0, fa);
+        ob.frags(b0, fb);
+        mma();
+      }
+    };
+    if (oa.full && ob.full) loop(std::true_type{});
+    else loop(std::false_type{});
+    if (kbeg + full * KD < kend && full % KS == ks) {
+      oa.template load<false, true>(kbeg + full * KD, kend, a0);
+      ob.template load<false, true>(kbeg + full * KD, kend, b0);
+      oa.frags(a0, fa);
+      ob.frags(b0, fb);
+      mma();
     }
   }
 
   double ss = 0.0;
+  // rows 2 li and 2 li + 1 of block pair bp, the four columns of block a
+  auto store = [&](int a, int bp, const acc_t& x0, const acc_t& x1) {
+    const int64_t gm = m0 + 32 * bp + 2 * li;
 #pragma unroll
-  for (int a = 0; a < TN; ++a) {
+    for (int r = 0; r < 4; ++r) {
+      const int64_t gn = n0 + block_row(a, Mfma<T>::row(lk, r));
+      if (gm >= g.M || gn >= g.N) continue;
+      if (g.sym) {  // beta = 0
+        const T v[2] = {g.alpha * x0[r], g.alpha * x1[r]};
 #pragma unroll
-    for (int b = 0; b < TM; ++b) {
-      const int64_t gm = m0 + wm0 + b * 16 + li;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t gn = n0 + wn0 + a * 16 + Mfma<T>::row(lk, r);
-        if (gm < M && gn < N) {
-          T* cp = Cz + gm + gn * ldc;
-          T v = alpha * acc[a][b][r];
-          if (beta != T(0)) v += beta * (*cp);
-          *cp = v;
-          ss += (double)v * (double)v;
+        for (int e = 0; e < 2; ++e)
+          if (gm + e <= gn) {
+            C[gm + e + gn * g.ldc] = v[e];
+            if (g.mirror) C[gn + (gm + e) * g.ldc] = v[e];
+          }
+        continue;
+      }
+      T* cp = C + gm + gn * g.ldc;
+      if (gm + 1 < g.M) {
+        v2_t v = {g.alpha * x0[r], g.alpha * x1[r]};
+        if (g.beta != T(0)) {
+          const v2_t c = *reinterpret_cast<const v2_t*>(cp);
+          v[0] += g.beta * c[0];
+          v[1] += g.beta * c[1];
         }
+        *reinterpret_cast<v2_t*>(cp) = v;
+        ss += (double)v[0] * (double)v[0] + (double)v[1] * (double)v[1];
+      } else {
+        T v = g.alpha * x0[r];
+        if (g.beta != T(0)) v += g.beta * (*cp);
+        *cp = v;
+        ss += (double)v * (double)v;
       }
     }
+  };
+  if constexpr (KS == 1) {
+    if (live) {
+#pragma unroll
+      for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int bp = 0; bp < TM / 2; ++bp) store(a, bp, acc[a][2 * bp], acc[a][2 * bp + 1]);
+    }
+  } else {
+    static_assert(WM * WN == 1 && KS == 4, "the four waves share one tile");
+    T(*part)[TN * TM * 4][64] = reinterpret_cast<T(*)[TN * TM * 4][64]>(sm);
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < TN; ++a)
+#pragma unroll
+      for (int b = 0; b < TM; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) part[wave][(a * TM + b) * 4 + r][lane] = acc[a][b][r];
+    __syncthreads();
+    // block pairs dealt to the waves, partial tiles added in wave order
+    for (int t = wave; t < TN * TM / 2; t += 4) {
+      const int a = t / (TM / 2), bp = t % (TM / 2);
+      acc_t x[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = (a * TM + 2 * bp + e) * 4 + r;
+          x[e][r] = ((part[0][i][lane] + part[1][i][lane]) + part[2][i][lane]) + part[3][i][lane];
+        }
+      store(a, bp, x[0], x[1]);
+    }
   }
-  if (sumsq) {
+  if (g.sumsq) {
     __shared__ double red[kThreads / 64];
     for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
     if (lane == 0) red[wave] = ss;
@@ -203,26 +415,31 @@ gemm_kernel(int64_t M, int64_t N, int64_t K, int64_t kchunk, T alpha, const T* _
     if (tid == 0) {
       double t = 0;
       for (int w = 0; w < kThreads / 64; ++w) t += red[w];
-      sumsq[tm + (int64_t)gridDim.x * tn] = t;
+      g.sumsq[tm + (int64_t)g.gx * tn] = t;
     }
   }
 }
 
-// C = sum_z W[z] (+ beta*C), W[z] is M x N with leading dimension M.
+// C = sum_z W[z] (+ beta*C), W[z] is M x N with leading dimension M, added in
+// double.  sym: the
+// entries on and above the diagonal, each stored on both sides of it.
 template <typename T>
 __global__ void splitk_reduce_kernel(int64_t M, int64_t N, int splits, const T* __restrict__ W,
-                                     T beta, T* __restrict__ C, int64_t ldc) {
+                                     T beta, T* __restrict__ C, int64_t ldc, int sym) {
   int64_t total = M * N;
   for (int64_t idx = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; idx < total;
        idx += (int64_t)gridDim.x * blockDim.x) {
     int64_t i = idx % M, j = idx / M;
-    T s = T(0);
+    if (sym && i > j) continue;
+    double s = 0.0;
     // loads issued ahead of the (in-order) adds
 #pragma unroll 8
-    for (int z = 0; z < splits; ++z) s += W[(int64_t)z * total + idx];
+    for (int z = 0; z < splits; ++z) s += (double)W[(int64_t)z * total + idx];
     T* cp = C + i + j * ldc;
-    if (beta != T(0)) s += beta * (*cp);
-    *cp = s;
+    T v = (T)s;
+    if (beta != T(0)) v += beta * (*cp);
+    *cp = v;
+    if (sym) C[j + i * ldc] = v;
   }
 }
 
@@ -241,88 +458,106 @@ __global__ void sum_partials_kernel(int64_t n, const double* __restrict__ part,
   if (threadIdx.x == 0) *out = red[0];
 }
 
-// C(i, j) <- C(j, i) for i > j: the strictly lower triangle from the upper one
+// How a product is cut: the workgroup tile and the number of k slices.
+enum GemmTile { kTile128x64 = 0, kTile64x32 = 1, kTile32x32 = 2 };
+struct GemmPlan {
+  int tile;
+  int splits;
+  int64_t gx, gy, tiles, kchunk;
+};
+
+// The cheapest cut by a model of the kernel's time in microseconds: the
+// workgroups run in rounds of one a CU (one wave on every SIMD), each as long as
+// a wave's MFMAs (64 cycles each in FP64, 32 in FP32) plus half a microsecond;
+// k slices add a launch and their traffic.  Against the best of all cuts,
+// measured on 25 shapes (26 to 50000 rows, 20 to 1792 columns), its choice was
+// within 8% of the fastest.
 template <typename T>
-__global__ void mirror_lower_kernel(int64_t n, T* __restrict__ C, int64_t ldc) {
-  const int64_t total = n * n;
-  for (int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * 256) {
-    const int64_t i = idx % n, j = idx / n;
-    if (i > j) C[i + j * ldc] = C[j + i * ldc];
+static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice) {
+  static const struct {
+    int bm, bn, ks, mfma;
+    double slow;  // measured time over the MFMAs' (operand loads a wave does not share)
+  } kTiles[3] = {{128, 64, 1, 8, 1.0}, {64, 32, 4, 8, 1.05}, {32, 32, 4, 4, 1.05}};
+  constexpr int64_t depth = KBlock<T>::kDepth;
+  constexpr double kMfmaUs = (sizeof(T) == 8 ? 64.0 : 32.0) / 2400.0;
+  const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
+  const int64_t kblocks = (K + depth - 1) / depth;
+  GemmPlan best{};
+  double best_cost = 1e300;
+  for (int t = 0; t < 3; ++t) {
+    const auto& d = kTiles[t];
+    const int64_t gx = (M + d.bm - 1) / d.bm, gy = (N + d.bn - 1) / d.bn;
+    int64_t tiles = gx * gy;
+    if (sym) {
+      tiles = 0;
+      for (int64_t y = 0; y < gy; ++y) tiles += sym_tiles(y, gx, d.bm, d.bn);
+    }
+    int64_t smax = one_slice ? 1 : kblocks / (2 * d.ks);
+    smax = smax < 1 ? 1 : (smax > 64 ? 64 : smax);
+    // FP32: a wave's running sum takes at most 512 products where the output
+    // is small enough to be sliced (its rounding grows with the length: at
+    // 65536 rows the Gram behind the last CholeskyQR step needs it)
+    int64_t smin = 1;
+    if (sizeof(T) == 4 && !one_slice && M * N <= (int64_t(1) << 20)) {
+      smin = (K + 512 * d.ks - 1) / (512 * d.ks);
+      smin = smin < smax ? smin : smax;
+    }
+    for (int64_t s = smin; s <= smax; ++s) {
+      const int64_t kb = (kblocks + s - 1) / s;
+      if ((kblocks + kb - 1) / kb != s && s > smin) continue;  // as with a smaller s
+      const double wave = (double)((kb + d.ks - 1) / d.ks) * d.mfma * KBlock<T>::kSteps * kMfmaUs;
+      double cost = (double)((tiles * s + cus - 1) / cus) * (wave * d.slow + 0.5);
+      if (s > 1) cost += 2.0 + 2e-6 * (double)s * (double)M * (double)N * sizeof(T) / 8;
+      if (cost < best_cost) {
+        best_cost = cost;
+        best = GemmPlan{t, (int)((kblocks + kb - 1) / kb), gx, gy, tiles, kb * depth};
+      }
+    }
   }
+  return best;
 }
 
-template <typename T, int BM, int BN, int BK>
-static int launch_gemm(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t K, T alpha,
-                       const T* A, int64_t lda, const T* B, int64_t ldb, T beta, T* C,
-                       int64_t ldc, double* sumsq_partials, const char* tag) {
-  const int64_t gx = (M + BM - 1) / BM, gy = (N + BN - 1) / BN;
-  if (gy > 65535) return set_error("gemm: N=%lld too large for the grid", (long long)N);
-  // A^T A with beta = 0: only the tiles that reach the diagonal or above are
-  // formed, the strictly lower triangle is copied from the upper one afterwards
-  const bool tA0 = (ta == 'T' || ta == 't'), tB0 = (tb == 'T' || tb == 't');
-  const bool sym = A == B && lda == ldb && tA0 && !tB0 && M == N && beta == T(0) &&
-                   !sumsq_partials;
-  int64_t tiles = gx * gy;
-  if (sym) {
-    tiles = 0;
-    for (int64_t bx = 0; bx < gx; ++bx)
-      for (int64_t by = 0; by < gy; ++by) tiles += (bx * BM < by * BN + BN) ? 1 : 0;
-  }
-  // split K when the output has too few tiles to fill the CUs
-  int splits = 1;
-  const int64_t target = 2LL * (c->num_cus > 0 ? c->num_cus : 256);
-  if (!sumsq_partials && tiles < target && K >= 4 * 256) {
-    int64_t maxs = K / 256;
-    const int64_t cap = BN <= 32 ? 128 : 64;  // skinny tiles: more, shorter slices
-    if (maxs > cap) maxs = cap;
-    splits = pick_k_slices(tiles, target, maxs);
-  }
-  int64_t kchunk = K;
-  if (splits > 1) {
-    kchunk = (K + splits - 1) / splits;
-    kchunk = (kchunk + BK - 1) / BK * BK;
-    splits = (int)((K + kchunk - 1) / kchunk);
-  }
+template <typename T, bool TA, bool TB>
+static void gemm_launch_tile(Context* c, int tile, dim3 grid, const GemmArgs<T>& g) {
+  if (tile == kTile128x64)
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 2, 2>), grid, dim3(kThreads), 0, c->stream, g);
+  else if (tile == kTile64x32)
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 1, 1>), grid, dim3(kThreads), 0, c->stream, g);
+  else
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 2, 2, 1, 1>), grid, dim3(kThreads), 0, c->stream, g);
+}
+
+template <typename T>
+static int launch_gemm(Context* c, const GemmPlan& pl, char ta, char tb, int64_t M, int64_t N,
+                       int64_t K, T alpha, const T* A, int64_t lda, const T* B, int64_t ldb, T beta,
+                       T* C, int64_t ldc, double* sumsq_partials, bool sym, const char* tag) {
   DBuf<T> work;
-  T* Cout = C;
-  int64_t ldo = ldc, zstride = 0;
-  T a_eff = alpha, b_eff = beta;
-  if (splits > 1) {
-    RSVD_TRY(work.alloc((size_t)(M * N * splits)));
-    Cout = work.p;
-    ldo = M;
-    zstride = M * N;
-    b_eff = T(0);
+  GemmArgs<T> g{M, N, K, pl.kchunk, alpha, A, lda, B, ldb, beta, C, ldc, 0, sumsq_partials,
+                sym ? 1 : 0, sym ? 1 : 0, (int)pl.gx, (int)pl.gy};
+  if (pl.splits > 1) {
+    RSVD_TRY(work.alloc((size_t)(M * N * pl.splits)));
+    g.C = work.p;
+    g.ldc = M;
+    g.zstride = M * N;
+    g.beta = T(0);
+    g.mirror = 0;
   }
-  dim3 grid((unsigned)gx, (unsigned)gy, (unsigned)splits);
   {
     KTimer kt(c, tag);
+    const dim3 grid((unsigned)pl.tiles, (unsigned)pl.splits);
     const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
-#define RSVD_GEMM_LAUNCH(TA_, TB_)                                                          \
-  hipLaunchKernelGGL((gemm_kernel<T, TA_, TB_, BM, BN, BK>), grid, dim3(kThreads), 0,         \
-                     c->stream, M, N, K, kchunk, a_eff, A, lda, B, ldb, b_eff, Cout, ldo,    \
-                     zstride, sumsq_partials, sym ? 1 : 0)
-    if (!tA && !tB) RSVD_GEMM_LAUNCH(false, false);
-    else if (tA && !tB) RSVD_GEMM_LAUNCH(true, false);
-    else if (!tA && tB) RSVD_GEMM_LAUNCH(false, true);
-    else RSVD_GEMM_LAUNCH(true, true);
-#undef RSVD_GEMM_LAUNCH
+    if (!tA && !tB) gemm_launch_tile<T, false, false>(c, pl.tile, grid, g);
+    else if (tA && !tB) gemm_launch_tile<T, true, false>(c, pl.tile, grid, g);
+    else if (!tA && tB) gemm_launch_tile<T, false, true>(c, pl.tile, grid, g);
+    else gemm_launch_tile<T, true, true>(c, pl.tile, grid, g);
     RSVD_LAUNCH_CHECK();
   }
-  if (splits > 1) {
+  if (pl.splits > 1) {
     int64_t total = M * N;
     int blocks = (int)((total + 255) / 256);
     if (blocks > 4096) blocks = 4096;
     hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks), dim3(256), 0, c->stream, M, N,
-                       splits, (const T*)work.p, beta, C, ldc);
-    RSVD_LAUNCH_CHECK();
-  }
-  if (sym) {
-    const int64_t total = M * M;
-    int blocks = (int)((total + 255) / 256);
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(mirror_lower_kernel<T>, dim3(blocks), dim3(256), 0, c->stream, M, C, ldc);
+                       pl.splits, (const T*)work.p, beta, C, ldc, sym ? 1 : 0);
     RSVD_LAUNCH_CHECK();
   }
   return 0;
@@ -409,13 +644,14 @@ static int gemm_any(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t 
     RSVD_LAUNCH_CHECK();
     return 0;
   }
-  // N <= 32 (a product with a panel of 32 or fewer columns): a 128 x 32 tile,
-  // no half-empty 128 x 64 tile
-  if (N <= 32)
-    return launch_gemm<T, 128, 32, 16>(c, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-                                       nullptr, tag);
-  return launch_gemm<T, 128, 64, 16>(c, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-                                     nullptr, tag);
+  if (N > 32 && (N + 63) / 64 > 65535)
+    return set_error("gemm: N=%lld too large for the grid", (long long)N);
+  // A^T A or B B^T with beta = 0: the entries on and above the diagonal are
+  // formed and stored on both sides of it
+  const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
+  const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == T(0);
+  return launch_gemm<T>(c, gemm_plan<T>(c, M, N, K, sym, false), ta, tb, M, N, K, alpha, A, lda, B,
+                        ldb, beta, C, ldc, nullptr, sym, tag);
 }
 
 int gemm_f64(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t K, double alpha,
@@ -444,12 +680,14 @@ int gemm_f64_deflate(Context* c, int64_t M, int64_t N, int64_t K, const double* 
     RSVD_HIP(hipMemsetAsync(sumsq, 0, sizeof(double), c->stream));
     return 0;
   }
-  const int64_t gx = (M + 127) / 128, gy = (N + 63) / 64;
+  const int64_t k = K > 0 ? K : 1;
+  const GemmPlan pl = gemm_plan<double>(c, M, N, k, false, true);
+  const int64_t nparts = pl.gx * pl.gy;
   DBuf<double> part;
-  RSVD_TRY(part.alloc((size_t)(gx * gy)));
-  RSVD_TRY((launch_gemm<double, 128, 64, 16>(c, 'N', 'N', M, N, K > 0 ? K : 1, -1.0, Q, ldq, B,
-                                             ldb, 1.0, C, ldc, part.p, "gemm_f64_deflate")));
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, c->stream, gx * gy,
+  RSVD_TRY(part.alloc((size_t)nparts));
+  RSVD_TRY(launch_gemm<double>(c, pl, 'N', 'N', M, N, k, -1.0, Q, ldq, B, ldb, 1.0, C, ldc, part.p,
+                               false, "gemm_f64_deflate"));
+  hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, c->stream, nparts,
                      (const double*)part.p, sumsq);
   RSVD_LAUNCH_CHECK();
   return 0;

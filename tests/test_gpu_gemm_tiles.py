@@ -1,0 +1,63 @@
+"""FP64 / FP32 products at the edges of the GEMM's tiles (32 and 128 rows, 32 and 64 columns), of
+its k blocks (16 FP64, 32 FP32 elements) and of its k slices, every transposition, Grams
+(A^T A and B B^T, one operand passed twice), and leading dimensions beyond the rows."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (31, 33, 15), (32, 32, 16), (33, 31, 17), (127, 64, 31), (128, 65, 32),
+          (129, 63, 33), (64, 1, 4097), (1, 64, 700), (400, 26, 200), (257, 300, 1000)]
+
+
+def _padded(rng, rows, cols, pad, dtype):
+    """A (rows + pad) x cols device buffer and the rows x cols matrix in it; the rest is NaN."""
+    full = np.full((rows + pad, cols), np.nan, dtype=dtype)
+    full[:rows] = rng.standard_normal((rows, cols))
+    return full, full[:rows].astype(np.float64)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T"), ("T", "T")])
+def test_gemm_edges(gpu_lib, ta, tb, dtype):
+    rp = gpu_lib
+    eps = np.finfo(dtype).eps
+    for q, (m, n, k) in enumerate(SHAPES):
+        rng = np.random.default_rng(100 + q)
+        pad = (0, 1, 3)[q % 3]
+        fa, A = _padded(rng, *((m, k) if ta == "N" else (k, m)), pad, dtype)
+        fb, B = _padded(rng, *((k, n) if tb == "N" else (n, k)), pad, dtype)
+        fc, C0 = _padded(rng, m, n, pad, dtype)
+        dA, dB, dC = (rp.DeviceMatrix.from_host(x) for x in (fa, fb, fc))
+        beta = (0.0, -0.5)[q % 2]
+        rc = rp.load().rsvd_dev_gemm(0 if dtype == np.float64 else 1, ta.encode(), tb.encode(), m,
+                                     n, k, 2.0, dA.ptr, fa.shape[0], dB.ptr, fb.shape[0], beta,
+                                     dC.ptr, fc.shape[0])
+        assert rc == 0, rp.last_error()
+        oA, oB = (A if ta == "N" else A.T), (B if tb == "N" else B.T)
+        got = dC.to_host()
+        # every term once: at most k roundings of the running sum, then alpha and beta
+        bound = (k + 4) * eps * (2.0 * np.abs(oA) @ np.abs(oB) + np.abs(C0))
+        err = np.abs(got[:m] - (2.0 * oA @ oB + beta * C0))
+        assert np.all(err <= bound), (m, n, k, float((err / bound).max()))
+        assert np.all(np.isnan(got[m:]))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n,k", [(1, 5), (20, 2000), (33, 400), (64, 64), (110, 2000),
+                                 (129, 5001), (300, 50)])
+def test_gram_is_symmetric(gpu_lib, n, k, dtype):
+    rp = gpu_lib
+    eps = np.finfo(dtype).eps
+    rng = np.random.default_rng(n)
+    for ta in "TN":
+        X = rng.standard_normal((k, n) if ta == "T" else (n, k)).astype(dtype)
+        dX, dG = rp.DeviceMatrix.from_host(X), rp.DeviceMatrix(n, n, dtype)
+        rc = rp.load().rsvd_dev_gemm(0 if dtype == np.float64 else 1, ta.encode(),
+                                     b"N" if ta == "T" else b"T", n, n, k, 1.0, dX.ptr,
+                                     X.shape[0], dX.ptr, X.shape[0], 0.0, dG.ptr, n)
+        assert rc == 0, rp.last_error()
+        G = dG.to_host()
+        Y = X.astype(np.float64) if ta == "T" else X.T.astype(np.float64)
+        assert np.array_equal(G, G.T)
+        assert np.all(np.abs(G - Y.T @ Y) <= (k + 4) * eps * (np.abs(Y).T @ np.abs(Y)))
