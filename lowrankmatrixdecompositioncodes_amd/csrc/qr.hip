@@ -93,178 +93,150 @@ __device__ __forceinline__ void ci_put(const double (&v)[4], double (*T)[CHP]) {
   }
 }
 
-// 1 / d to about one ulp: the hardware reciprocal estimate and two Newton
-// steps (shorter than a correctly rounded division on the serial path).
-__device__ __forceinline__ double ci_rcp(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = fma(r, fma(-d, r, 1.0), r);
-  r = fma(r, fma(-d, r, 1.0), r);
-  return r;
+// v of lane J of the 16-lane row the lane is in (a data-parallel move).
+template <int J>
+__device__ __forceinline__ double ci_bcast(double v) {
+  union {
+    double d;
+    int i[2];
+  } u = {v};
+  u.i[0] = __builtin_amdgcn_mov_dpp(u.i[0], 0x150 + J, 0xf, 0xf, true);  // row_newbcast:J
+  u.i[1] = __builtin_amdgcn_mov_dpp(u.i[1], 0x150 + J, 0xf, 0xf, true);
+  return u.d;
 }
 
-// Unnormalised right-looking Cholesky of Dm (upper triangle valid, kb x kb),
-// four pivots per barrier.  A step takes the pivot rows P = j .. j + 3: every
-// thread eliminates the 4 x 4 pivot block itself (the same instructions on
-// the same LDS entries in every thread, so all copies agree) and the pivot
-// rows at the columns it needs (its row a and its four columns), then
-// subtracts sum_{w in P} U_wa U_wc / U_ww from its entries of the rows below
-// P.  A pivot that is not above kCholRelTol * ref (or is not finite) sets
-// *bad and is replaced (by 1 when it is not positive) so the factorisation
-// runs to the end.  Rows stay in registers; the rows of the next step are
-// stored before the barrier that ends a step, all rows at the end.  On exit Dm
-// holds R_kk (zero below the diagonal and past kb) and sqd / invd its diagonal
-// and reciprocals.
-__device__ void ci_factor(double (*Dm)[CHP], int kb, const double* ref, double* piv,
-                          double* sqd, double* invd, int* bad) {
-  constexpr int PB = 4;
-  const int tid = threadIdx.x, a = tid & (CB - 1), c0 = (tid >> 5) * 4;
-  double own[4];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) own[q] = Dm[a][c0 + q];
-  // All eight steps run on full 4 x 4 blocks: the rows and columns past kb
-  // are zero, their pivots are taken as 1 and change nothing, so the step
-  // body has no bounds on the block.
-  for (int j = 0; j < CB; j += PB) {
-    // S of the pivot block (upper part) and of the pivot rows at column a
-    // (x = 0) and at columns c0 .. c0 + 3 (x = 1 .. 4)
-    double U[PB][PB], X[PB][5], rinv[PB];
-#pragma unroll
-    for (int u = 0; u < PB; ++u) {
-#pragma unroll
-      for (int v = u; v < PB; ++v) U[u][v] = Dm[j + u][j + v];
-      X[u][0] = Dm[j + u][a];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) X[u][1 + q] = Dm[j + u][c0 + q];
-    }
-    // eliminate inside the pivot block, pivot by pivot
-#pragma unroll
-    for (int u = 0; u < PB; ++u) {
-#pragma unroll
-      for (int w = 0; w < u; ++w) {
-        const double l = U[w][u] * rinv[w];
-#pragma unroll
-        for (int v = u; v < PB; ++v) U[u][v] -= l * U[w][v];
-#pragma unroll
-        for (int x = 0; x < 5; ++x) X[u][x] -= l * X[w][x];
-      }
-      double d = U[u][u];
-      const bool pad = j + u >= kb;
-      const bool ok = pad | ((d > kCholRelTol * ref[pad ? 0 : j + u]) & isfinite(d));
-      d = pad ? 1.0 : (ok ? d : ((d > 0.0 && isfinite(d)) ? d : 1.0));
-      rinv[u] = ci_rcp(d);
-      if (tid == 0) {
-        if (!ok) *bad = 1;
-        piv[j + u] = d;
-      }
-    }
-    if (a >= j + PB && a < kb) {
-      // rows below P: the Schur complement update
-#pragma unroll
-      for (int u = 0; u < PB; ++u) {
-        const double l = X[u][0] * rinv[u];
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (c0 + q >= a && c0 + q < kb) own[q] -= l * X[u][1 + q];
-      }
-      if (a < j + 2 * PB) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if (c0 + q >= a && c0 + q < kb) Dm[a][c0 + q] = own[q];
-      }
-    } else if (a >= j && a < j + PB) {
-      // a pivot row: its eliminated values are final
-#pragma unroll
-      for (int u = 0; u < PB; ++u)
-        if (a == j + u) {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) own[q] = X[u][1 + q];
-        }
-    }
-    __syncthreads();
+// Cholesky and inverse of a 16 x 16 block in the registers of a 16-lane row:
+// lane c holds column c of the symmetric block (a[r], all rows) and column c of
+// the identity (e[r]); step j scales row j by 1 / sqrt(pivot) and subtracts it
+// from the rows below, u_jr broadcast from lane r.  On exit a[r] (r <= c) is
+// R(r, c), e[r] is R^-1(c, r) (zero for r < c) and piv lane c's pivot.  The steps
+// from kb on (padding) are left out.  A pivot that is not positive gives NaN
+// from there on; the caller's test of piv reports it.
+template <int J>
+__device__ __forceinline__ void ci_chol16_step(double (&a)[16], double (&e)[16], int c, int kb,
+                                               double* piv) {
+  if (J >= kb) return;
+  const double d = ci_bcast<J>(a[J]);
+  *piv = (c == J) ? d : *piv;
+  // 1 / sqrt(d): the hardware estimate and one third-order step
+  const double y0 = __builtin_amdgcn_rsq(d);
+  const double r = fma(-d * y0, y0, 1.0);
+  const double y = fma(y0 * r, fma(0.375, r, 0.5), y0);
+  a[J] *= y;
+  e[J] *= y;
+  const double u = a[J], w = e[J];
+  // (one compile-time broadcast a row below)
+#define RSVD_CI_ROW(R)                     \
+  if constexpr (R > J && R < 16) {         \
+    const double m = ci_bcast<R>(u);       \
+    a[R] = fma(-m, u, a[R]);               \
+    e[R] = fma(-m, w, e[R]);               \
   }
-  if (a < kb) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      if (c0 + q >= a && c0 + q < kb) Dm[a][c0 + q] = own[q];
-  }
-  if (tid < kb) {
-    const double sj = sqrt(piv[tid]);
-    sqd[tid] = sj;
-    invd[tid] = 1.0 / sj;
-  }
-  __syncthreads();
-  // normalise: R[j][c] = U[j][c] / sqrt(U[j][j])
-  for (int e = tid; e < CB * CB; e += 256) {
-    const int i = e & (CB - 1), c = e >> 5;
-    double v = 0.0;
-    if (i < kb && c < kb) v = (c > i) ? Dm[i][c] * invd[i] : (c == i ? sqd[i] : 0.0);
-    Dm[i][c] = v;
-  }
-  __syncthreads();
-}
-
-// Xk = R_kk^-1 (upper, zero past kb) by blocked inversion on all threads:
-// the four 8 x 8 diagonal blocks by back substitution (a thread per column),
-// then X_12 = -X_11 R_12 X_22 for the two 16 x 16 diagonal blocks and for the
-// whole tile, each as two small products with a barrier between.  Tw is
-// scratch.  Ends with a barrier.
-__device__ void ci_tri_inv(const double (*Rk)[CHP], const double* invd, int kb,
-                           double (*Xk)[CHP], double (*Tw)[CHP]) {
-  const int tid = threadIdx.x;
-  for (int e = tid; e < CB * CB; e += 256) Xk[e & (CB - 1)][e >> 5] = 0.0;
-  __syncthreads();
-  if (tid < CB) {
-    const int c = tid, b0 = c & ~7;
-    double x[8];
-#pragma unroll
-    for (int r = 7; r >= 0; --r) {
-      double s = 0.0;
-#pragma unroll
-      for (int u = 7; u > r; --u) s = fma(Rk[b0 + r][b0 + u], x[u], s);
-      const double ir = (b0 + r < kb) ? invd[b0 + r] : 0.0;
-      x[r] = (b0 + r > c) ? 0.0 : ((b0 + r == c) ? ir : -s * ir);
-    }
-#pragma unroll
-    for (int r = 0; r < 8; ++r) Xk[b0 + r][c] = (c < kb) ? x[r] : 0.0;
-  }
-  __syncthreads();
-  // 8 -> 16: blocks at b0 = 0 and 16, sub-blocks of 8
-  if (tid < 128) {
-    const int b0 = (tid >> 6) * 16, r = (tid >> 3) & 7, c = tid & 7;
-    double s = 0.0;  // T = R_12 X_22
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s = fma(Rk[b0 + r][b0 + 8 + u], Xk[b0 + 8 + u][b0 + 8 + c], s);
-    Tw[b0 + r][c] = s;
-  }
-  __syncthreads();
-  if (tid < 128) {
-    const int b0 = (tid >> 6) * 16, r = (tid >> 3) & 7, c = tid & 7;
-    double s = 0.0;  // X_12 = -X_11 T
-#pragma unroll
-    for (int u = 0; u < 8; ++u) s = fma(Xk[b0 + r][b0 + u], Tw[b0 + u][c], s);
-    Xk[b0 + r][b0 + 8 + c] = -s;
-  }
-  __syncthreads();
-  // 16 -> 32
-  {
-    const int r = tid >> 4, c = tid & 15;
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) s = fma(Rk[r][16 + u], Xk[16 + u][16 + c], s);
-    Tw[r][c] = s;
-  }
-  __syncthreads();
-  {
-    const int r = tid >> 4, c = tid & 15;
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) s = fma(Xk[r][u], Tw[u][c], s);
-    Xk[r][16 + c] = -s;
-  }
-  __syncthreads();
+  RSVD_CI_ROW(1) RSVD_CI_ROW(2) RSVD_CI_ROW(3) RSVD_CI_ROW(4) RSVD_CI_ROW(5)
+  RSVD_CI_ROW(6) RSVD_CI_ROW(7) RSVD_CI_ROW(8) RSVD_CI_ROW(9) RSVD_CI_ROW(10)
+  RSVD_CI_ROW(11) RSVD_CI_ROW(12) RSVD_CI_ROW(13) RSVD_CI_ROW(14) RSVD_CI_ROW(15)
+#undef RSVD_CI_ROW
+  if constexpr (J < 15) ci_chol16_step<J + 1>(a, e, c, kb, piv);
 }
 
 typedef double ci_d4 __attribute__((ext_vector_type(4)));
+
+// One wave: acc + op(P) Q for 16 x 16 blocks of LDS tiles (row-major, CHP):
+// op(P) = P^T reads P[k][i].  Register r of lane l is entry (4 r + l / 16,
+// l % 16).
+template <bool TA>
+__device__ __forceinline__ ci_d4 ci_mm16(const double* P, const double* Q, ci_d4 acc) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int k = 4 * s + lk;
+    const double p = TA ? P[k * CHP + li] : P[li * CHP + k];
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p, Q[k * CHP + li], acc, 0, 0, 0);
+  }
+  return acc;
+}
+__device__ __forceinline__ void ci_st16(double* C, const ci_d4& v, double scale) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) C[(4 * r + lk) * CHP + li] = scale * v[r];
+}
+// One wave's LDS operations complete in order; this keeps the compiler from
+// moving them across.
+__device__ __forceinline__ void ci_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Cholesky Dm = R^T R (upper triangle read, kb x kb valid, zero beyond) and Xk =
+// R^-1 of a 32 x 32 tile, by 16 x 16 blocks on wave 0 alone: the two diagonal
+// blocks in registers (ci_chol16_step), the products between them on the FP64
+// matrix cores.  On exit Dm holds R, both zero below the diagonal and past kb;
+// Tw is scratch; *bad is set on a bad pivot (see above).  Ends with a barrier.
+// The chain of 32 pivots is what a launch waits for: four pivots a barrier with
+// every thread eliminating the pivot block (and a blocked inverse after it) took
+// 24k cycles and a launch 14.9 us at n = 110; a broadcast and two multiply-adds a
+// row and pivot, 10.5 us.
+__device__ void ci_factor_inv(double (*Dm)[CHP], int kb, const double* ref, double (*Xk)[CHP],
+                              double (*Tw)[CHP], int* bad) {
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+    bool b = false;
+#pragma unroll 1
+    for (int h = 0; h < 2; ++h) {
+      const int o = 16 * h, kh = kb - o;
+      double a[16], e[16];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        a[r] = Dm[o + (r < c ? r : c)][o + (r < c ? c : r)];
+        e[r] = (r == c) ? 1.0 : 0.0;
+      }
+      double piv = 1.0;
+      ci_chol16_step<0>(a, e, c, kh, &piv);
+      // a pivot must be finite and above kCholRelTol times its diagonal entry
+      b |= c < kh && !(piv > kCholRelTol * ref[o + c] && piv < INFINITY);
+      ci_wave_fence();
+      // row group g of the wave stores a quarter of the rows
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if ((r >> 2) == g) {
+          const bool in = r < kh && c < kh;
+          Dm[o + r][o + c] = (in && r <= c) ? a[r] : 0.0;
+          Xk[o + c][o + r] = in ? e[r] : 0.0;
+        }
+      ci_wave_fence();
+      const ci_d4 z = {0.0, 0.0, 0.0, 0.0};
+      if (h == 0) {
+        // R_B = X_A^T B, then C - R_B^T R_B in place
+        ci_d4 p = ci_mm16<true>(&Xk[0][0], &Dm[0][16], z);
+        ci_wave_fence();
+        ci_st16(&Dm[0][16], p, 1.0);
+        ci_wave_fence();
+        p = ci_mm16<true>(&Dm[0][16], &Dm[0][16], z);
+        double cv[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = 4 * r + g;
+          cv[r] = Dm[16 + (i < c ? i : c)][16 + (i < c ? c : i)] - p[r];
+        }
+        ci_wave_fence();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          Dm[16 + 4 * r + g][16 + c] = cv[r];
+          Dm[16 + 4 * r + g][c] = 0.0;
+          Xk[16 + 4 * r + g][c] = 0.0;
+        }
+        ci_wave_fence();
+      } else {
+        // X_AC = -X_A R_B X_C
+        ci_st16(&Tw[0][0], ci_mm16<false>(&Dm[0][16], &Xk[16][16], z), 1.0);
+        ci_wave_fence();
+        ci_st16(&Xk[0][16], ci_mm16<false>(&Xk[0][0], &Tw[0][0], z), -1.0);
+      }
+    }
+    if (b) *bad = 1;
+  }
+  __syncthreads();
+}
+
 
 // acc += the wave's 16 x 16 quadrant (wave / 2, wave % 2) of op(A) B over the
 // padded 32 x 32 tiles (op(A) = A^T when TA), on the FP64 matrix cores: eight
@@ -297,7 +269,7 @@ cholinv_panel_kernel(int64_t n, double* __restrict__ G, double* __restrict__ R,
                      double* __restrict__ diag0, int k, int* __restrict__ fail) {
   __shared__ double Dm[CB][CHP], Xk[CB][CHP], T1[CB][CHP], T2[CB][CHP], T3[CB][CHP],
       T4[CB][CHP];
-  __shared__ double refd[CB], piv[CB], sqd[CB], invd[CB];
+  __shared__ double refd[CB];
   __shared__ int bad;
   const int tid = threadIdx.x;
   const int64_t p = (int64_t)k * CB;
@@ -361,9 +333,7 @@ cholinv_panel_kernel(int64_t n, double* __restrict__ G, double* __restrict__ R,
   if (tid == 0) bad = 0;
   __syncthreads();
   if (role == 0 && k == 0 && ti == tj && tid < bw(ti)) diag0[pti + tid] = T3[tid][tid];
-  ci_factor(Dm, kb, refd, piv, sqd, invd, &bad);
-
-  ci_tri_inv(Dm, invd, kb, Xk, T4);
+  ci_factor_inv(Dm, kb, refd, Xk, T4, &bad);
 
   const ci_d4 z4 = {0.0, 0.0, 0.0, 0.0};
   const int cl = ci_col();
@@ -372,7 +342,7 @@ cholinv_panel_kernel(int64_t n, double* __restrict__ G, double* __restrict__ R,
     // here any more), then the trailing tile
     const ci_d4 pa = ci_mma<true>(Xk, T1, z4);
     const ci_d4 pb = (tj != ti) ? ci_mma<true>(Xk, T2, z4) : z4;
-    // Dm's last reads (inside ci_tri_inv) were before its closing barrier
+    // Dm's last reads (inside ci_factor_inv) were before its closing barrier
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       T4[ci_row(r)][cl] = pa[r];
