@@ -23,10 +23,10 @@ namespace {
 // the update cancelled to below this fraction of its last exact value
 constexpr double kTol3z = 1.0536712127723509e-08;
 
-// vn1 = vn2 = ||A(:, j)||, perm = identity; one wave per column.
+// vn1 = vn2 = ||A(:, j)||, pos = identity; one wave per column.
 __global__ void __launch_bounds__(256)
 pqr_init_kernel(int64_t m, int64_t n, const double* __restrict__ A, int64_t lda,
-                double* __restrict__ vn1, double* __restrict__ vn2, int* __restrict__ perm) {
+                double* __restrict__ vn1, double* __restrict__ vn2, int* __restrict__ pos) {
   const int lane = threadIdx.x & 63;
   const int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (j >= n) return;
@@ -37,132 +37,187 @@ pqr_init_kernel(int64_t m, int64_t n, const double* __restrict__ A, int64_t lda,
   if (lane == 0) {
     vn1[j] = sqrt(s);
     vn2[j] = vn1[j];
-    perm[j] = (int)j;
+    pos[j] = (int)j;
   }
 }
 
-// Step i, part 1 (one workgroup): pivot = first index of max vn1[i..n)
-// (idamax), swap it into column i (vn of the pivot's slot inherits column i's,
-// as dlaqp2), then the reflector of A(i:m, i) in dlarfg's convention: beta =
-// -sign(alpha) hypot(alpha, ||x||), tau = (beta - alpha) / beta, v = x /
-// (alpha - beta), R_ii = beta; tau = 0 for a single row or a zero x.
-__global__ void __launch_bounds__(1024)
-pqr_pivot_kernel(int64_t m, int64_t n, double* __restrict__ A, int64_t lda, int64_t i,
-                 double* __restrict__ vn1, double* __restrict__ vn2, int* __restrict__ perm,
-                 double* __restrict__ tau) {
-  __shared__ double sv[16];
-  __shared__ int64_t si[16];
-  __shared__ int64_t s_pvt;
-  __shared__ double s_scale;
+// Step i of the factorisation, one launch.  Columns stay where they are in
+// memory; pos[c] is the place of column c in the current order (places < i hold
+// the pivots so far).  Every workgroup finds the pivot for itself -- the first
+// place (idamax) with the largest vn1 among places i .. n-1, the two places
+// swapped as dlaqp2 swaps the columns -- and its reflector in dlarfg's
+// convention: beta = -sign(alpha) hypot(alpha, ||x||), tau = (beta - alpha) /
+// beta, v = x / (alpha - beta); tau = 0 for a single row or a zero x.  Then each
+// wave applies it to its own column (rows i .. m-1) and downdates that column's
+// partial norm (dlaqp2's rule, recomputed from the column when the downdate
+// cancelled).  Workgroup 0 keeps v, beta and tau in V, beta, tau, so that the
+// pivot column is only read; vn1 and pos are double-buffered for the same reason.
+// A step is bound by latency (two dependent rounds of loads, two reductions and
+// the launch), so one launch that repeats the pivot's work in every workgroup
+// beats a pivot launch and an update launch: 7.5 us against 11.4 us a step at
+// 384 x 1200.
+// LDSV: the pivot column's rows fit the LDS buffer.
+constexpr int kPqrLds = 4096, kPqrKeep = 8;
+
+template <bool LDSV>
+__global__ void __launch_bounds__(256)
+pqr_step_kernel(int64_t m, int64_t n, double* __restrict__ A, int64_t lda, int64_t i,
+                const double* __restrict__ vn1, double* __restrict__ vn1_out,
+                double* __restrict__ vn2, const int* __restrict__ pos, int* __restrict__ pos_out,
+                double* __restrict__ V, double* __restrict__ betas, double* __restrict__ tau) {
+  __shared__ double xs[LDSV ? kPqrLds : 1];
+  __shared__ double sv[4];
+  __shared__ int sp[4], sc[4], s_ci;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int64_t c = (int64_t)blockIdx.x * 4 + w;
+  const bool have = c < n;
+  double* y = A + (have ? c : 0) * lda + i;  // row i of the wave's column
+  const int64_t len = m - i;
+  // the wave's column in registers (the first kPqrKeep chunks of 64 rows)
+  double yk[kPqrKeep];
+#pragma unroll
+  for (int q = 0; q < kPqrKeep; ++q) {
+    const int64_t r = lane + 64 * q;
+    yk[q] = (have && r < len) ? y[r] : 0.0;
+  }
+  const int my_pos = have ? pos[c] : 0;
+  const double n1 = have ? vn1[c] : 0.0;
+  // pivot: the largest norm, the smallest place among equals
   double best = -1.0;
-  int64_t bidx = n;
-  for (int64_t j = i + tid; j < n; j += 1024) {
+  int bp = (int)n, bc = 0;
+  for (int64_t j = tid; j < n; j += 256) {
+    const int p = pos[j];
     const double v = vn1[j];
-    if (v > best) { best = v; bidx = j; }
+    if (p == (int)i) s_ci = (int)j;
+    if (p >= (int)i && (v > best || (v == best && p < bp))) {
+      best = v;
+      bp = p;
+      bc = (int)j;
+    }
   }
   for (int off = 32; off > 0; off >>= 1) {
     const double ov = __shfl_xor(best, off, 64);
-    const int64_t oi = __shfl_xor(bidx, off, 64);
-    if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
-  }
-  if (lane == 0) { sv[w] = best; si[w] = bidx; }
-  __syncthreads();
-  if (tid == 0) {
-    double b = sv[0];
-    int64_t bi = si[0];
-    for (int k = 1; k < 16; ++k)
-      if (sv[k] > b || (sv[k] == b && si[k] < bi)) { b = sv[k]; bi = si[k]; }
-    s_pvt = (bi < n) ? bi : i;
-  }
-  __syncthreads();
-  const int64_t pvt = s_pvt;
-  if (pvt != i) {
-    double* ci = A + i * lda;
-    double* cp = A + pvt * lda;
-    for (int64_t r = tid; r < m; r += 1024) {
-      const double t = ci[r];
-      ci[r] = cp[r];
-      cp[r] = t;
+    const int op = __shfl_xor(bp, off, 64), oc = __shfl_xor(bc, off, 64);
+    if (ov > best || (ov == best && op < bp)) {
+      best = ov;
+      bp = op;
+      bc = oc;
     }
+  }
+  if (lane == 0) {
+    sv[w] = best;
+    sp[w] = bp;
+    sc[w] = bc;
+  }
+  __syncthreads();
+  best = sv[0];
+  bp = sp[0];
+  bc = sc[0];
+  for (int k = 1; k < 4; ++k)
+    if (sv[k] > best || (sv[k] == best && sp[k] < bp)) {
+      best = sv[k];
+      bp = sp[k];
+      bc = sc[k];
+    }
+  if (bp >= (int)n) {  // no comparable norm (NaN): the column in place i
+    bp = (int)i;
+    bc = s_ci;
+  }
+  const int new_pos = c == bc ? (int)i : (my_pos == (int)i ? bp : my_pos);
+  if (have && lane == 0) pos_out[c] = new_pos;
+  // reflector
+  const double* x = A + (int64_t)bc * lda + i;
+  const double alpha = x[0];
+  double ss = 0.0;
+  for (int64_t r = 1 + tid; r < len; r += 256) {
+    const double t = x[r];
+    if (LDSV) xs[r] = t;
+    ss += t * t;
+  }
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off, 64);
+  __syncthreads();  // sv has been read
+  if (lane == 0) sv[w] = ss;
+  __syncthreads();
+  ss = ((sv[0] + sv[1]) + sv[2]) + sv[3];
+  double t = 0.0, scale = 0.0, beta = alpha;
+  if (len > 1 && ss != 0.0) {
+    const double xn = sqrt(ss);
+    const double a = fabs(alpha), big = fmax(a, xn), sml = fmin(a, xn);
+    const double h = (sml == 0.0) ? big : big * sqrt(1.0 + (sml / big) * (sml / big));
+    beta = (alpha >= 0.0) ? -h : h;
+    t = (beta - alpha) / beta;
+    scale = 1.0 / (alpha - beta);
+  }
+  auto v_at = [&](int64_t r) { return (LDSV ? xs[r] : x[r]) * scale; };  // r > 0
+  if (blockIdx.x == 0) {
+    for (int64_t r = 1 + tid; r < len; r += 256)
+      V[i + r + i * m] = t != 0.0 ? v_at(r) : (LDSV ? xs[r] : x[r]);
     if (tid == 0) {
-      const int t = perm[pvt];
-      perm[pvt] = perm[i];
-      perm[i] = t;
-      vn1[pvt] = vn1[i];
-      vn2[pvt] = vn2[i];
+      betas[i] = beta;
+      tau[i] = t;
     }
   }
-  __syncthreads();
-  double* x = A + i + i * lda;
-  const int64_t len = m - i;
-  double s = 0.0;
-  for (int64_t r = 1 + tid; r < len; r += 1024) s += x[r] * x[r];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) sv[w] = s;
-  __syncthreads();
-  if (tid == 0) {
-    double ss = 0.0;
-    for (int k = 0; k < 16; ++k) ss += sv[k];
-    const double alpha = x[0];
-    if (len <= 1 || ss == 0.0) {
-      tau[i] = 0.0;
-      s_scale = 0.0;
-    } else {
-      const double xn = sqrt(ss);
-      const double a = fabs(alpha), big = fmax(a, xn), sml = fmin(a, xn);
-      const double h = (sml == 0.0) ? big : big * sqrt(1.0 + (sml / big) * (sml / big));
-      const double beta = (alpha >= 0.0) ? -h : h;
-      tau[i] = (beta - alpha) / beta;
-      s_scale = 1.0 / (alpha - beta);
-      x[0] = beta;
-    }
-  }
-  __syncthreads();
-  const double sc = s_scale;
-  if (sc != 0.0)
-    for (int64_t r = 1 + tid; r < len; r += 1024) x[r] *= sc;
-}
-
-// Step i, part 2: columns c > i get H_i applied (rows i..m-1) and their
-// partial norms downdated (dlaqp2's rule, recomputed from the column when the
-// downdate cancelled); one wave per column.
-__global__ void __launch_bounds__(256)
-pqr_update_kernel(int64_t m, int64_t n, double* __restrict__ A, int64_t lda, int64_t i,
-                  double* __restrict__ vn1, double* __restrict__ vn2,
-                  const double* __restrict__ tau) {
-  const int lane = threadIdx.x & 63;
-  const int64_t c = i + 1 + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (c >= n) return;
-  const double t = tau[i];
-  const double* v = A + i * lda;  // v_i = 1, v_r = A(r, i) below
-  double* y = A + c * lda;
-  double yi = y[i];
+  if (!have || new_pos <= (int)i) return;
+  double yi = y[0];
   if (t != 0.0) {
     double s = 0.0;
-    for (int64_t r = i + lane; r < m; r += 64) s += (r == i ? 1.0 : v[r]) * y[r];
+#pragma unroll
+    for (int q = 0; q < kPqrKeep; ++q) {
+      const int64_t r = lane + 64 * q;
+      if (r < len) s += (r == 0 ? 1.0 : v_at(r)) * yk[q];
+    }
+    for (int64_t r = lane + 64 * kPqrKeep; r < len; r += 64) s += v_at(r) * y[r];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
     const double wv = t * s;
-    for (int64_t r = i + lane; r < m; r += 64) y[r] -= (r == i ? 1.0 : v[r]) * wv;
+#pragma unroll
+    for (int q = 0; q < kPqrKeep; ++q) {
+      const int64_t r = lane + 64 * q;
+      if (r < len) {
+        yk[q] -= (r == 0 ? 1.0 : v_at(r)) * wv;
+        y[r] = yk[q];
+      }
+    }
+    for (int64_t r = lane + 64 * kPqrKeep; r < len; r += 64) y[r] -= v_at(r) * wv;
     yi -= wv;
   }
-  const double n1 = vn1[c];
+  double nv = n1;
   if (n1 != 0.0) {
     double temp = fabs(yi) / n1;
     temp = fmax(1.0 - temp * temp, 0.0);
     const double r2 = n1 / vn2[c];
     if (temp * r2 * r2 <= kTol3z) {
       double s = 0.0;
-      for (int64_t r = i + 1 + lane; r < m; r += 64) s += y[r] * y[r];
-      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-      if (lane == 0) {
-        const double nv = (i + 1 < m) ? sqrt(s) : 0.0;
-        vn1[c] = nv;
-        vn2[c] = nv;
+#pragma unroll
+      for (int q = 0; q < kPqrKeep; ++q) {
+        const int64_t r = lane + 64 * q;
+        if (r > 0 && r < len) s += yk[q] * yk[q];
       }
-    } else if (lane == 0) {
-      vn1[c] = n1 * sqrt(temp);
+      for (int64_t r = lane + 64 * kPqrKeep; r < len; r += 64) s += y[r] * y[r];
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+      nv = len > 1 ? sqrt(s) : 0.0;
+      if (lane == 0) vn2[c] = nv;
+    } else {
+      nv = n1 * sqrt(temp);
     }
+  }
+  if (lane == 0) vn1_out[c] = nv;
+}
+
+// LAPACK's layout of the result: column place j of Out is column c = perm[j]
+// with the rows above the diagonal from A, the diagonal from betas and the
+// reflector below it.
+__global__ void __launch_bounds__(256)
+pqr_gather_kernel(int64_t m, int64_t n, int64_t kmax, const double* __restrict__ A, int64_t lda,
+                  const int* __restrict__ pos, const double* __restrict__ V,
+                  const double* __restrict__ betas, double* __restrict__ Out,
+                  int* __restrict__ perm) {
+  const int64_t c = blockIdx.x, j = pos[c];
+  if (threadIdx.x == 0) perm[j] = (int)c;
+  for (int64_t r = threadIdx.x; r < m; r += 256) {
+    double v = A[r + c * lda];
+    if (j < kmax && r == j) v = betas[j];
+    if (j < kmax && r > j) v = V[r + j * m];
+    Out[r + j * m] = v;
   }
 }
 
@@ -266,25 +321,37 @@ int pivoted_qr_f64(Context* c, int64_t m, int64_t n, double* A, int64_t lda, int
                    double* tau) {
   if (m <= 0 || n <= 0) return 0;
   if (lda < m) return set_error("pivoted_qr: lda %lld < m %lld", (long long)lda, (long long)m);
-  DBuf<double> vn1, vn2;
-  RSVD_TRY(vn1.alloc((size_t)n));
-  RSVD_TRY(vn2.alloc((size_t)n));
-  KTimer kt(c, "pivoted_qr");
-  hipLaunchKernelGGL(pqr_init_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, c->stream, m,
-                     n, (const double*)A, lda, vn1.p, vn2.p, perm);
-  RSVD_LAUNCH_CHECK();
   const int64_t kmax = m < n ? m : n;
+  DBuf<double> vn1, vn2, V, betas, W;
+  DBuf<int> pos;
+  RSVD_TRY(vn1.alloc((size_t)(2 * n)));
+  RSVD_TRY(vn2.alloc((size_t)n));
+  RSVD_TRY(pos.alloc((size_t)(2 * n)));
+  RSVD_TRY(V.alloc((size_t)(m * kmax)));
+  RSVD_TRY(betas.alloc((size_t)kmax));
+  RSVD_TRY(W.alloc((size_t)(m * n)));
+  KTimer kt(c, "pivoted_qr");
+  const dim3 grid((unsigned)((n + 3) / 4));
+  hipLaunchKernelGGL(pqr_init_kernel, grid, dim3(256), 0, c->stream, m, n, (const double*)A, lda,
+                     vn1.p, vn2.p, pos.p);
+  RSVD_LAUNCH_CHECK();
   for (int64_t i = 0; i < kmax; ++i) {
-    hipLaunchKernelGGL(pqr_pivot_kernel, dim3(1), dim3(1024), 0, c->stream, m, n, A, lda, i,
-                       vn1.p, vn2.p, perm, tau);
+    const int64_t in = (i & 1) * n, out = n - in;
+    if (m - i <= kPqrLds)
+      hipLaunchKernelGGL(pqr_step_kernel<true>, grid, dim3(256), 0, c->stream, m, n, A, lda, i,
+                         (const double*)(vn1.p + in), vn1.p + out, vn2.p,
+                         (const int*)(pos.p + in), pos.p + out, V.p, betas.p, tau);
+    else
+      hipLaunchKernelGGL(pqr_step_kernel<false>, grid, dim3(256), 0, c->stream, m, n, A, lda, i,
+                         (const double*)(vn1.p + in), vn1.p + out, vn2.p,
+                         (const int*)(pos.p + in), pos.p + out, V.p, betas.p, tau);
     RSVD_LAUNCH_CHECK();
-    const int64_t rest = n - i - 1;
-    if (rest > 0) {
-      hipLaunchKernelGGL(pqr_update_kernel, dim3((unsigned)((rest + 3) / 4)), dim3(256), 0,
-                         c->stream, m, n, A, lda, i, vn1.p, vn2.p, (const double*)tau);
-      RSVD_LAUNCH_CHECK();
-    }
   }
+  hipLaunchKernelGGL(pqr_gather_kernel, dim3((unsigned)n), dim3(256), 0, c->stream, m, n, kmax,
+                     (const double*)A, lda, (const int*)(pos.p + (kmax & 1) * n),
+                     (const double*)V.p, (const double*)betas.p, W.p, perm);
+  RSVD_LAUNCH_CHECK();
+  RSVD_TRY(copy2d_f64(c, m, n, W.p, m, A, lda));
   return 0;
 }
 
