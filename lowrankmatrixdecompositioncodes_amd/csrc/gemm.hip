@@ -32,6 +32,9 @@
 //         i = 4*r + l/16     for v_mfma_f64_16x16x4f64
 // srcA is fed from op(B) and srcB from op(A), so accumulator lanes run along M
 // and the epilogue writes contiguous segments of column-major C.
+//
+// The same kernel with the FP32 operands rounded (or split) to bf16 in registers
+// serves the smaller products of gemm_lp.hip.
 #include <algorithm>
 #include <climits>
 #include <type_traits>
@@ -44,6 +47,7 @@ namespace rsvd {
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
 template <typename T>
 struct Mfma;
@@ -231,7 +235,11 @@ __host__ __device__ __forceinline__ int64_t sym_tiles(int64_t tn, int64_t gx, in
 // A workgroup (four waves) owns a (16 TM WM) x (16 TN WN) tile of C; KS = 4 /
 // (WM WN) waves share a wave tile and deal its k blocks among them, their
 // partial tiles added in wave order through LDS at the end.
-template <typename T, bool TA, bool TB, int TM, int TN, int WM, int WN>
+// SPLIT (FP32 operands): 0 multiplies on the FP32 matrix cores; 1 rounds the
+// operands to bf16, 3 splits them into bf16 hi + lo and takes hi hi + hi lo + lo
+// hi (gemm_lp.hip), both in registers on the way to v_mfma_f32_16x16x32_bf16 --
+// one MFMA (three) for the 32-deep block, the same accumulator layout.
+template <typename T, bool TA, bool TB, int TM, int TN, int WM, int WN, int SPLIT = 0>
 __global__ void __launch_bounds__(kThreads, 2)
 gemm_kernel(const GemmArgs<T> g) {
   constexpr int KS = 4 / (WM * WN);
@@ -295,6 +303,33 @@ gemm_kernel(const GemmArgs<T> g) {
     typename OpB::Raw b0, b1;
     T fa[TM][SS], fb[TN][SS];
     auto mma = [&]() {
+      if constexpr (SPLIT != 0) {
+        bf16x8_t ah[TM], al[TM], bh[TN], bl[TN];
+        auto cut = [](const T(&x)[KBlock<T>::kSteps], bf16x8_t& h, bf16x8_t& l) {
+#pragma unroll
+          for (int s = 0; s < KBlock<T>::kSteps; ++s) {
+            const __bf16 v = (__bf16)x[s];
+            h[s] = v;
+            if (SPLIT == 3) l[s] = (__bf16)(x[s] - (float)v);
+          }
+        };
+#pragma unroll
+        for (int a = 0; a < TN; ++a) cut(fb[a], bh[a], bl[a]);
+#pragma unroll
+        for (int b = 0; b < TM; ++b) cut(fa[b], ah[b], al[b]);
+#pragma unroll
+        for (int a = 0; a < TN; ++a)
+#pragma unroll
+          for (int b = 0; b < TM; ++b) {
+            f4_t d = acc[a][b];
+            if (SPLIT == 3) {
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[a], al[b], d, 0, 0, 0);
+              d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bl[a], ah[b], d, 0, 0, 0);
+            }
+            acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bh[a], ah[b], d, 0, 0, 0);
+          }
+        return;
+      }
 #pragma unroll
       for (int s = 0; s < SS; ++s)
 #pragma unroll
@@ -473,13 +508,17 @@ struct GemmPlan {
 // measured on 25 shapes (26 to 50000 rows, 20 to 1792 columns), its choice was
 // within 8% of the fastest.
 template <typename T>
-static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice) {
+static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice,
+                          int split = 0) {
   static const struct {
     int bm, bn, ks, mfma;
     double slow;  // measured time over the MFMAs' (operand loads a wave does not share)
   } kTiles[3] = {{128, 64, 1, 8, 1.0}, {64, 32, 4, 8, 1.05}, {32, 32, 4, 4, 1.05}};
   constexpr int64_t depth = KBlock<T>::kDepth;
-  constexpr double kMfmaUs = (sizeof(T) == 8 ? 64.0 : 32.0) / 2400.0;
+  // cycles of a 16 x 16 block of C and a k block; the split modes wait for their
+  // operands (1.5 to 2 KB a block) far longer than for their MFMAs (16 each)
+  const double block_us = (split == 0 ? (sizeof(T) == 8 ? 64.0 : 32.0) * KBlock<T>::kSteps
+                                      : 250.0) / 2400.0;
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
   GemmPlan best{};
@@ -505,7 +544,7 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
     for (int64_t s = smin; s <= smax; ++s) {
       const int64_t kb = (kblocks + s - 1) / s;
       if ((kblocks + kb - 1) / kb != s && s > smin) continue;  // as with a smaller s
-      const double wave = (double)((kb + d.ks - 1) / d.ks) * d.mfma * KBlock<T>::kSteps * kMfmaUs;
+      const double wave = (double)((kb + d.ks - 1) / d.ks) * d.mfma * block_us;
       double cost = (double)((tiles * s + cus - 1) / cus) * (wave * d.slow + 0.5);
       if (s > 1) cost += 2.0 + 2e-6 * (double)s * (double)M * (double)N * sizeof(T) / 8;
       if (cost < best_cost) {
@@ -517,17 +556,20 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
   return best;
 }
 
-template <typename T, bool TA, bool TB>
+template <typename T, bool TA, bool TB, int SPLIT>
 static void gemm_launch_tile(Context* c, int tile, dim3 grid, const GemmArgs<T>& g) {
   if (tile == kTile128x64)
-    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 2, 2>), grid, dim3(kThreads), 0, c->stream, g);
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 2, 2, SPLIT>), grid, dim3(kThreads), 0,
+                       c->stream, g);
   else if (tile == kTile64x32)
-    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 1, 1>), grid, dim3(kThreads), 0, c->stream, g);
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 4, 2, 1, 1, SPLIT>), grid, dim3(kThreads), 0,
+                       c->stream, g);
   else
-    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 2, 2, 1, 1>), grid, dim3(kThreads), 0, c->stream, g);
+    hipLaunchKernelGGL((gemm_kernel<T, TA, TB, 2, 2, 1, 1, SPLIT>), grid, dim3(kThreads), 0,
+                       c->stream, g);
 }
 
-template <typename T>
+template <typename T, int SPLIT = 0>
 static int launch_gemm(Context* c, const GemmPlan& pl, char ta, char tb, int64_t M, int64_t N,
                        int64_t K, T alpha, const T* A, int64_t lda, const T* B, int64_t ldb, T beta,
                        T* C, int64_t ldc, double* sumsq_partials, bool sym, const char* tag) {
@@ -546,10 +588,10 @@ static int launch_gemm(Context* c, const GemmPlan& pl, char ta, char tb, int64_t
     KTimer kt(c, tag);
     const dim3 grid((unsigned)pl.tiles, (unsigned)pl.splits);
     const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
-    if (!tA && !tB) gemm_launch_tile<T, false, false>(c, pl.tile, grid, g);
-    else if (tA && !tB) gemm_launch_tile<T, true, false>(c, pl.tile, grid, g);
-    else if (!tA && tB) gemm_launch_tile<T, false, true>(c, pl.tile, grid, g);
-    else gemm_launch_tile<T, true, true>(c, pl.tile, grid, g);
+    if (!tA && !tB) gemm_launch_tile<T, false, false, SPLIT>(c, pl.tile, grid, g);
+    else if (tA && !tB) gemm_launch_tile<T, true, false, SPLIT>(c, pl.tile, grid, g);
+    else if (!tA && tB) gemm_launch_tile<T, false, true, SPLIT>(c, pl.tile, grid, g);
+    else gemm_launch_tile<T, true, true, SPLIT>(c, pl.tile, grid, g);
     RSVD_LAUNCH_CHECK();
   }
   if (pl.splits > 1) {
@@ -652,6 +694,18 @@ static int gemm_any(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t 
   const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == T(0);
   return launch_gemm<T>(c, gemm_plan<T>(c, M, N, K, sym, false), ta, tb, M, N, K, alpha, A, lda, B,
                         ldb, beta, C, ldc, nullptr, sym, tag);
+}
+
+int gemm_split(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t N, int64_t K,
+               float alpha, const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
+               float* C, int64_t ldc, int split) {
+  const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
+  const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == 0.0f;
+  const GemmPlan pl = gemm_plan<float>(c, M, N, K, sym, false, split);
+  return split == 1 ? launch_gemm<float, 1>(c, pl, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C,
+                                            ldc, nullptr, sym, tag)
+                    : launch_gemm<float, 3>(c, pl, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C,
+                                            ldc, nullptr, sym, tag);
 }
 
 int gemm_f64(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t K, double alpha,

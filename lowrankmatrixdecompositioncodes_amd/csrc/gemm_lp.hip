@@ -388,6 +388,21 @@ __global__ void splitk_reduce_f32_kernel(int64_t M, int64_t N, int splits,
   }
 }
 
+// Products that leave the 128 x 128 tiles and the A-streaming kernel short of
+// workgroups: the small-tile kernel of gemm.hip, which rounds its operands in
+// registers.  Measured before and here, split-bf16: Grams up to 1024 columns
+// always (101 columns of 5003 rows 47 and 9 us, 544 of 65536 194 and 162 us, 256 of
+// 50000 78 and 45 us); others up to 4 GFLOP (1024 x 64 x 512 39 and 6 us, 2000 x 64 x
+// 2000 134 and 14 us, 5003 x 101 x 3001 54 and 47 us).  Past it the operands that
+// the staged tiles share win: 3000 x 3000 x 300 53 us there, 80 us here.
+static bool lp_direct(bool tA, bool tB, int64_t M, int64_t N, int64_t K, const float* A,
+                      int64_t lda, const float* B, int64_t ldb, float beta, int split) {
+  if (split == 6 || M == 0 || N == 0 || K == 0) return false;
+  if (M > 65535LL * LBM || N > 65535LL * LBN) return false;  // as the tiled kernel's grid
+  const bool gram = A == B && lda == ldb && tA && !tB && M == N && beta == 0.0f && N <= 1024;
+  return gram || 2.0 * (double)M * (double)N * (double)K <= 4e9;
+}
+
 int gemm_bf16(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t N, int64_t K,
               float alpha, const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
               float* C, int64_t ldc, int split) {
@@ -396,7 +411,8 @@ int gemm_bf16(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t 
   const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   // skinny right operand and enough row blocks to fill the GPU: the
   // A-streaming kernel, which reads op(A) once
-  if (M > 0 && N > 0 && K >= 32 && !tB && apass_suitable(c, M, N))
+  if (M > 0 && N > 0 && K >= 32 && !tB && apass_suitable(c, M, N) &&
+      !lp_direct(tA, tB, M, N, K, A, lda, B, ldb, beta, split))
     return apass_bf16(c, tag, tA, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, split);
   return gemm_bf16_general(c, tag, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, split);
 }
@@ -506,6 +522,11 @@ int gemm_bf16_general(Context* c, const char* tag, char ta, char tb, int64_t M, 
   if (M < 0 || N < 0 || K < 0) return set_error("gemm_bf16: negative dimension");
   if (M == 0 || N == 0) return 0;
   if (K == 0) return gemm_f32(c, ta, tb, M, N, 0, alpha, A, lda, B, ldb, beta, C, ldc);
+  if (split != 1 && split != 3 && split != 6)
+    return set_error("gemm_bf16: split must be 1, 3 or 6");
+  const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
+  if (lp_direct(tA, tB, M, N, K, A, lda, B, ldb, beta, split))
+    return gemm_split(c, tag, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, split);
   return gemm_bf16_tiled(c, tag, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, split,
                          nullptr);
 }

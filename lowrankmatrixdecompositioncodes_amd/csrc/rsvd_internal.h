@@ -236,6 +236,11 @@ int gemm_bf16(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t 
 int gemm_bf16_deflate(Context* c, int64_t M, int64_t N, int64_t K, const float* Q, int64_t ldq,
                       const float* Bt, int64_t ldbt, float* C, int64_t ldc, double* sumsq,
                       int64_t klo);
+// The small-tile kernel of gemm.hip in bf16 (split 1) or split-bf16 (split 3), for
+// the products that gemm_bf16 chooses it for.
+int gemm_split(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t N, int64_t K,
+               float alpha, const float* A, int64_t lda, const float* B, int64_t ldb, float beta,
+               float* C, int64_t ldc, int split);
 // C = C - Qp*Bp with fused FP64 sum of squares of the updated C into *sumsq
 // (device scalar, overwritten).
 int gemm_f64_deflate(Context* c, int64_t M, int64_t N, int64_t K, const double* Q, int64_t ldq,
