@@ -13,12 +13,22 @@
 //            tile of one matrix, split-bf16 matrix cores with fp32
 //            accumulation, A_i streamed once; work items of all matrices in
 //            one grid, largest matrices first
-//   borth    CholeskyQR2 of Y_i (m_i x 48) per matrix: FP64 Gram, FP64
-//            Cholesky in LDS (first pass shifted by 1e-14 tr G so it never
-//            breaks down), Y <- Y R^-1, twice
-//   bfinal   G = B B^T (FP64, from B^T = A^T Q), two-sided Jacobi in LDS,
-//            ascending eigenvalues, sigma = sqrt(lambda), last k kept
-//            (rra.c:175-225), U = Q Uhat, V = B^T Uhat Sigma^-1
+//   bgram    FP64 Gram partials of the 256-row slabs of Y_i (or Z_i, x 48)
+//   bchol    per matrix: the partials' sum, FP64 Cholesky in LDS (first pass
+//            shifted by 1e-14 tr G so it never breaks down), R^-1
+//   bapply   per slab: X <- X R^-1; the first pass of CholeskyQR2 forms the next
+//            pass's Gram partial from the rows it has just written, the second
+//            writes the rows tiled for the pass over A as well
+//   bjacobi  per matrix: G = B B^T (FP64, from B^T = A^T Q), two-sided Jacobi in
+//            LDS, ascending eigenvalues, sigma = sqrt(lambda), last k kept
+//            (rra.c:175-225)
+//   bout     per slab: U = Q Uhat and V = B^T Uhat Sigma^-1
+// The row work is cut into slabs so that a large matrix is spread over as many
+// workgroups as it has slabs: with one workgroup a matrix for the whole of
+// CholeskyQR2 (and for the whole final stage), the largest of the batch set the
+// time of 200 matrices and the chunks' latencies that of 4096 (orth Y / orth Z /
+// final: 0.38 / 0.25 / 0.47 ms and 1.64 / 1.06 / 2.55 ms; now 0.12 / 0.09 / 0.42 and
+// 1.13 / 0.45 / 2.35, the tiling of Q for the next pass included).
 // Sketch widths are padded to 48 columns (three 16-wide tiles; l_i = k_i + p
 // <= 48), padding columns are zero throughout.  The pass kernels have
 // variants (rows per wave RT = 1, 2, 4) chosen per batch layout by timing
@@ -38,6 +48,7 @@
 #include <numeric>
 #include <vector>
 
+#include "chol16.h"
 #include "jacobi_rot.h"
 #include "rng.h"
 #include "rsvd_internal.h"
@@ -63,6 +74,7 @@ struct BMat {
   int64_t t;      // tiled skinny operand (bf16x8 units), 2 planes x KB x 3 x 64
   int64_t kbmax;  // KB capacity of the tile slot
   int64_t u, s, v;  // outputs: U (m x k, ld m), S (k), V (n x k, ld n)
+  int64_t gy, gz;   // first Gram partial of Y_i's and Z_i's slabs
   uint64_t seed;
   int32_t aligned;  // A_i rows 16-byte aligned (m % 4 == 0 and offset % 4 == 0)
   int32_t pad;
@@ -100,15 +112,14 @@ __global__ void bomega_kernel(const BMat* __restrict__ mats, float* __restrict__
 }
 
 // ---------------------------------------------------------------- tiling
-// item = (matrix, k block); 192 threads: tile nt = tid / 64, lane = tid % 64.
-template <bool FROM_Y>
+// Omega to the pass's tiles.  item = (matrix, k block); 192 threads: tile nt = tid / 64, lane = tid % 64.
 __global__ void __launch_bounds__(192)
 btile_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
              const float* __restrict__ work, bf16x8_t* __restrict__ tiles) {
   const BItem it = items[blockIdx.x];
   const BMat d = mats[it.mat];
-  const int64_t K = FROM_Y ? d.m : d.n;
-  const float* X = work + (FROM_Y ? d.y : d.z);
+  const int64_t K = d.n;
+  const float* X = work + d.z;
   const int64_t KB = (K + 31) / 32;
   const int64_t kb = it.tile;
   const int nt = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -287,11 +298,9 @@ __device__ __forceinline__ void chunk_store(float (*Xs)[kL + 1], const float (&p
 // holds X[i = l % 16][k = l / 16], srcB lane l holds Y[k = l / 16][j = l % 16],
 // and the accumulator's register r of lane l holds D[4 r + l / 16][l % 16].
 
-// Gram G = X^T X (both triangles; FP64 products of the fp32 entries, exact,
-// and FP64 accumulation) of X (R x 48, ld R, first l columns, zero beyond),
-// staged in 64-row chunks.  Wave w takes rows 16 w .. 16 w + 15 of every
-// chunk (four k steps of 4) for the six upper 16 x 16 tiles; the waves'
-// partial tiles are added in wave order at the end (deterministic).
+// Gram X^T X of X (R x 48, ld R, first l columns, zero beyond): FP64 products of
+// the fp32 entries (exact) and FP64 accumulation, staged in 64-row chunks; only
+// the six upper 16 x 16 tiles are formed.
 // One staged chunk's contribution to the wave's six upper 16 x 16 Gram tiles
 // (wave w: chunk rows 16 w .. 16 w + 15, four k steps of 4).
 __device__ __forceinline__ void gram_chunk(const float (*Xs)[kL + 1], d4_t (&acc)[6]) {
@@ -311,62 +320,20 @@ __device__ __forceinline__ void gram_chunk(const float (*Xs)[kL + 1], d4_t (&acc
   }
 }
 
-// G (both triangles) = the sum of the four waves' tiles, added in wave order.
-__device__ void gram_store(const d4_t (&acc)[6], double (*G)[kLP]) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int li = lane & 15, lk = lane >> 4;
-  const int ti[6] = {0, 0, 0, 1, 1, 2}, tj[6] = {0, 1, 2, 1, 2, 2};
-  for (int w = 0; w < 4; ++w) {
-    __syncthreads();
-    if (wave == w) {
-#pragma unroll
-      for (int t = 0; t < 6; ++t)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int i = 16 * ti[t] + 4 * r + lk, j = 16 * tj[t] + li;
-          const double v = (w == 0) ? acc[t][r] : G[i][j] + acc[t][r];
-          G[i][j] = v;
-          if (ti[t] != tj[t]) G[j][i] = v;
-        }
-    }
-  }
-  __syncthreads();
-}
-
-__device__ __forceinline__ void lds_gram(const float* __restrict__ X, int64_t R, int l, float (*Xs)[kL + 1],
-                         double (*G)[kLP]) {
-  d4_t acc[6];
-#pragma unroll
-  for (int t = 0; t < 6; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
-  float pre[kChunkLoads];
-  chunk_fetch(X, R, l, 0, pre);
-  for (int64_t r0 = 0; r0 < R; r0 += 64) {
-    __syncthreads();
-    chunk_store(Xs, pre);
-    __syncthreads();
-    if (r0 + 64 < R) chunk_fetch(X, R, l, r0 + 64, pre);  // in flight during the MFMAs
-    gram_chunk(Xs, acc);
-  }
-  gram_store(acc, G);
-}
-
-// borth's Gram as a call of its own: inlined there it raises the kernel's
-// register pressure past the three-workgroup budget (bfinal inlines it)
-__device__ __noinline__ void lds_gram_call(const float* __restrict__ X, int64_t R, int l,
-                                           float (*Xs)[kL + 1], double (*G)[kLP]) {
-  lds_gram(X, R, l, Xs, G);
-}
-
-// P(pi.., pk..) Q(qk.., qj..): one 16 x 16 x 16 product of LDS blocks on the
-// FP64 matrix cores (four k steps of 4; the layout above): lane l's register
-// r holds row 4 r + l / 16, column l % 16 of the product.
+// op(P) Q + acc for 16 x 16 blocks of LDS arrays on the FP64 matrix cores (four k
+// steps of 4; the layout above): op(P) is the block at (pi, pk), or with TA the
+// transpose of the one at (pk, pi).  Lane l's register r holds row 4 r + l / 16,
+// column l % 16.
+template <bool TA>
 __device__ __forceinline__ d4_t mm16(const double (*P)[kLP], int pi, int pk,
                                      const double (*Q)[kLP], int qk, int qj, d4_t acc) {
   const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(P[pi + li][pk + 4 * s + lk],
-                                               Q[qk + 4 * s + lk][qj + li], acc, 0, 0, 0);
+  for (int s = 0; s < 4; ++s) {
+    const int k = 4 * s + lk;
+    const double p = TA ? P[pk + k][pi + li] : P[pi + li][pk + k];
+    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(p, Q[qk + k][qj + li], acc, 0, 0, 0);
+  }
   return acc;
 }
 __device__ __forceinline__ void st16(double (*C)[kLP], int ci, int cj, const d4_t& v,
@@ -376,186 +343,278 @@ __device__ __forceinline__ void st16(double (*C)[kLP], int ci, int cj, const d4_
   for (int r = 0; r < 4; ++r) C[ci + 4 * r + lk][cj + li] = scale * v[r];
 }
 
-// Ri = R^-1 for the upper-triangular R in G (kL x kL; rows and columns >= l
-// zero, rinv[i] = 1 / R_ii for i < l), by 16 x 16 blocks: the three diagonal
-// blocks D_b = R_bb^-1 at once (48 threads, one column each, column-oriented
-// substitution in registers: a step is one multiply and independent
-// multiply-adds), then on the FP64 matrix cores
-//   Ri01 = -D0 R01 D1,  Ri12 = -D1 R12 D2,  Ri02 = -D0 (R01 Ri12 + R02 D2).
-// Entries in rows or columns >= l, and below the diagonal, are zero.
-__device__ __forceinline__ void blocked_tri_inv(const double (*G)[kLP], double (*Ri)[kLP], int l,
-                                const double* rinv) {
-  static_assert(kL == 48, "three 16 x 16 blocks");
-  const int tid = threadIdx.x, wave = tid >> 6;
-  // the lower blocks are zero
-  for (int e = tid; e < 3 * 256; e += 256) {
-    const int t = e >> 8, i = (e >> 4) & 15, j = e & 15;
-    const int bi = t == 0 ? 1 : 2, bj = t == 2 ? 1 : 0;
-    Ri[16 * bi + i][16 * bj + j] = 0.0;
-  }
-  if (tid < 48) {
-    const int b = tid >> 4, cc = tid & 15, o = 16 * b;
-    double x[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) x[r] = (r == cc && o + cc < l) ? 1.0 : 0.0;
-#pragma unroll
-    for (int r = 15; r >= 0; --r) {
-      x[r] *= (o + r < l) ? rinv[o + r] : 0.0;
-#pragma unroll
-      for (int q = 0; q < r; ++q) x[q] = fma(-G[o + q][o + r], x[r], x[q]);
-      // keep each step's reads in the step (hoisted together they spill)
-      __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-    for (int r = 0; r < 16; ++r) Ri[o + r][o + cc] = x[r];
-  }
-  __syncthreads();
-  // T01 = R01 D1 and T12 = R12 D2 into the (still free) blocks of Ri01, Ri12
+// One wave's LDS operations complete in order; this keeps the compiler from
+// moving them across.
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// One wave: the upper triangle of G (kL x kL, LDS, rows and columns >= l zero)
+// becomes R^-1 of its Cholesky factor G = R^T R, by 16 x 16 blocks: a diagonal
+// block is factored and inverted in registers (chol16.h), what couples the blocks
+// runs on the FP64 matrix cores.  Diagonal blocks come out with zeros below the
+// diagonal, the strictly lower blocks are not touched, and rows and columns >= l
+// are zero.  False if a pivot was not positive (it counted as 1).
+__device__ __forceinline__ bool wave_chol_inv(double (*G)[kLP], int l) {
+  static_assert(kNT == 3, "the inverse below is written out for three blocks");
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const d4_t z = {0.0, 0.0, 0.0, 0.0};
-  if (wave == 0) st16(Ri, 0, 16, mm16(G, 0, 16, Ri, 16, 16, z), 1.0);
-  if (wave == 1) st16(Ri, 16, 32, mm16(G, 16, 32, Ri, 32, 32, z), 1.0);
-  __syncthreads();
-  // Ri01 = -D0 T01, Ri12 = -D1 T12, in place: a wave reads its whole block
-  // through the products before its stores (LDS operations of one wave stay
-  // in program order)
-  if (wave == 0) st16(Ri, 0, 16, mm16(Ri, 0, 0, Ri, 0, 16, z), -1.0);
-  if (wave == 1) st16(Ri, 16, 32, mm16(Ri, 16, 16, Ri, 16, 32, z), -1.0);
-  __syncthreads();
-  if (wave == 0) {
-    // U = R01 Ri12 + R02 D2 into Ri02's block, then Ri02 = -D0 U in place
-    st16(Ri, 0, 32, mm16(G, 0, 32, Ri, 32, 32, mm16(G, 0, 16, Ri, 16, 32, z)), 1.0);
-    st16(Ri, 0, 32, mm16(Ri, 0, 0, Ri, 0, 32, z), -1.0);
-  }
-  __syncthreads();
-}
-
-// In-place upper Cholesky of G (l x l, upper triangle used) -> R in the upper
-// triangle (G = R^T R, zero below), then Ri = R^-1 (upper).  shift is added
-// to the diagonal first.  Returns through *ok (shared) whether every pivot
-// was positive (a non-positive one is replaced by 1).
-// Factorisation: unnormalised right-looking elimination, one barrier per
-// step: thread (row a = tid % 64, columns 12 (tid / 64) ..) keeps its 12
-// entries in registers, subtracts U_j,a U_j,c / U_j,j at step j and publishes
-// row j + 1 when it owns it.  Inverse: blocked_tri_inv.
-__device__ __noinline__ void lds_chol_inv(double (*G)[kLP], double (*Ri)[kLP], int l, double shift, int* ok) {
-  __shared__ double piv[kL], inv[kL];
-  const int tid = threadIdx.x, a = tid & 63, c0 = (tid >> 6) * 12;
-  if (tid == 0) *ok = 1;
-  if (tid < l) G[tid][tid] += shift;
-  __syncthreads();
-  double own[12];
+  bool bad = false;
+#pragma unroll 1
+  for (int h = 0; h < kNT; ++h) {
+    const int o = 16 * h, kh = l - o;
+    double a[16], e[16];
 #pragma unroll
-  for (int q = 0; q < 12; ++q) own[q] = (a < l && c0 + q < l) ? G[a][c0 + q] : 0.0;
-  for (int j = 0; j < l; ++j) {
-    double d = G[j][j];
-    const bool good = d > 0.0;
-    if (!good) d = 1.0;
-    if (tid == 0) {
-      if (!good) *ok = 0;
-      piv[j] = d;
+    for (int r = 0; r < 16; ++r) {
+      a[r] = G[o + (r < c ? r : c)][o + (r < c ? c : r)];
+      e[r] = (r == c) ? 1.0 : 0.0;
     }
-    if (a > j && a < l) {
-      const double u = G[j][a] * rcp_nr(d);  // reciprocal: off the division path
+    double piv = 1.0;
+    chol16_step<0, true>(a, e, c, kh, &piv);
+    bad |= c < kh && !(piv > 0.0);
+    wave_fence();
+    // row group g of the wave stores a quarter of X_hh = R_hh^-1
 #pragma unroll
-      for (int q = 0; q < 12; ++q)
-        if (c0 + q >= a && c0 + q < l) own[q] -= u * G[j][c0 + q];
-      if (a == j + 1) {
+    for (int r = 0; r < 16; ++r)
+      if ((r >> 2) == g) G[o + c][o + r] = (r < kh && c < kh) ? e[r] : 0.0;
+    wave_fence();
+    // R_hj = X_hh^T G_hj, then G_ij -= R_hi^T R_hj
+    for (int j = h + 1; j < kNT; ++j) {
+      const d4_t p = mm16<true>(G, o, o, G, o, 16 * j, z);
+      wave_fence();
+      st16(G, o, 16 * j, p, 1.0);
+    }
+    wave_fence();
+    for (int j = h + 1; j < kNT; ++j)
+      for (int i = h + 1; i <= j; ++i) {
+        const d4_t p = mm16<true>(G, 16 * i, o, G, o, 16 * j, z);
 #pragma unroll
-        for (int q = 0; q < 12; ++q)
-          if (c0 + q >= a && c0 + q < l) G[a][c0 + q] = own[q];
+        for (int r = 0; r < 4; ++r) G[16 * i + 4 * r + g][16 * j + c] -= p[r];
+        wave_fence();
       }
-    }
-    __syncthreads();
   }
-  if (tid < l) {
-    const double sj = sqrt(piv[tid]);
-    piv[tid] = sj;
-    inv[tid] = 1.0 / sj;
-  }
-  __syncthreads();
-  for (int e = tid; e < kL * kL; e += 256) {
-    const int i = e % kL, c = e / kL;
-    double v = 0.0;
-    if (i < l && c < l) v = (c > i) ? G[i][c] * inv[i] : (c == i ? piv[i] : 0.0);
-    G[i][c] = v;
-  }
-  __syncthreads();
-  blocked_tri_inv(G, Ri, l, inv);
+  // X12 = -X1 (R12 X2), X02 = -X0 (R01 X12 + R02 X2), X01 = -X0 (R01 X1), each
+  // product read whole before it is stored
+  auto put = [&](int i, int j, const d4_t& v, double scale) {
+    wave_fence();
+    st16(G, i, j, v, scale);
+    wave_fence();
+  };
+  put(16, 32, mm16<false>(G, 16, 32, G, 32, 32, z), 1.0);
+  put(16, 32, mm16<false>(G, 16, 16, G, 16, 32, z), -1.0);
+  put(0, 32, mm16<false>(G, 0, 32, G, 32, 32, mm16<false>(G, 0, 16, G, 16, 32, z)), 1.0);
+  put(0, 32, mm16<false>(G, 0, 0, G, 0, 32, z), -1.0);
+  put(0, 16, mm16<false>(G, 0, 16, G, 16, 16, z), 1.0);
+  put(0, 16, mm16<false>(G, 0, 0, G, 0, 16, z), -1.0);
+  return __builtin_amdgcn_ballot_w64(bad) == 0;
 }
 
-// out (R x kout, ld ldo) = scale_j * X W for X (R x 48, ld R, first l
-// columns used) and W (48 x kout, LDS, FP64; rows >= l must be finite), in
-// 64-row chunks staged in LDS, on the FP64 matrix cores: wave w computes rows
-// 16 w .. 16 w + 15 of the chunk against the three 16-column tiles of W
-// (twelve k steps of 4).  The results go back through the chunk's LDS so the
-// stores are coalesced; out may alias X (each chunk is fully read first).
-__device__ void lds_rows_times(const float* X, int64_t R, int l, float (*Xs)[kL + 1],
-                               const double (*W)[kLP], int kout, const double* scale, float* out,
-                               int64_t ldo) {
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+// One staged 64-row chunk times W (48 x 48, LDS, FP64; rows >= l finite), on the
+// FP64 matrix cores: wave w computes rows 16 w .. 16 w + 15 of the chunk against
+// the three 16-column tiles of W (twelve k steps of 4); the results, scaled by
+// column and rounded to float, replace the chunk in LDS.  Ends with a barrier.
+__device__ __forceinline__ void chunk_times(float (*Xs)[kL + 1], const double (*W)[kLP],
+                                            const double* scale, int kout) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int li = lane & 15, lk = lane >> 4;
-  float pre[kChunkLoads];
-  chunk_fetch(X, R, l, 0, pre);
-  for (int64_t r0 = 0; r0 < R; r0 += 64) {
-    const int rows = (int)((R - r0) < 64 ? (R - r0) : 64);
-    __syncthreads();
-    chunk_store(Xs, pre);
-    __syncthreads();
-    // the next chunk's rows are disjoint from this chunk's output rows, so the
-    // prefetch is safe when out aliases X
-    if (r0 + 64 < R) chunk_fetch(X, R, l, r0 + 64, pre);
-    d4_t acc[kNT];
+  d4_t acc[kNT];
 #pragma unroll
-    for (int t = 0; t < kNT; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < kNT; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int s = 0; s < kL / 4; ++s) {
-      const double a = (double)Xs[16 * wave + li][4 * s + lk];
-#pragma unroll
-      for (int t = 0; t < kNT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, W[4 * s + lk][16 * t + li], acc[t], 0, 0,
-                                                      0);
-    }
-    __syncthreads();  // every wave has read the chunk
+  for (int s = 0; s < kL / 4; ++s) {
+    const double a = (double)Xs[16 * wave + li][4 * s + lk];
 #pragma unroll
     for (int t = 0; t < kNT; ++t)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int c = 16 * t + li;
-        const double v = acc[t][r];
-        Xs[16 * wave + 4 * r + lk][c] = (float)((scale && c < kout) ? v * scale[c] : v);
-      }
-    __syncthreads();
-    for (int e = tid; e < 64 * kout; e += 256) {
-      const int r = e & 63, c = e >> 6;
-      if (r < rows) out[r0 + r + (int64_t)c * ldo] = Xs[r][c];
-    }
+      acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, W[4 * s + lk][16 * t + li], acc[t], 0, 0, 0);
   }
+  // a wave reads and writes its own sixteen rows only: its reads above come
+  // before its writes, no barrier in between
+#pragma unroll
+  for (int t = 0; t < kNT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int c = 16 * t + li;
+      const double v = acc[t][r];
+      Xs[16 * wave + 4 * r + lk][c] = (float)((scale && c < kout) ? v * scale[c] : v);
+    }
   __syncthreads();
+}
+
+// Rows of the chunk at r0 (below `end`) and columns below kout to out (ld ldo).
+__device__ __forceinline__ void chunk_write(const float (*Xs)[kL + 1], int64_t r0, int64_t end,
+                                            int kout, float* __restrict__ out, int64_t ldo) {
+  for (int e = threadIdx.x; e < 64 * kout; e += 256) {
+    const int r = e & 63, c = e >> 6;
+    if (r0 + r < end) out[r0 + r + (int64_t)c * ldo] = Xs[r][c];
+  }
 }
 
 // ---------------------------------------------------------------- orth
-// CholeskyQR2 of Y_i (FROM_Z: Z_i) per matrix, one workgroup each.
+constexpr int kSlab = 256;               // rows of a slab (four chunks)
+constexpr int kGramPart = 6 * 256;       // doubles of a Gram partial: six upper tiles
+
+// The workgroup's partial Gram (the four waves' tiles added in wave order) to
+// part, through LDS: each wave in turn adds its tiles.
+__device__ __forceinline__ void gram_partial_out(const d4_t (&acc)[6], double* lds,
+                                                 double* __restrict__ part) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  for (int w = 0; w < 4; ++w) {
+    __syncthreads();
+    if (wave == w) {
+#pragma unroll
+      for (int t = 0; t < 6; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          double* p = lds + t * 256 + r * 64 + lane;
+          *p = (w == 0) ? acc[t][r] : *p + acc[t][r];
+        }
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < kGramPart; e += 256) part[e] = lds[e];
+}
+
+// G (both triangles, LDS) = the sum of a matrix's partials, in slab order, by a
+// workgroup of WAVES waves (1 or 4).
+template <int WAVES>
+__device__ __forceinline__ void gram_partials_in(const double* __restrict__ part, int slabs,
+                                                 double (*G)[kLP]) {
+  constexpr int Q = kGramPart / (64 * WAVES);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  double v[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) v[q] = 0.0;
+  for (int s = 0; s < slabs; ++s)
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      v[q] += part[(int64_t)s * kGramPart + (q * WAVES + wave) * 64 + lane];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const int t = (q * WAVES + wave) >> 2, r = (q * WAVES + wave) & 3;
+    // upper tile t of (0,0) (0,1) (0,2) (1,1) (1,2) (2,2)
+    const int ti = t < 3 ? 0 : (t < 5 ? 1 : 2), tj = t < 3 ? t : (t < 5 ? t - 2 : 2);
+    const int i = 16 * ti + 4 * r + lk, j = 16 * tj + li;
+    G[i][j] = v[q];
+    if (ti != tj) G[j][i] = v[q];
+  }
+  __syncthreads();
+}
+
 template <bool FROM_Z>
-__global__ void __launch_bounds__(256, 3)
-borth_kernel(const BMat* __restrict__ mats, const int* __restrict__ order, float* __restrict__ work,
-             int* __restrict__ flags) {
+__global__ void __launch_bounds__(256, 4)
+bgram_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
+             const float* __restrict__ work, double* __restrict__ gpart) {
   __shared__ float Xs[64][kL + 1];
+  __shared__ double P[kGramPart];
+  const BItem it = items[blockIdx.x];
+  const BMat d = mats[it.mat];
+  const int64_t R = FROM_Z ? d.n : d.m;
+  const float* X = work + (FROM_Z ? d.z : d.y);
+  const int64_t b0 = (int64_t)it.tile * kSlab, end = b0 + kSlab < R ? b0 + kSlab : R;
+  d4_t acc[6];
+#pragma unroll
+  for (int t = 0; t < 6; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
+  float pre[kChunkLoads];
+  chunk_fetch(X, R, d.l, b0, pre);
+  for (int64_t r0 = b0; r0 < end; r0 += 64) {
+    __syncthreads();
+    chunk_store(Xs, pre);
+    __syncthreads();
+    if (r0 + 64 < end) chunk_fetch(X, R, d.l, r0 + 64, pre);  // in flight during the MFMAs
+    gram_chunk(Xs, acc);
+  }
+  gram_partial_out(acc, P, gpart + ((FROM_Z ? d.gz : d.gy) + it.tile) * kGramPart);
+}
+
+// shift: 1 in the first pass of CholeskyQR2.  A wave a matrix, eight to a CU: with
+// four waves and a barrier a pivot (at 38 KB of LDS and 256 registers, one matrix a
+// CU) 4096 matrices took 0.77 ms, here 0.06 ms.
+template <bool FROM_Z>
+__global__ void __launch_bounds__(64)
+bchol_kernel(const BMat* __restrict__ mats, const int* __restrict__ order,
+             const double* __restrict__ gpart, double* __restrict__ rinv, int shift,
+             int* __restrict__ flags) {
   __shared__ double G[kL][kLP];
-  __shared__ double Ri[kL][kLP];
-  __shared__ int ok;
-  const BMat d = mats[order[blockIdx.x]];  // largest first
+  const int mat = order[blockIdx.x];  // largest first
+  const BMat d = mats[mat];
+  const int64_t R = FROM_Z ? d.n : d.m;
+  const int lane = threadIdx.x;
+  gram_partials_in<1>(gpart + (FROM_Z ? d.gz : d.gy) * kGramPart, (int)((R + kSlab - 1) / kSlab),
+                      G);
+  if (shift) {
+    double tr = 0.0;
+    for (int j = 0; j < d.l; ++j) tr += G[j][j];
+    wave_fence();
+    if (lane < d.l) G[lane][lane] += 1e-14 * tr;
+    wave_fence();
+  }
+  if (!wave_chol_inv(G, d.l) && lane == 0) atomicOr(flags, 1);
+  wave_fence();
+  double* out = rinv + (int64_t)mat * kL * kL;
+  for (int e = lane; e < kL * kL; e += 64) {
+    const int i = e / kL, j = e % kL;
+    out[e] = (i >> 4) <= (j >> 4) ? G[i][j] : 0.0;
+  }
+}
+
+// One slab of X <- X R^-1.  LAST = false: the Gram partial of the new rows;
+// true: the new rows rounded to the pass's split-bf16 tiles as well.
+template <bool FROM_Z, bool LAST>
+__global__ void __launch_bounds__(256, 4)
+bapply_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
+              float* __restrict__ work, const double* __restrict__ rinv,
+              double* __restrict__ gpart, bf16x8_t* __restrict__ tiles) {
+  __shared__ float Xs[64][kL + 1];
+  __shared__ __align__(16) double W[kL][kLP];
+  static_assert(kL * kLP >= kGramPart, "the partial Gram takes W's place at the end");
+  const BItem it = items[blockIdx.x];
+  const BMat d = mats[it.mat];
   const int64_t R = FROM_Z ? d.n : d.m;
   float* X = work + (FROM_Z ? d.z : d.y);
-  const int l = d.l;
-  for (int pass = 0; pass < 2; ++pass) {
-    lds_gram_call(X, R, l, Xs, G);
-    double tr = 0.0;
-    for (int j = 0; j < l; ++j) tr += G[j][j];
-    __syncthreads();  // every thread has read the diagonal before it is shifted
-    lds_chol_inv(G, Ri, l, pass == 0 ? 1e-14 * tr : 0.0, &ok);
-    if (!ok && threadIdx.x == 0) atomicOr(flags, 1);
-    lds_rows_times(X, R, l, Xs, Ri, l, nullptr, X, R);
+  const int64_t b0 = (int64_t)it.tile * kSlab, end = b0 + kSlab < R ? b0 + kSlab : R;
+  const int tid = threadIdx.x, lane = tid & 63;
+  float pre[kChunkLoads];
+  chunk_fetch(X, R, d.l, b0, pre);
+  const double* Wg = rinv + (int64_t)it.mat * kL * kL;
+  for (int e = tid; e < kL * kL; e += 256) W[e / kL][e % kL] = Wg[e];
+  d4_t acc[6];
+#pragma unroll
+  for (int t = 0; t < 6; ++t) acc[t] = d4_t{0.0, 0.0, 0.0, 0.0};
+  const int64_t KB = (R + 31) / 32;
+  bf16x8_t* T = tiles + d.t;
+  for (int64_t r0 = b0; r0 < end; r0 += 64) {
+    __syncthreads();
+    chunk_store(Xs, pre);
+    __syncthreads();
+    // rows of other chunks: the write below does not touch them
+    if (r0 + 64 < end) chunk_fetch(X, R, d.l, r0 + 64, pre);
+    chunk_times(Xs, W, nullptr, d.l);
+    chunk_write(Xs, r0, end, d.l, X, R);
+    if (!LAST) {
+      gram_chunk(Xs, acc);
+    } else {
+      // two 32-row k blocks x three column tiles, the layout of btile_kernel;
+      // rows past the end are zero in LDS
+      for (int u = tid >> 6; u < 2 * kNT; u += 4) {
+        const int kbl = u / kNT, nt = u % kNT;
+        const int64_t kb = r0 / 32 + kbl;
+        if (kb >= KB) continue;
+        const int col = nt * 16 + (lane & 15), row = 32 * kbl + 8 * (lane >> 4);
+        bf16x8_t h, lo;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float v = Xs[row + e][col];
+          const __bf16 hb = (__bf16)v;
+          h[e] = hb;
+          lo[e] = (__bf16)(v - (float)hb);
+        }
+        T[(kb * kNT + nt) * 64 + lane] = h;
+        T[((KB + kb) * kNT + nt) * 64 + lane] = lo;
+      }
+    }
   }
+  if (!LAST)
+    gram_partial_out(acc, &W[0][0], gpart + ((FROM_Z ? d.gz : d.gy) + it.tile) * kGramPart);
 }
 
 // ---------------------------------------------------------------- final
@@ -651,22 +710,21 @@ __device__ double lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* si
   return sc;
 }
 
-__global__ void __launch_bounds__(256, 3)
-bfinal_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
-              float* __restrict__ work, float* __restrict__ U,
-              double* __restrict__ S, float* __restrict__ V) {
-  __shared__ float Xs[64][kL + 1];
+// The small eigenproblem of a matrix from the Gram partials of B^T: S, the
+// selected eigenvectors (48 x 48, zero padding) and 1 / sigma.
+__global__ void __launch_bounds__(256)
+bjacobi_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
+               const double* __restrict__ gpart, double* __restrict__ evecs,
+               double* __restrict__ isig, double* __restrict__ S) {
   __shared__ double H[kL][kLP];
   __shared__ double J[kL][kLP];
-  __shared__ double sig[kL];
   __shared__ int order[kL];
   __shared__ int flag;
-  const BMat d = mats[mat_order[blockIdx.x]];  // largest first
+  const int mat = mat_order[blockIdx.x];  // largest first
+  const BMat d = mats[mat];
   const int l = d.l, k = d.k;
   const int np = l + (l & 1);
-  const float* Q = work + d.y;   // m x 48, orthonormal
-  const float* Bt = work + d.z;  // n x 48 = A^T Q
-  lds_gram(Bt, d.n, l, Xs, H);   // H = B B^T (l x l)
+  gram_partials_in<4>(gpart + d.gz * kGramPart, (int)((d.n + kSlab - 1) / kSlab), H);
   const int tid = threadIdx.x;
   if (np > l) {
     // odd l: one padding row / column, decoupled
@@ -691,21 +749,45 @@ bfinal_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
     const int e = order[l - k + tid];
     const double lam = H[e][e] / sc;
     const double s = lam < 0.0 ? 0.0 : sqrt(lam);  // NaN stays NaN
-    sig[tid] = s;
+    isig[(int64_t)mat * kL + tid] = 1.0 / s;
     S[d.s + tid] = s;
   }
-  __syncthreads();
-  // selected eigenvectors (columns order[l - k + j]) into H (its diagonal
-  // was read above), 1 / sigma
+  double* out = evecs + (int64_t)mat * kL * kL;
   for (int e = tid; e < kL * kL; e += 256) {
-    const int c = e % kL, j = e / kL;
-    H[c][j] = (c < l && j < k) ? J[c][order[l - k + j]] : 0.0;  // zero padding: finite
+    const int c = e / kL, j = e % kL;
+    out[e] = (c < l && j < k) ? J[c][order[l - k + j]] : 0.0;  // zero padding: finite
   }
-  if (tid < k) sig[tid] = 1.0 / sig[tid];
-  __syncthreads();
-  // U = Q Uhat_sel (m x k), V = B^T Uhat_sel Sigma^-1 (n x k)
-  lds_rows_times(Q, d.m, l, Xs, H, k, nullptr, U + d.u, d.m);
-  lds_rows_times(Bt, d.n, l, Xs, H, k, sig, V + d.v, d.n);
+}
+
+// A slab of U = Q Uhat (FROM_Z = false) or V = B^T Uhat Sigma^-1 (true).
+template <bool FROM_Z>
+__global__ void __launch_bounds__(256)
+bout_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
+            const float* __restrict__ work, const double* __restrict__ evecs,
+            const double* __restrict__ isig, float* __restrict__ out) {
+  __shared__ float Xs[64][kL + 1];
+  __shared__ double W[kL][kLP];
+  __shared__ double sig[kL];
+  const BItem it = items[blockIdx.x];
+  const BMat d = mats[it.mat];
+  const int64_t R = FROM_Z ? d.n : d.m;
+  const float* X = work + (FROM_Z ? d.z : d.y);
+  float* O = out + (FROM_Z ? d.v : d.u);
+  const int64_t b0 = (int64_t)it.tile * kSlab, end = b0 + kSlab < R ? b0 + kSlab : R;
+  const int tid = threadIdx.x;
+  float pre[kChunkLoads];
+  chunk_fetch(X, R, d.l, b0, pre);
+  const double* Wg = evecs + (int64_t)it.mat * kL * kL;
+  for (int e = tid; e < kL * kL; e += 256) W[e / kL][e % kL] = Wg[e];
+  if (FROM_Z && tid < d.k) sig[tid] = isig[(int64_t)it.mat * kL + tid];
+  for (int64_t r0 = b0; r0 < end; r0 += 64) {
+    __syncthreads();
+    chunk_store(Xs, pre);
+    __syncthreads();
+    if (r0 + 64 < end) chunk_fetch(X, R, d.l, r0 + 64, pre);
+    chunk_times(Xs, W, FROM_Z ? sig : nullptr, d.k);
+    chunk_write(Xs, r0, end, d.k, O, R);
+  }
 }
 
 __global__ void bclear_kernel(int* __restrict__ p) {
@@ -719,11 +801,13 @@ struct Plan {
   int q = 0;
   DBuf<BMat> mats;
   DBuf<BItem> it_nn, it_tn;         // pass items per RT variant chosen
-  DBuf<BItem> it_tile_n, it_tile_m;  // tiling items (K = n_i / K = m_i)
-  int n_nn = 0, n_tn = 0, n_tile_n = 0, n_tile_m = 0;
+  DBuf<BItem> it_tile_n;             // tiling items (K = n_i)
+  DBuf<BItem> it_slab_y, it_slab_z;  // 256-row slabs of Y_i / Z_i
+  int n_nn = 0, n_tn = 0, n_tile_n = 0, n_slab_y = 0, n_slab_z = 0;
   int rt_nn = 1, rt_tn = 1;
   DBuf<float> work;
   DBuf<bf16x8_t> tiles;
+  DBuf<double> gpart, rinv, isig;  // Gram partials, R^-1 (or Uhat) and 1 / sigma per matrix
   DBuf<int> flags;
   const float* A = nullptr;
   float* U = nullptr;
@@ -769,12 +853,13 @@ std::vector<BItem> pass_items(const Plan& P, bool ta, int rt_code) {
   return v;
 }
 
-std::vector<BItem> tile_items(const Plan& P, bool from_y) {
+// items of `rows` rows of the matrices' Y_i (from_y) or Z_i
+std::vector<BItem> row_items(const Plan& P, bool from_y, int rows) {
   std::vector<BItem> v;
   for (int i : P.by_cost) {
     const BMat& d = P.host[i];
     const int64_t K = from_y ? d.m : d.n;
-    for (int64_t kb = 0; kb < (K + 31) / 32; ++kb) v.push_back({i, (int32_t)kb});
+    for (int64_t t = 0; t < (K + rows - 1) / rows; ++t) v.push_back({i, (int32_t)t});
   }
   return v;
 }
@@ -811,26 +896,55 @@ int launch_pass(Context* c, Plan& P, bool ta, int rt, const BItem* items, int ni
   return 0;
 }
 
-int launch_tile(Context* c, Plan& P, bool from_y) {
-  const int n = from_y ? P.n_tile_m : P.n_tile_n;
-  if (n == 0) return 0;
-  if (from_y)
-    hipLaunchKernelGGL((btile_kernel<true>), dim3((unsigned)n), dim3(192), 0, c->stream, P.mats.p,
-                       P.it_tile_m.p, (const float*)P.work.p, P.tiles.p);
-  else
-    hipLaunchKernelGGL((btile_kernel<false>), dim3((unsigned)n), dim3(192), 0, c->stream,
-                       P.mats.p, P.it_tile_n.p, (const float*)P.work.p, P.tiles.p);
+int launch_tile(Context* c, Plan& P) {
+  hipLaunchKernelGGL(btile_kernel, dim3((unsigned)P.n_tile_n), dim3(192), 0, c->stream, P.mats.p,
+                     P.it_tile_n.p, (const float*)P.work.p, P.tiles.p);
   RSVD_LAUNCH_CHECK();
   return 0;
 }
 
+template <bool FROM_Z>
+int launch_orth_of(Context* c, Plan& P) {
+  const BItem* items = FROM_Z ? P.it_slab_z.p : P.it_slab_y.p;
+  const dim3 slabs((unsigned)(FROM_Z ? P.n_slab_z : P.n_slab_y)), mats((unsigned)P.count);
+  hipLaunchKernelGGL(bgram_kernel<FROM_Z>, slabs, dim3(256), 0, c->stream, P.mats.p, items,
+                     (const float*)P.work.p, P.gpart.p);
+  RSVD_LAUNCH_CHECK();
+  for (int pass = 0; pass < 2; ++pass) {
+    hipLaunchKernelGGL(bchol_kernel<FROM_Z>, mats, dim3(64), 0, c->stream, P.mats.p,
+                       (const int*)P.order.p, (const double*)P.gpart.p, P.rinv.p, pass == 0 ? 1 : 0,
+                       P.flags.p);
+    RSVD_LAUNCH_CHECK();
+    if (pass == 0)
+      hipLaunchKernelGGL((bapply_kernel<FROM_Z, false>), slabs, dim3(256), 0, c->stream, P.mats.p,
+                         items, P.work.p, (const double*)P.rinv.p, P.gpart.p, P.tiles.p);
+    else
+      hipLaunchKernelGGL((bapply_kernel<FROM_Z, true>), slabs, dim3(256), 0, c->stream, P.mats.p,
+                         items, P.work.p, (const double*)P.rinv.p, P.gpart.p, P.tiles.p);
+    RSVD_LAUNCH_CHECK();
+  }
+  return 0;
+}
+
+// CholeskyQR2 of Y_i (or Z_i), the result tiled for the next pass over A as well
 int launch_orth(Context* c, Plan& P, bool from_z) {
-  if (from_z)
-    hipLaunchKernelGGL((borth_kernel<true>), dim3((unsigned)P.count), dim3(256), 0, c->stream,
-                       P.mats.p, (const int*)P.order.p, P.work.p, P.flags.p);
-  else
-    hipLaunchKernelGGL((borth_kernel<false>), dim3((unsigned)P.count), dim3(256), 0, c->stream,
-                       P.mats.p, (const int*)P.order.p, P.work.p, P.flags.p);
+  return from_z ? launch_orth_of<true>(c, P) : launch_orth_of<false>(c, P);
+}
+
+int launch_final(Context* c, Plan& P) {
+  hipLaunchKernelGGL(bgram_kernel<true>, dim3((unsigned)P.n_slab_z), dim3(256), 0, c->stream,
+                     P.mats.p, P.it_slab_z.p, (const float*)P.work.p, P.gpart.p);
+  RSVD_LAUNCH_CHECK();
+  hipLaunchKernelGGL(bjacobi_kernel, dim3((unsigned)P.count), dim3(256), 0, c->stream, P.mats.p,
+                     (const int*)P.order.p, (const double*)P.gpart.p, P.rinv.p, P.isig.p, P.S);
+  RSVD_LAUNCH_CHECK();
+  hipLaunchKernelGGL(bout_kernel<false>, dim3((unsigned)P.n_slab_y), dim3(256), 0, c->stream,
+                     P.mats.p, P.it_slab_y.p, (const float*)P.work.p, (const double*)P.rinv.p,
+                     (const double*)P.isig.p, P.U);
+  RSVD_LAUNCH_CHECK();
+  hipLaunchKernelGGL(bout_kernel<true>, dim3((unsigned)P.n_slab_z), dim3(256), 0, c->stream,
+                     P.mats.p, P.it_slab_z.p, (const float*)P.work.p, (const double*)P.rinv.p,
+                     (const double*)P.isig.p, P.V);
   RSVD_LAUNCH_CHECK();
   return 0;
 }
@@ -842,23 +956,17 @@ int enqueue_all(Context* c, Plan& P) {
   hipLaunchKernelGGL(bomega_kernel, dim3((unsigned)P.count, kL), dim3(256), 0, c->stream,
                      P.mats.p, P.work.p);
   RSVD_LAUNCH_CHECK();
-  RSVD_TRY(launch_tile(c, P, false));
+  RSVD_TRY(launch_tile(c, P));
   RSVD_TRY(launch_pass(c, P, false, P.rt_nn, P.it_nn.p, P.n_nn));  // Y = A Omega
   RSVD_TRY(launch_orth(c, P, false));
   for (int it = 1; it < P.q; ++it) {
-    RSVD_TRY(launch_tile(c, P, true));
     RSVD_TRY(launch_pass(c, P, true, P.rt_tn, P.it_tn.p, P.n_tn));  // Z = A^T Q
     RSVD_TRY(launch_orth(c, P, true));
-    RSVD_TRY(launch_tile(c, P, false));
     RSVD_TRY(launch_pass(c, P, false, P.rt_nn, P.it_nn.p, P.n_nn));  // Y = A Z
     RSVD_TRY(launch_orth(c, P, false));
   }
-  RSVD_TRY(launch_tile(c, P, true));
   RSVD_TRY(launch_pass(c, P, true, P.rt_tn, P.it_tn.p, P.n_tn));  // B^T = A^T Q
-  hipLaunchKernelGGL(bfinal_kernel, dim3((unsigned)P.count), dim3(256), 0, c->stream, P.mats.p,
-                     (const int*)P.order.p, P.work.p, P.U, P.S, P.V);
-  RSVD_LAUNCH_CHECK();
-  return 0;
+  return launch_final(c, P);
 }
 
 // Autotuner: time each RT variant of both pass kernels on this batch (after
@@ -917,13 +1025,8 @@ int autotune(Context* c, Plan& P) {
     (void)hipEventRecord(e0, c->stream);
     if (st == 0) rc = launch_orth(c, P, false);
     else if (st == 1) rc = launch_orth(c, P, true);
-    else if (st == 2) {
-      hipLaunchKernelGGL(bfinal_kernel, dim3((unsigned)P.count), dim3(256), 0, c->stream, P.mats.p,
-                         (const int*)P.order.p, P.work.p, P.U, P.S, P.V);
-      rc = hipGetLastError() == hipSuccess ? 0 : set_error("batched: final launch failed");
-    } else {
-      rc = launch_tile(c, P, false);
-    }
+    else if (st == 2) rc = launch_final(c, P);
+    else rc = launch_tile(c, P);
     (void)hipEventRecord(e1, c->stream);
     if (rc) break;
     (void)hipEventSynchronize(e1);
@@ -972,7 +1075,7 @@ int fixed_rank_batched(Context* c, int count, const int* m, const int* n, const 
     P->S = dS;
     P->V = dV;
     P->host.resize(count);
-    int64_t wofs = 0, tofs = 0;
+    int64_t wofs = 0, tofs = 0, gy = 0, gz = 0;
     for (int i = 0; i < count; ++i) {
       BMat& d = P->host[i];
       d.m = m[i];
@@ -990,6 +1093,10 @@ int fixed_rank_batched(Context* c, int count, const int* m, const int* n, const 
       d.u = u_off[i];
       d.s = s_off[i];
       d.v = v_off[i];
+      d.gy = gy;
+      gy += (d.m + kSlab - 1) / kSlab;
+      d.gz = gz;
+      gz += (d.n + kSlab - 1) / kSlab;
       d.seed = seed + (uint64_t)i;
       d.aligned = (d.m % 4 == 0) && (d.a % 4 == 0) && (reinterpret_cast<uintptr_t>(dA) % 16 == 0);
       d.pad = 0;
@@ -1008,8 +1115,12 @@ int fixed_rank_batched(Context* c, int count, const int* m, const int* n, const 
     RSVD_TRY(P->work.alloc((size_t)wofs));
     RSVD_TRY(P->tiles.alloc((size_t)tofs));
     RSVD_TRY(P->flags.alloc(1));
-    RSVD_TRY(upload_items(c, tile_items(*P, false), P->it_tile_n, &P->n_tile_n));
-    RSVD_TRY(upload_items(c, tile_items(*P, true), P->it_tile_m, &P->n_tile_m));
+    RSVD_TRY(P->gpart.alloc((size_t)((gy > gz ? gy : gz) * kGramPart)));
+    RSVD_TRY(P->rinv.alloc((size_t)count * kL * kL));
+    RSVD_TRY(P->isig.alloc((size_t)count * kL));
+    RSVD_TRY(upload_items(c, row_items(*P, false, 32), P->it_tile_n, &P->n_tile_n));
+    RSVD_TRY(upload_items(c, row_items(*P, true, kSlab), P->it_slab_y, &P->n_slab_y));
+    RSVD_TRY(upload_items(c, row_items(*P, false, kSlab), P->it_slab_z, &P->n_slab_z));
     // one eager run so the tuner times the passes on real operands
     P->rt_nn = P->rt_tn = 1;
     RSVD_TRY(upload_items(c, pass_items(*P, false, 1), P->it_nn, &P->n_nn));

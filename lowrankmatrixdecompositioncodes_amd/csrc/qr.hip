@@ -10,6 +10,7 @@
 // LAPACK sign convention, hhqr.hip) runs instead.
 #include <cmath>
 
+#include "chol16.h"
 #include "rsvd_internal.h"
 
 namespace rsvd {
@@ -93,52 +94,6 @@ __device__ __forceinline__ void ci_put(const double (&v)[4], double (*T)[CHP]) {
   }
 }
 
-// v of lane J of the 16-lane row the lane is in (a data-parallel move).
-template <int J>
-__device__ __forceinline__ double ci_bcast(double v) {
-  union {
-    double d;
-    int i[2];
-  } u = {v};
-  u.i[0] = __builtin_amdgcn_mov_dpp(u.i[0], 0x150 + J, 0xf, 0xf, true);  // row_newbcast:J
-  u.i[1] = __builtin_amdgcn_mov_dpp(u.i[1], 0x150 + J, 0xf, 0xf, true);
-  return u.d;
-}
-
-// Cholesky and inverse of a 16 x 16 block in the registers of a 16-lane row:
-// lane c holds column c of the symmetric block (a[r], all rows) and column c of
-// the identity (e[r]); step j scales row j by 1 / sqrt(pivot) and subtracts it
-// from the rows below, u_jr broadcast from lane r.  On exit a[r] (r <= c) is
-// R(r, c), e[r] is R^-1(c, r) (zero for r < c) and piv lane c's pivot.  The steps
-// from kb on (padding) are left out.  A pivot that is not positive gives NaN
-// from there on; the caller's test of piv reports it.
-template <int J>
-__device__ __forceinline__ void ci_chol16_step(double (&a)[16], double (&e)[16], int c, int kb,
-                                               double* piv) {
-  if (J >= kb) return;
-  const double d = ci_bcast<J>(a[J]);
-  *piv = (c == J) ? d : *piv;
-  // 1 / sqrt(d): the hardware estimate and one third-order step
-  const double y0 = __builtin_amdgcn_rsq(d);
-  const double r = fma(-d * y0, y0, 1.0);
-  const double y = fma(y0 * r, fma(0.375, r, 0.5), y0);
-  a[J] *= y;
-  e[J] *= y;
-  const double u = a[J], w = e[J];
-  // (one compile-time broadcast a row below)
-#define RSVD_CI_ROW(R)                     \
-  if constexpr (R > J && R < 16) {         \
-    const double m = ci_bcast<R>(u);       \
-    a[R] = fma(-m, u, a[R]);               \
-    e[R] = fma(-m, w, e[R]);               \
-  }
-  RSVD_CI_ROW(1) RSVD_CI_ROW(2) RSVD_CI_ROW(3) RSVD_CI_ROW(4) RSVD_CI_ROW(5)
-  RSVD_CI_ROW(6) RSVD_CI_ROW(7) RSVD_CI_ROW(8) RSVD_CI_ROW(9) RSVD_CI_ROW(10)
-  RSVD_CI_ROW(11) RSVD_CI_ROW(12) RSVD_CI_ROW(13) RSVD_CI_ROW(14) RSVD_CI_ROW(15)
-#undef RSVD_CI_ROW
-  if constexpr (J < 15) ci_chol16_step<J + 1>(a, e, c, kb, piv);
-}
-
 typedef double ci_d4 __attribute__((ext_vector_type(4)));
 
 // One wave: acc + op(P) Q for 16 x 16 blocks of LDS tiles (row-major, CHP):
@@ -168,7 +123,7 @@ __device__ __forceinline__ void ci_wave_fence() {
 
 // Cholesky Dm = R^T R (upper triangle read, kb x kb valid, zero beyond) and Xk =
 // R^-1 of a 32 x 32 tile, by 16 x 16 blocks on wave 0 alone: the two diagonal
-// blocks in registers (ci_chol16_step), the products between them on the FP64
+// blocks in registers (chol16_step), the products between them on the FP64
 // matrix cores.  On exit Dm holds R, both zero below the diagonal and past kb;
 // Tw is scratch; *bad is set on a bad pivot (see above).  Ends with a barrier.
 // The chain of 32 pivots is what a launch waits for: four pivots a barrier with
@@ -190,7 +145,7 @@ __device__ void ci_factor_inv(double (*Dm)[CHP], int kb, const double* ref, doub
         e[r] = (r == c) ? 1.0 : 0.0;
       }
       double piv = 1.0;
-      ci_chol16_step<0>(a, e, c, kh, &piv);
+      chol16_step<0, false>(a, e, c, kh, &piv);
       // a pivot must be finite and above kCholRelTol times its diagonal entry
       b |= c < kh && !(piv > kCholRelTol * ref[o + c] && piv < INFINITY);
       ci_wave_fence();
