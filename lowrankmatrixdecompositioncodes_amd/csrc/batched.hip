@@ -19,16 +19,16 @@
 //   bapply   per slab: X <- X R^-1; the first pass of CholeskyQR2 forms the next
 //            pass's Gram partial from the rows it has just written, the second
 //            writes the rows tiled for the pass over A as well
-//   bjacobi  per matrix: G = B B^T (FP64, from B^T = A^T Q), two-sided Jacobi in
-//            LDS, ascending eigenvalues, sigma = sqrt(lambda), last k kept
-//            (rra.c:175-225)
+//   bjacobi  per matrix: G = B B^T (FP64, from B^T = A^T Q), two-sided Jacobi (G in
+//            LDS, eigenvectors in registers), ascending eigenvalues, sigma =
+//            sqrt(lambda), last k kept (rra.c:175-225)
 //   bout     per slab: U = Q Uhat and V = B^T Uhat Sigma^-1
 // The row work is cut into slabs so that a large matrix is spread over as many
 // workgroups as it has slabs: with one workgroup a matrix for the whole of
 // CholeskyQR2 (and for the whole final stage), the largest of the batch set the
 // time of 200 matrices and the chunks' latencies that of 4096 (orth Y / orth Z /
-// final: 0.38 / 0.25 / 0.47 ms and 1.64 / 1.06 / 2.55 ms; now 0.12 / 0.09 / 0.42 and
-// 1.13 / 0.45 / 2.35, the tiling of Q for the next pass included).
+// final: 0.38 / 0.25 / 0.47 ms and 1.64 / 1.06 / 2.55 ms; now 0.12 / 0.08 / 0.23 and
+// 1.07 / 0.43 / 1.49, the tiling of Q for the next pass included).
 // Sketch widths are padded to 48 columns (three 16-wide tiles; l_i = k_i + p
 // <= 48), padding columns are zero throughout.  The pass kernels have
 // variants (rows per wave RT = 1, 2, 4) chosen per batch layout by timing
@@ -474,11 +474,11 @@ __device__ __forceinline__ void gram_partial_out(const d4_t (&acc)[6], double* l
   for (int e = threadIdx.x; e < kGramPart; e += 256) part[e] = lds[e];
 }
 
-// G (both triangles, LDS) = the sum of a matrix's partials, in slab order, by a
+// G (both triangles, LDS, row pitch ldg) = the sum of a matrix's partials, in slab order, by a
 // workgroup of WAVES waves (1 or 4).
 template <int WAVES>
 __device__ __forceinline__ void gram_partials_in(const double* __restrict__ part, int slabs,
-                                                 double (*G)[kLP]) {
+                                                 double* G, int ldg) {
   constexpr int Q = kGramPart / (64 * WAVES);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
   double v[Q];
@@ -494,8 +494,8 @@ __device__ __forceinline__ void gram_partials_in(const double* __restrict__ part
     // upper tile t of (0,0) (0,1) (0,2) (1,1) (1,2) (2,2)
     const int ti = t < 3 ? 0 : (t < 5 ? 1 : 2), tj = t < 3 ? t : (t < 5 ? t - 2 : 2);
     const int i = 16 * ti + 4 * r + lk, j = 16 * tj + li;
-    G[i][j] = v[q];
-    if (ti != tj) G[j][i] = v[q];
+    G[i * ldg + j] = v[q];
+    if (ti != tj) G[j * ldg + i] = v[q];
   }
   __syncthreads();
 }
@@ -540,7 +540,7 @@ bchol_kernel(const BMat* __restrict__ mats, const int* __restrict__ order,
   const int64_t R = FROM_Z ? d.n : d.m;
   const int lane = threadIdx.x;
   gram_partials_in<1>(gpart + (FROM_Z ? d.gz : d.gy) * kGramPart, (int)((R + kSlab - 1) / kSlab),
-                      G);
+                      &G[0][0], kLP);
   if (shift) {
     double tr = 0.0;
     for (int j = 0; j < d.l; ++j) tr += G[j][j];
@@ -560,7 +560,7 @@ bchol_kernel(const BMat* __restrict__ mats, const int* __restrict__ order,
 // One slab of X <- X R^-1.  LAST = false: the Gram partial of the new rows;
 // true: the new rows rounded to the pass's split-bf16 tiles as well.
 template <bool FROM_Z, bool LAST>
-__global__ void __launch_bounds__(256, 4)
+__global__ void __launch_bounds__(256, LAST ? 4 : 3)
 bapply_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
               float* __restrict__ work, const double* __restrict__ rinv,
               double* __restrict__ gpart, bf16x8_t* __restrict__ tiles) {
@@ -618,145 +618,177 @@ bapply_kernel(const BMat* __restrict__ mats, const BItem* __restrict__ items,
 }
 
 // ---------------------------------------------------------------- final
-__device__ __forceinline__ int circle(int pos, int r, int N) {
-  return pos == 0 ? 0 : 1 + ((pos - 1 + r) % (N - 1));
+// Two-sided Jacobi on H (n x n, positive semidefinite, upper triangle in LDS) in
+// the odd-even order: step t rotates the neighbours (2 i - t % 2, 2 i + 1 - t % 2) and
+// exchanges them, so that n steps meet every pair once and every step's positions
+// are known at compile time.  Of the four waves one keeps the rows of V in
+// registers and three take the 2 x 2 blocks of H; the first of the three computes
+// a step's rotations.  With the round-robin order both matrices were in LDS, H in
+// full, and indices and angles were read for every block: 450 LDS operations of a
+// wave a step and 0.37 ms for 200 matrices (1.89 for 4096), here 60 and 0.18 (1.03).
+//
+// A pair's transformation is [[u, v], [v, -u]] with u = sin, v = cos of rotation():
+// the rotation and the exchange.  Position p has index p + 1 in H: positions -1, n
+// and n + 1 are zero rows that pair with an end left over by the step, which then
+// keeps its place (u, v = 1, 0).
+constexpr int kJR = kL + 3, kJP = kL + 4;  // rows of H and their pitch
+constexpr int kJPairs = kL / 2 + 1;
+typedef double d2_t __attribute__((ext_vector_type(2)));
+
+// Pairs K0 .. K1 - 1 of a step of parity PAR applied to a row of V.
+template <int PAR, int K0, int K1>
+__device__ __forceinline__ void rotate_row(double (&v)[kL], const d2_t* uv, int pairs) {
+#pragma unroll
+  for (int k0 = K0; k0 < K1; k0 += 4) {
+    if (k0 >= pairs) continue;
+#pragma unroll
+    for (int k = k0; k < (k0 + 4 < K1 ? k0 + 4 : K1); ++k) {
+      const int p = 2 * k - PAR, q = p + 1;
+      const bool pin = p >= 0 && p < kL, qin = q < kL;
+      const d2_t r = uv[k];
+      const double x = pin ? v[p] : 0.0, y = qin ? v[q] : 0.0;
+      if (pin) v[p] = fma(r.x, x, r.y * y);
+      if (qin) v[q] = fma(r.y, x, -r.x * y);
+    }
+  }
 }
 
-// two-sided cyclic Jacobi on H (np x np, np even, positive semidefinite) with
-// J accumulated.  A step: threads 0..np/2-1 compute the rotation of their pair
-// once (round-robin pairing) and publish it with the pair's two indices;
-// after a barrier the 2 x 2 blocks of H (pairs bi x bj: thread t takes bi in
-// {t / 16, t / 16 + 16}, bj in {t % 16, t % 16 + 16}) and the (row, pair)
-// entries of J (row t % 64, pairs t / 64 + 4 i) are updated in parallel, in
-// place (the pairs partition the indices, so the blocks are disjoint, and the
-// step's rotations were read before the barrier) -- fixed strides, no
-// division by the runtime size.
-// Sweeps until a sweep's rotations pass the loose stop of rotation() (the
-// outputs are fp32: eigenvalues good to ~1e-8 relative, eigenvectors of
-// separated eigenvalues to ~1e-8).  Returns the power of two H was scaled by.
-__device__ double lds_jacobi(double (*H)[kLP], double (*J)[kLP], int np, int* sig_flag) {
-  __shared__ double rc[kL / 2], rs[kL / 2];
-  __shared__ int pp[kL / 2], qq[kL / 2];
-  const int tid = threadIdx.x;
-  const int half = np / 2;
-  double (*Hc)[kLP] = H;
-  for (int e = tid; e < np * np; e += 256) J[e / np][e % np] = (e / np == e % np) ? 1.0 : 0.0;
+// The small eigenproblem of a matrix from the Gram partials of B^T: S, the
+// selected eigenvectors (48 x 48, zero padding) and 1 / sigma.  Sweeps until one's
+// rotations pass the loose stop of rotation() (the outputs are fp32: eigenvalues
+// good to ~1e-8 relative, eigenvectors of separated eigenvalues to ~1e-8).
+__global__ void __launch_bounds__(256, 3)
+bjacobi_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
+               const double* __restrict__ gpart, double* __restrict__ evecs,
+               double* __restrict__ isig, double* __restrict__ S) {
+  __shared__ __align__(16) double H[kJR * kJP];
+  __shared__ __align__(16) d2_t uv[2][kJPairs];
+  __shared__ int rank[kL];
+  __shared__ int more;
+  static_assert(kJR * kJP >= kL * kLP, "the eigenvectors are staged in H's place");
+  const int mat = mat_order[blockIdx.x];  // largest first
+  const BMat d = mats[mat];
+  const int n = d.l, k = d.k, pairs = n / 2 + 1;
+  const int tid = threadIdx.x, lane = tid & 63;
+  for (int e = tid; e < kJR * kJP; e += 256) H[e] = 0.0;
+  if (tid < 2 * kJPairs) uv[tid / kJPairs][tid % kJPairs] = d2_t{1.0, 0.0};
   __syncthreads();
-  // H is positive semidefinite (a Gram matrix): ||H||_F <= trace(H); scaled to
-  // a trace of order one (rotation() relies on it)
+  gram_partials_in<4>(gpart + d.gz * kGramPart, (int)((d.n + kSlab - 1) / kSlab), H + kJP + 1, kJP);
+  // H is a Gram matrix: ||H||_F <= trace(H); scaled to a trace of order one
+  // (rotation() relies on it)
   double tr = 0.0;
-  for (int i = 0; i < np; ++i) tr += fabs(Hc[i][i]);
+  for (int i = 1; i <= n; ++i) tr += fabs(H[i * (kJP + 1)]);
   const double sc = unit_scale(tr);
   const float flo = (float)(4.0 * 2.220446049250313e-16 * tr * sc);
   const RotStop stop = rot_stop(true);
   __syncthreads();
-  for (int e = tid; e < np * np; e += 256) Hc[e / np][e % np] *= sc;
-  __syncthreads();
-  for (int sweep = 0; sweep < 40; ++sweep) {
-    if (tid == 0) *sig_flag = 0;
-    __syncthreads();
-    bool sig = false;
-    for (int t = 0; t < np - 1; ++t) {
-      if (tid < half) {
-        const int p = circle(tid, t, np), q = circle(np - 1 - tid, t, np);
-        double c, sn;
-        bool sg;
-        rotation(Hc[p][p], Hc[q][q], Hc[p][q], flo, stop, &c, &sn, &sg);
-        rc[tid] = c;
-        rs[tid] = sn;
-        pp[tid] = p;
-        qq[tid] = q;
-        sig |= sg;
-      }
-      __syncthreads();
-      static_assert(kL / 2 <= 32, "pair indices below 32: two strides of 16");
+  for (int e = tid; e < kJR * kJP; e += 256) H[e] *= sc;
+  // the row wave is another one from workgroup to workgroup: a SIMD gets its
+  // share of both kinds
+  const int role = ((tid >> 6) + (int)blockIdx.x) & 3;  // 3: rows of V
+  // this thread's blocks (bi <= bj) of the upper triangle of pairs, row by row
+  constexpr int kBlocks = (kJPairs * (kJPairs + 1) / 2 + 191) / 192;
+  int bi[kBlocks], bj[kBlocks];
+  const int nblk = role == 3 ? 0 : pairs * (pairs + 1) / 2;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int bi = (tid >> 4) + 16 * (e >> 1), bj = (tid & 15) + 16 * (e & 1);
-        if (bi >= half || bj >= half) continue;
-        const int pi = pp[bi], qi = qq[bi], pj = pp[bj], qj = qq[bj];
-        const double ci = rc[bi], si = rs[bi], cj = rc[bj], sj = rs[bj];
-        const double h00 = Hc[pi][pj], h01 = Hc[pi][qj], h10 = Hc[qi][pj], h11 = Hc[qi][qj];
-        const double x00 = cj * h00 - sj * h01, x01 = sj * h00 + cj * h01;
-        const double x10 = cj * h10 - sj * h11, x11 = sj * h10 + cj * h11;
-        const double y00 = ci * x00 - si * x10, y01 = ci * x01 - si * x11;
-        double y10 = si * x00 + ci * x10;
-        const double y11 = si * x01 + ci * x11;
-        if (bi == bj) y10 = y01;  // the diagonal blocks stay exactly symmetric
-        Hc[pi][pj] = y00;
-        Hc[pi][qj] = y01;
-        Hc[qi][pj] = y10;
-        Hc[qi][qj] = y11;
+  for (int b = 0; b < kBlocks; ++b) {
+    int i = 0, j = role * 64 + lane + 192 * b;
+    if (j < nblk)
+      while (j >= pairs - i) {
+        j -= pairs - i;
+        ++i;
       }
-      static_assert(kL <= 64, "a J row per lane of a wave");
-      for (int k = tid >> 6; k < half; k += 4) {
-        const int x = tid & 63;
-        if (x >= np) continue;
-        const int pk = pp[k], qk = qq[k];
-        const double ck = rc[k], sk = rs[k];
-        const double jp = J[x][pk], jq = J[x][qk];
-        J[x][pk] = ck * jp - sk * jq;
-        J[x][qk] = sk * jp + ck * jq;
+    bi[b] = i;
+    bj[b] = j + i;
+  }
+  double v[kL];
+#pragma unroll
+  for (int p = 0; p < kL; ++p) v[p] = (p == lane) ? 1.0 : 0.0;
+  __syncthreads();
+  int par = 0, buf = 0;
+  bool pending = false;  // the second half of the last step is not in v yet
+  auto second_half = [&]() {
+    if (par) rotate_row<0, kL / 4, kJPairs>(v, uv[buf ^ 1], pairs);  // of the other parity
+    else rotate_row<1, kL / 4, kJPairs>(v, uv[buf ^ 1], pairs);
+  };
+  for (int sweep = 0; sweep < 40 && n > 1; ++sweep) {
+    bool sig = false;
+    for (int t = 0; t < n; ++t) {
+      if (role == 0) {
+        if (lane < pairs) {
+          const int p = 2 * lane - par, ip = p + 1;
+          double c, s;
+          bool sg;
+          rotation(H[ip * (kJP + 1)], H[(ip + 1) * (kJP + 1)], H[ip * (kJP + 1) + 1], flo, stop, &c,
+                   &s, &sg);
+          const bool pair = p >= 0 && p + 1 < n;
+          uv[buf][lane] = pair ? d2_t{s, c} : d2_t{1.0, 0.0};
+          sig |= pair & sg;
+        }
+        if (t == n - 1) {
+          const bool any = __builtin_amdgcn_ballot_w64(sig) != 0;
+          if (lane == 0) more = any;
+        }
+      } else if (role == 3 && pending) {
+        second_half();
       }
       __syncthreads();
+      if (role == 3) {
+        if (par) rotate_row<1, 0, kL / 4>(v, uv[buf], pairs);
+        else rotate_row<0, 0, kL / 4>(v, uv[buf], pairs);
+      } else {
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) {
+          if (role * 64 + lane + 192 * b >= nblk) continue;
+          double* h = H + (2 * bi[b] + 1 - par) * kJP + 2 * bj[b] + 1 - par;
+          const d2_t ri = uv[buf][bi[b]], rj = uv[buf][bj[b]];
+          const double h00 = h[0], h01 = h[1], h11 = h[kJP + 1];
+          const double h10 = bi[b] == bj[b] ? h01 : h[kJP];  // below the diagonal: not kept
+          const double x00 = fma(rj.x, h00, rj.y * h01), x01 = fma(rj.y, h00, -rj.x * h01);
+          const double x10 = fma(rj.x, h10, rj.y * h11), x11 = fma(rj.y, h10, -rj.x * h11);
+          h[0] = fma(ri.x, x00, ri.y * x10);
+          h[1] = fma(ri.x, x01, ri.y * x11);
+          h[kJP] = fma(ri.y, x00, -ri.x * x10);
+          h[kJP + 1] = fma(ri.y, x01, -ri.x * x11);
+        }
+      }
+      __syncthreads();
+      buf ^= 1;
+      par ^= 1;
+      pending = true;
     }
-    if (sig) *sig_flag = 1;
-    __syncthreads();
-    const int any = *sig_flag;
-    __syncthreads();
-    if (!any) break;
+    if (!more) break;
   }
-  __syncthreads();
-  return sc;
-}
-
-// The small eigenproblem of a matrix from the Gram partials of B^T: S, the
-// selected eigenvectors (48 x 48, zero padding) and 1 / sigma.
-__global__ void __launch_bounds__(256)
-bjacobi_kernel(const BMat* __restrict__ mats, const int* __restrict__ mat_order,
-               const double* __restrict__ gpart, double* __restrict__ evecs,
-               double* __restrict__ isig, double* __restrict__ S) {
-  __shared__ double H[kL][kLP];
-  __shared__ double J[kL][kLP];
-  __shared__ int order[kL];
-  __shared__ int flag;
-  const int mat = mat_order[blockIdx.x];  // largest first
-  const BMat d = mats[mat];
-  const int l = d.l, k = d.k;
-  const int np = l + (l & 1);
-  gram_partials_in<4>(gpart + d.gz * kGramPart, (int)((d.n + kSlab - 1) / kSlab), H);
-  const int tid = threadIdx.x;
-  if (np > l) {
-    // odd l: one padding row / column, decoupled
-    for (int e = tid; e < np; e += 256) H[l][e] = H[e][l] = 0.0;
-  }
-  __syncthreads();
-  const double sc = lds_jacobi(H, J, np, &flag);  // H: sc times the eigenvalues
-  // ascending order of the l real eigenvalues: rank by counting
-  if (tid < l) {
+  if (role == 3 && pending) second_half();
+  // ascending order of the eigenvalues: rank by counting; the last k are kept,
+  // output j <- the eigenpair of rank n - k + j
+  if (tid < n) {
     // NaN ranks as +Inf, ties by index: the ranks are a permutation
-    const double lam = isnan(H[tid][tid]) ? INFINITY : H[tid][tid];
+    const double own = H[(tid + 1) * (kJP + 1)], lam = isnan(own) ? INFINITY : own;
     int rk = 0;
-    for (int j = 0; j < l; ++j) {
-      const double o = isnan(H[j][j]) ? INFINITY : H[j][j];
+    for (int j = 0; j < n; ++j) {
+      const double x = H[(j + 1) * (kJP + 1)], o = isnan(x) ? INFINITY : x;
       rk += (o < lam) || (o == lam && j < tid);
     }
-    order[rk] = tid;
+    const int j = rk - (n - k);
+    rank[tid] = j;
+    if (j >= 0) {
+      const double l = own / sc, s = l < 0.0 ? 0.0 : sqrt(l);  // NaN stays NaN
+      isig[(int64_t)mat * kL + j] = 1.0 / s;
+      S[d.s + j] = s;
+    }
   }
   __syncthreads();
-  // the last k in ascending order: output j <- eigenpair order[l - k + j]
-  if (tid < k) {
-    const int e = order[l - k + tid];
-    const double lam = H[e][e] / sc;
-    const double s = lam < 0.0 ? 0.0 : sqrt(lam);  // NaN stays NaN
-    isig[(int64_t)mat * kL + tid] = 1.0 / s;
-    S[d.s + tid] = s;
+  for (int e = tid; e < kL * kLP; e += 256) H[e] = 0.0;  // zero padding: finite
+  __syncthreads();
+  if (role == 3 && lane < n) {
+#pragma unroll
+    for (int p = 0; p < kL; ++p)
+      if (p < n && rank[p] >= 0) H[lane * kLP + rank[p]] = v[p];
   }
+  __syncthreads();
   double* out = evecs + (int64_t)mat * kL * kL;
-  for (int e = tid; e < kL * kL; e += 256) {
-    const int c = e / kL, j = e % kL;
-    out[e] = (c < l && j < k) ? J[c][order[l - k + j]] : 0.0;  // zero padding: finite
-  }
+  for (int e = tid; e < kL * kL; e += 256) out[e] = H[e / kL * kLP + e % kL];
 }
 
 // A slab of U = Q Uhat (FROM_Z = false) or V = B^T Uhat Sigma^-1 (true).
