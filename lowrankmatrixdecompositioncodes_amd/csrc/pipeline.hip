@@ -142,13 +142,15 @@ int fixed_rank_f64(Context* c, const double* A, int64_t m, int64_t n, int64_t ld
   RSVD_TRY(gemm_f64_tag(c, "apass_f64", 'N', 'N', m, l, n, 1.0, A, lda, Om, ldo, 0.0, Y.p, m));  // rra.c:95
   int fb = 0, f1 = 0;
   for (int j = 1; j < q; ++j) {                                        // rra.c:101-126
-    if ((2 * j - 2) % s == 0) { RSVD_TRY(orth_f64(c, m, l, Y.p, m, nullptr, &f1)); fb += f1; }
+    if ((2 * j - 2) % s == 0) { RSVD_TRY(orth_range_f64(c, m, l, Y, &f1)); fb += f1; }
     RSVD_TRY(gemm_f64_tag(c, "apass_f64", 'T', 'N', n, l, m, 1.0, A, lda, Y.p, m, 0.0, Z.p, n));
-    if ((2 * j - 1) % s == 0) { RSVD_TRY(orth_f64(c, n, l, Z.p, n, nullptr, &f1)); fb += f1; }
+    if ((2 * j - 1) % s == 0) { RSVD_TRY(orth_range_f64(c, n, l, Z, &f1)); fb += f1; }
     RSVD_TRY(gemm_f64_tag(c, "apass_f64", 'N', 'N', m, l, n, 1.0, A, lda, Z.p, n, 0.0, Y.p, m));
   }
-  RSVD_TRY(orth_f64(c, m, l, Y.p, m, nullptr, &f1));                   // rra.c:129-130
-  fb += f1;
+  for (int pass = 0; pass < 2; ++pass) {                               // rra.c:129-130
+    RSVD_TRY(orth_range_f64(c, m, l, Y, &f1));
+    fb += f1;
+  }
   if (info) { info->qr_fallbacks = fb; info->l = l; }
   return svd_from_Q_f64(c, A, m, n, lda, Y.p, m, l, k, vnum, U, ldu, S, V, ldv, info);
 }

@@ -9,6 +9,7 @@
 // reported back to the host and the blocked Householder QR (geqrf + orgqr,
 // LAPACK sign convention, hhqr.hip) runs instead.
 #include <cmath>
+#include <utility>
 
 #include "chol16.h"
 #include "rsvd_internal.h"
@@ -456,6 +457,35 @@ int orth_f64(Context* c, int64_t m, int64_t n, double* Y, int64_t ldy, double* R
     return 0;
   }
   if (R) RSVD_TRY(gemm_f64(c, 'N', 'N', n, n, n, 1.0, G2.p, n, G1.p, n, 0.0, R, n));
+  return 0;
+}
+
+int orth_range_f64(Context* c, int64_t m, int64_t n, DBuf<double>& Y, int* used_fallback) {
+  if (used_fallback) *used_fallback = 0;
+  if (n == 0 || m == 0) return 0;
+  if (m < n) return set_error("orth: m=%lld < n=%lld (thin QR needs m >= n)", (long long)m,
+                              (long long)n);
+  DBuf<double> W, G, R, Rinv, diag0, acc;
+  RSVD_TRY(W.alloc(Y.n));
+  RSVD_TRY(G.alloc((size_t)(n * n)));
+  RSVD_TRY(R.alloc((size_t)(n * n)));
+  RSVD_TRY(Rinv.alloc((size_t)(n * n)));
+  RSVD_TRY(acc.alloc((size_t)(n * n)));
+  RSVD_TRY(diag0.alloc((size_t)n));
+  RSVD_TRY(gemm_f64(c, 'T', 'N', n, n, m, 1.0, Y.p, m, Y.p, m, 0.0, G.p, n));
+  RSVD_TRY(chol_inv_launch(c, n, G.p, R.p, Rinv.p, c->flag_dev, diag0.p, acc.p));
+  // the pivot test's verdict goes to the host ahead of the product, which runs
+  // while the host waits for it: Y stays as it is until it is known
+  RSVD_TRY(flag_queue(c));
+  RSVD_TRY(gemm_f64(c, 'N', 'N', m, n, n, 1.0, Y.p, m, Rinv.p, n, 0.0, W.p, m));
+  int h = 0;
+  RSVD_TRY(flag_wait(c, &h));
+  if (h) {
+    if (used_fallback) *used_fallback = 1;
+    RSVD_HIP(hipMemsetAsync(c->flag_dev, 0, sizeof(int), c->stream));
+    return householder_qr_f64(c, m, n, Y.p, m, nullptr, W.p);
+  }
+  std::swap(Y.p, W.p);
   return 0;
 }
 

@@ -62,6 +62,10 @@ struct Context {
   // pinned host slot for the small device -> host reads of the control flow
   // (convergence and breakdown flags, norms); allocated on first use, kept
   void* pinned = nullptr;
+  // a device int that is zero between calls, and the event behind its copy on
+  // its way to pinned memory (flag_queue)
+  int* flag_dev = nullptr;
+  hipEvent_t flag_ev = nullptr;
   // recorded on the null stream at the entry of device-pointer routines
   hipEvent_t entry_ev = nullptr;
   // Allocation-free mode: while scratch_mode is set, dmalloc hands out
@@ -104,6 +108,12 @@ int order_after_null_stream(Context* c);
 // dst <- bytes (<= 64) at device address src, after the work queued on the
 // library stream: one direct copy into pinned host memory, then a wait.
 int read_small(Context* c, void* dst, const void* src, size_t bytes);
+
+// The context's flag on its way to the host behind the work queued so far, and its
+// value once it has arrived; work may be queued in between.  One at a time; who
+// reads it set clears it.
+int flag_queue(Context* c);
+int flag_wait(Context* c, int* value);
 
 // Device buffer from the pool (contents undefined).  free() returns it.
 int dmalloc(void** p, size_t bytes);
@@ -295,6 +305,14 @@ int coldot_f64(Context* c, int64_t L, int64_t n, const double* X, int64_t ldx, c
 // (optional) reports which path ran.
 int orth_f64(Context* c, int64_t m, int64_t n, double* Y, int64_t ldy, double* R,
              int* used_fallback);
+// Y (m x n, ld m) <- a basis of its range, orthonormal to eps cond(Y)^2: one
+// CholeskyQR step (the buffer may be swapped for another of its size).  Enough
+// for the steps of a power iteration, which pass on a range and need it well
+// conditioned; called twice it is CholeskyQR2.  The same pivot test (cond(Y) up
+// to about 3e6) and Householder fallback as orth_f64.  The power iteration of a
+// 2000 x 1000 SVD (l = 110) took 0.17 ms a step with orth_f64 and its two waits,
+// here 0.08.
+int orth_range_f64(Context* c, int64_t m, int64_t n, DBuf<double>& Y, int* used_fallback);
 // Householder QR in place (blocked geqrf + orgqr, LAPACK's reflectors and
 // sign convention), R (n x n, ld n) optional.  vwork (optional, m * min(n, 32)
 // doubles, device) holds the panel reflectors; allocated when null.

@@ -51,6 +51,10 @@ int ctx_get(Context** out) {
     RSVD_HIP(hipStreamCreateWithFlags(&g_ctx.stream, hipStreamNonBlocking));
     RSVD_HIP(hipEventCreateWithFlags(&g_ctx.entry_ev, hipEventDisableTiming));
     RSVD_HIP(hipHostMalloc(&g_ctx.pinned, 64, hipHostMallocDefault));
+    RSVD_HIP(hipEventCreateWithFlags(&g_ctx.flag_ev, hipEventDisableTiming));
+    RSVD_HIP(hipMalloc(&g_ctx.flag_dev, sizeof(int)));
+    RSVD_HIP(hipMemset(g_ctx.flag_dev, 0, sizeof(int)));
+    RSVD_HIP(hipDeviceSynchronize());
     void* sp = nullptr;
     RSVD_HIP(hipGetSymbolAddress(&sp, HIP_SYMBOL(scratch)));
     if (!sp) return set_error("hipGetSymbolAddress(scratch) returned NULL");
@@ -74,6 +78,23 @@ int read_small(Context* c, void* dst, const void* src, size_t bytes) {
   RSVD_HIP(hipMemcpyAsync(c->pinned, src, bytes, hipMemcpyDeviceToHost, c->stream));
   RSVD_HIP(hipStreamSynchronize(c->stream));
   memcpy(dst, c->pinned, bytes);
+  return 0;
+}
+
+// The flag's place in the pinned slot: past the eight-byte words that the
+// eigensolver's sweeps use.
+constexpr size_t kFlagOffset = 32;
+
+int flag_queue(Context* c) {
+  RSVD_HIP(hipMemcpyAsync(static_cast<char*>(c->pinned) + kFlagOffset, c->flag_dev,
+                          sizeof(int), hipMemcpyDeviceToHost, c->stream));
+  RSVD_HIP(hipEventRecord(c->flag_ev, c->stream));
+  return 0;
+}
+
+int flag_wait(Context* c, int* value) {
+  RSVD_HIP(hipEventSynchronize(c->flag_ev));
+  *value = *reinterpret_cast<volatile int*>(static_cast<char*>(c->pinned) + kFlagOffset);
   return 0;
 }
 

@@ -1,0 +1,35 @@
+"""The fixed-rank SVD's orthonormalisation steps where one Cholesky factor is enough, where the
+second one is needed and where the factorisation breaks down, against the oracle on the same
+Omega (vnum = 1: the small SVD keeps small singular values)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SPECTRA = {"mild": lambda j: np.exp(-j / 20.0),
+           "steep": lambda j: 10.0 ** (-j / 6.0),          # cond(Y) about 3e5 at 33 columns
+           "breakdown": lambda j: 10.0 ** (-j / 2.0),      # 1e16: past the pivot test
+           "rank 12": lambda j: np.where(j < 12, 1.0 / (1.0 + j), 0.0)}
+
+
+@pytest.mark.parametrize("spectrum", SPECTRA)
+@pytest.mark.parametrize("q,s", [(1, 1), (2, 1), (3, 1), (3, 2)])
+def test_against_oracle(gpu_lib, oracle, spectrum, q, s):
+    m, n, k, p = 257, 130, 26, 7
+    rng = np.random.default_rng(3)
+    sigma = SPECTRA[spectrum](np.arange(float(n)))
+    U0, V0 = (np.linalg.qr(rng.standard_normal((d, n)))[0] for d in (m, n))
+    A = (U0 * sigma) @ V0.T
+    gpu_lib.set_seed(99)
+    try:
+        U, S, V = gpu_lib.low_rank_svd_rand_decomp_fixed_rank(A, k, p, 1, q, s)
+    finally:
+        gpu_lib.use_time_seed()
+    Ur, Sr, Vr = oracle.fixed_rank(A, k, p, 1, q, s, seed=99)
+    # the suite's bound for FP64 parity, of sigma_0 = 1
+    assert np.abs(np.diag(S) - np.diag(Sr)).max() < 1e-10
+    assert abs(np.linalg.norm(A - U @ S @ V.T) - np.linalg.norm(A - Ur @ Sr @ Vr.T)) < 1e-10
+    # columns whose own rounding, eps / sigma_j, is below 1e-9
+    keep = np.diag(S) > 1e-6
+    for X in (U[:, keep], V[:, keep]):
+        assert np.abs(X.T @ X - np.eye(keep.sum())).max() < 1e-9
