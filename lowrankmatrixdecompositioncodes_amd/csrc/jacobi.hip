@@ -499,22 +499,29 @@ int colnorms_f64(Context* c, int64_t L, int64_t n, double* W, int64_t ldw, doubl
   return 0;
 }
 
-// rank[j] = position of vals[j] in the sorted order (stable).
-__global__ void rank_kernel(int64_t n, const double* __restrict__ v, int descending,
-                            int64_t* __restrict__ rank) {
-  for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n;
-       j += (int64_t)gridDim.x * blockDim.x) {
-    // NaN ranks as +Inf and ties go by index: a strict total order, so the
-    // ranks are a permutation whatever the values (a NaN would otherwise
-    // compare false both ways and two entries would share a rank)
-    const double x = isnan(v[j]) ? INFINITY : v[j];
-    int64_t r = 0;
-    for (int64_t i = 0; i < n; ++i) {
-      const double y = isnan(v[i]) ? INFINITY : v[i];
-      bool before = descending ? (y > x) : (y < x);
-      if (before || (y == x && i < j)) ++r;
-    }
+// rank[j] = position of v[j] in the sorted order (stable), sorted[rank[j]] = v[j].  A
+// wave a value (a thread a value is a chain of n loads: 14 us at n = 110, 43 at
+// 317; here under 4, and the values' own launch is gone).
+__global__ void __launch_bounds__(256)
+rank_kernel(int64_t n, const double* __restrict__ v, int descending, int64_t* __restrict__ rank,
+            double* __restrict__ sorted) {
+  const int64_t j = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (j >= n) return;
+  // NaN ranks as +Inf and ties go by index: a strict total order, so the
+  // ranks are a permutation whatever the values (a NaN would otherwise
+  // compare false both ways and two entries would share a rank)
+  const double own = v[j], x = isnan(own) ? INFINITY : own;
+  int r = 0;
+  for (int64_t i = lane; i < n; i += 64) {
+    const double y = isnan(v[i]) ? INFINITY : v[i];
+    const bool before = descending ? (y > x) : (y < x);
+    r += before || (y == x && i < j);
+  }
+  for (int off = 32; off > 0; off >>= 1) r += __shfl_xor(r, off, 64);
+  if (lane == 0) {
     rank[j] = r;
+    sorted[r] = own;
   }
 }
 
@@ -527,13 +534,6 @@ __global__ void permute_cols_kernel(int64_t rows, int64_t n, const double* __res
     int64_t i = idx % rows, j = idx / rows;
     dst[i + rank[j] * ldd] = src[i + j * lds];
   }
-}
-
-__global__ void permute_vals_kernel(int64_t n, const double* __restrict__ src,
-                                    const int64_t* __restrict__ rank, double* __restrict__ dst) {
-  for (int64_t j = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n;
-       j += (int64_t)gridDim.x * blockDim.x)
-    dst[rank[j]] = src[j];
 }
 
 static int permute_matrix(Context* c, int64_t rows, int64_t n, double* X, int64_t ldx,
@@ -557,12 +557,8 @@ int sort_pairs_f64(Context* c, int64_t n, double* vals, int descending, double* 
   DBuf<double> tv;
   RSVD_TRY(rank.alloc((size_t)n));
   RSVD_TRY(tv.alloc((size_t)n));
-  int blocks = (int)((n + 255) / 256);
-  hipLaunchKernelGGL(rank_kernel, dim3(blocks), dim3(256), 0, c->stream, n, (const double*)vals,
-                     descending, rank.p);
-  RSVD_LAUNCH_CHECK();
-  hipLaunchKernelGGL(permute_vals_kernel, dim3(blocks), dim3(256), 0, c->stream, n,
-                     (const double*)vals, (const int64_t*)rank.p, tv.p);
+  hipLaunchKernelGGL(rank_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, c->stream, n,
+                     (const double*)vals, descending, rank.p, tv.p);
   RSVD_LAUNCH_CHECK();
   RSVD_HIP(hipMemcpyAsync(vals, tv.p, sizeof(double) * n, hipMemcpyDeviceToDevice, c->stream));
   RSVD_TRY(permute_matrix(c, rowsX, n, X, ldx, rank.p));
