@@ -506,7 +506,9 @@ struct GemmPlan {
 // a wave's MFMAs (64 cycles each in FP64, 32 in FP32) plus half a microsecond;
 // k slices add a launch and their traffic.  Against the best of all cuts,
 // measured on 25 shapes (26 to 50000 rows, 20 to 1792 columns), its choice was
-// within 8% of the fastest.
+// within 8% of the fastest.  In an allocation-free call the slices are no more
+// than the largest free range of the scratch array holds: a call never needs more
+// than its panels for the sake of a slice.
 template <typename T>
 static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice,
                           int split = 0) {
@@ -521,6 +523,7 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
                                       : 250.0) / 2400.0;
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
+  const int64_t room = c->scratch_mode ? (int64_t)(scratch_room(c) / sizeof(T)) / (M * N) : kblocks;
   GemmPlan best{};
   double best_cost = 1e300;
   for (int t = 0; t < 3; ++t) {
@@ -532,6 +535,7 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
       for (int64_t y = 0; y < gy; ++y) tiles += sym_tiles(y, gx, d.bm, d.bn);
     }
     int64_t smax = one_slice ? 1 : kblocks / (2 * d.ks);
+    smax = smax > room ? room : smax;
     smax = smax < 1 ? 1 : (smax > 64 ? 64 : smax);
     // FP32: a wave's running sum takes at most 512 products where the output
     // is small enough to be sliced (its rounding grows with the length: at

@@ -118,6 +118,8 @@ int flag_wait(Context* c, int* value);
 // Device buffer from the pool (contents undefined).  free() returns it.
 int dmalloc(void** p, size_t bytes);
 void dfree(void* p);
+// Bytes of the scratch array's largest free range (allocation-free calls).
+size_t scratch_room(const Context* c);
 // Release every pooled buffer back to HIP.
 void pool_trim();
 

@@ -136,6 +136,15 @@ static int scratch_alloc(Context* c, void** p, size_t bytes) {
   return 0;
 }
 
+size_t scratch_room(const Context* c) {
+  size_t at = 0, best = 0;
+  for (const auto& r : c->scratch_live) {
+    if (r.first - at > best) best = r.first - at;
+    at = r.first + r.second;
+  }
+  return kScratchBytes - at > best ? kScratchBytes - at : best;
+}
+
 static bool scratch_free(Context* c, void* p) {
   if (!c->scratch || p < (void*)c->scratch || p >= (void*)(c->scratch + kScratchBytes))
     return false;
