@@ -485,6 +485,9 @@ int orth_range_f64(Context* c, int64_t m, int64_t n, DBuf<double>& Y, int* used_
     RSVD_HIP(hipMemsetAsync(c->flag_dev, 0, sizeof(int), c->stream));
     return householder_qr_f64(c, m, n, Y.p, m, nullptr, W.p);
   }
+  // an allocation-free call keeps its panels in their places: a swap would leave a
+  // hole of m n doubles among them that a longer panel does not fit
+  if (c->scratch_mode) return copy2d_f64(c, m, n, W.p, m, Y.p, m);
   std::swap(Y.p, W.p);
   return 0;
 }

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
     (8303, 4466, 990, 10, 2, 2, 2, True),
     (6664, 5118, 864, 10, 2, 2, 1, False),
     (12000, 9000, 500, 10, 1, 2, 1, False),   # a product of a whole panel
+    (22344, 23872, 237, 10, 1, 2, 1, False),  # n > m: panels that must not move
 ])
 def test_noalloc_near_the_scratch_limit(gpu_lib, m, n, k, p, vnum, q, s, omega):
     rp = gpu_lib
