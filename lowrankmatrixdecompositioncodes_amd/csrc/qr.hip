@@ -473,16 +473,23 @@ int orth_range_f64(Context* c, int64_t m, int64_t n, DBuf<double>& Y, int* used_
   RSVD_TRY(acc.alloc((size_t)(n * n)));
   RSVD_TRY(diag0.alloc((size_t)n));
   RSVD_TRY(gemm_f64(c, 'T', 'N', n, n, m, 1.0, Y.p, m, Y.p, m, 0.0, G.p, n));
-  RSVD_TRY(chol_inv_launch(c, n, G.p, R.p, Rinv.p, c->flag_dev, diag0.p, acc.p));
-  // the pivot test's verdict goes to the host ahead of the product, which runs
-  // while the host waits for it: Y stays as it is until it is known
-  RSVD_TRY(flag_queue(c));
-  RSVD_TRY(gemm_f64(c, 'N', 'N', m, n, n, 1.0, Y.p, m, Rinv.p, n, 0.0, W.p, m));
+  auto factor_and_apply = [&](int* h) {
+    RSVD_TRY(chol_inv_launch(c, n, G.p, R.p, Rinv.p, c->flag_dev, diag0.p, acc.p));
+    // the pivot test's verdict goes to the host ahead of the product, which runs
+    // while the host waits for it: Y stays as it is until it is known
+    RSVD_TRY(flag_queue(c));
+    RSVD_TRY(gemm_f64(c, 'N', 'N', m, n, n, 1.0, Y.p, m, Rinv.p, n, 0.0, W.p, m));
+    return flag_wait(c, h);
+  };
   int h = 0;
-  RSVD_TRY(flag_wait(c, &h));
-  if (h) {
+  const int rc = factor_and_apply(&h);
+  // set by a bad pivot, or perhaps by one that an error kept from being read:
+  // either way the next factorisation finds it clear
+  if (rc || h) {
+    const hipError_t e = hipMemsetAsync(c->flag_dev, 0, sizeof(int), c->stream);
+    if (rc) return rc;
+    RSVD_HIP(e);
     if (used_fallback) *used_fallback = 1;
-    RSVD_HIP(hipMemsetAsync(c->flag_dev, 0, sizeof(int), c->stream));
     return householder_qr_f64(c, m, n, Y.p, m, nullptr, W.p);
   }
   // an allocation-free call keeps its panels in their places: a swap would leave a

@@ -33,3 +33,34 @@ def test_against_oracle(gpu_lib, oracle, spectrum, q, s):
     keep = np.diag(S) > 1e-6
     for X in (U[:, keep], V[:, keep]):
         assert np.abs(X.T @ X - np.eye(keep.sum())).max() < 1e-9
+
+
+def test_breakdown_leaves_nothing_behind(gpu_lib):
+    """A call whose orthonormalisations all break down (a zero matrix) between two calls on a
+    full-rank matrix: the second of them queues the products the first did, so no Cholesky
+    verdict of the call in between is read again."""
+    rp = gpu_lib
+    lib = rp.load()
+    m, n, k = 300, 200, 24
+    A = np.random.default_rng(8).standard_normal((m, n))
+    dA = rp.DeviceMatrix.from_host(A)
+    dZ = rp.DeviceMatrix.from_host(np.zeros((m, n)))
+    U, S, V = rp.DeviceMatrix(m, k), rp.DeviceMatrix(k, 1), rp.DeviceMatrix(n, k)
+
+    def call(X):
+        rc = lib.rsvd_dev_fixed_rank(X.ptr, m, n, m, k, 6, 1, 2, 1, 5, None, U.ptr, m, S.ptr,
+                                     V.ptr, n)
+        assert rc == 0, rp.last_error()
+        return rp.kstats("gemm_f64")[1], S.to_host()
+
+    lib.rsvd_kstats_reset()
+    lib.rsvd_kstats_enable(1)
+    try:
+        c0, s0 = call(dA)
+        c1, s1 = call(dZ)
+        c2, s2 = call(dA)
+    finally:
+        lib.rsvd_kstats_enable(0)
+        lib.rsvd_kstats_reset()
+    assert c1 - c0 > c0 and c2 - c1 == c0
+    assert np.all(s1 == 0.0) and np.array_equal(s0, s2)
