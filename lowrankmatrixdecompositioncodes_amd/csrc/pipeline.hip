@@ -147,7 +147,9 @@ int fixed_rank_f64(Context* c, const double* A, int64_t m, int64_t n, int64_t ld
     if ((2 * j - 1) % s == 0) { RSVD_TRY(orth_range_f64(c, n, l, Z, &f1)); fb += f1; }
     RSVD_TRY(gemm_f64_tag(c, "apass_f64", 'N', 'N', m, l, n, 1.0, A, lda, Z.p, n, 0.0, Y.p, m));
   }
-  for (int pass = 0; pass < 2; ++pass) {                               // rra.c:129-130
+  // two steps (CholeskyQR2), or the Householder QR that the first one ended in
+  f1 = 0;
+  for (int pass = 0; pass < 2 && !f1; ++pass) {                        // rra.c:129-130
     RSVD_TRY(orth_range_f64(c, m, l, Y, &f1));
     fb += f1;
   }

@@ -62,5 +62,28 @@ def test_breakdown_leaves_nothing_behind(gpu_lib):
     finally:
         lib.rsvd_kstats_enable(0)
         lib.rsvd_kstats_reset()
-    assert c1 - c0 > c0 and c2 - c1 == c0
+    assert c1 - c0 != c0 and c2 - c1 == c0
     assert np.all(s1 == 0.0) and np.array_equal(s0, s2)
+
+
+@pytest.mark.parametrize("rank,factors", [(60, 2), (12, 1)])
+def test_one_qr_after_a_breakdown(gpu_lib, rank, factors):
+    """The last orthonormalisation (q = 1: the only one) factors two Grams, or one that breaks
+    down: the Householder QR that follows is the end of it."""
+    rp = gpu_lib
+    lib = rp.load()
+    m, n, k = 300, 200, 24
+    rng = np.random.default_rng(9)
+    dA = rp.DeviceMatrix.from_host(rng.standard_normal((m, rank)) @ rng.standard_normal((rank, n)))
+    U, S, V = rp.DeviceMatrix(m, k), rp.DeviceMatrix(k, 1), rp.DeviceMatrix(n, k)
+    lib.rsvd_kstats_reset()
+    lib.rsvd_kstats_enable(1)
+    try:
+        rc = lib.rsvd_dev_fixed_rank(dA.ptr, m, n, m, k, 6, 2, 1, 1, 5, None, U.ptr, m, S.ptr,
+                                     V.ptr, n)
+        assert rc == 0, rp.last_error()
+        count = rp.kstats("chol_inv")[1]
+    finally:
+        lib.rsvd_kstats_enable(0)
+        lib.rsvd_kstats_reset()
+    assert count == factors
