@@ -55,7 +55,8 @@ pqr_init_kernel(int64_t m, int64_t n, const double* __restrict__ A, int64_t lda,
 // A step is bound by latency (two dependent rounds of loads, two reductions and
 // the launch), so one launch that repeats the pivot's work in every workgroup
 // beats a pivot launch and an update launch: 7.5 us against 11.4 us a step at
-// 384 x 1200.
+// 384 x 1200.  The repeated work, n norms a workgroup and n / 4 workgroups, grows as
+// n^2: pivoted_qr_f64 has the line.
 // LDSV: the pivot column's rows fit the LDS buffer.
 constexpr int kPqrLds = 4096, kPqrKeep = 8;
 
@@ -221,6 +222,133 @@ pqr_gather_kernel(int64_t m, int64_t n, int64_t kmax, const double* __restrict__
   }
 }
 
+// The factorisation in two launches a step, in place (pivoted_qr_f64 chooses it for
+// wide and for large matrices).
+// Step i, part 1 (one workgroup): pivot = first index of max vn1[i..n)
+// (idamax), swap it into column i (vn of the pivot's slot inherits column i's,
+// as dlaqp2), then the reflector of A(i:m, i) in dlarfg's convention: beta =
+// -sign(alpha) hypot(alpha, ||x||), tau = (beta - alpha) / beta, v = x /
+// (alpha - beta), R_ii = beta; tau = 0 for a single row or a zero x.
+__global__ void __launch_bounds__(1024)
+pqr_pivot_kernel(int64_t m, int64_t n, double* __restrict__ A, int64_t lda, int64_t i,
+                 double* __restrict__ vn1, double* __restrict__ vn2, int* __restrict__ perm,
+                 double* __restrict__ tau) {
+  __shared__ double sv[16];
+  __shared__ int64_t si[16];
+  __shared__ int64_t s_pvt;
+  __shared__ double s_scale;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  double best = -1.0;
+  int64_t bidx = n;
+  for (int64_t j = i + tid; j < n; j += 1024) {
+    const double v = vn1[j];
+    if (v > best) { best = v; bidx = j; }
+  }
+  for (int off = 32; off > 0; off >>= 1) {
+    const double ov = __shfl_xor(best, off, 64);
+    const int64_t oi = __shfl_xor(bidx, off, 64);
+    if (ov > best || (ov == best && oi < bidx)) { best = ov; bidx = oi; }
+  }
+  if (lane == 0) { sv[w] = best; si[w] = bidx; }
+  __syncthreads();
+  if (tid == 0) {
+    double b = sv[0];
+    int64_t bi = si[0];
+    for (int k = 1; k < 16; ++k)
+      if (sv[k] > b || (sv[k] == b && si[k] < bi)) { b = sv[k]; bi = si[k]; }
+    s_pvt = (bi < n) ? bi : i;
+  }
+  __syncthreads();
+  const int64_t pvt = s_pvt;
+  if (pvt != i) {
+    double* ci = A + i * lda;
+    double* cp = A + pvt * lda;
+    for (int64_t r = tid; r < m; r += 1024) {
+      const double t = ci[r];
+      ci[r] = cp[r];
+      cp[r] = t;
+    }
+    if (tid == 0) {
+      const int t = perm[pvt];
+      perm[pvt] = perm[i];
+      perm[i] = t;
+      vn1[pvt] = vn1[i];
+      vn2[pvt] = vn2[i];
+    }
+  }
+  __syncthreads();
+  double* x = A + i + i * lda;
+  const int64_t len = m - i;
+  double s = 0.0;
+  for (int64_t r = 1 + tid; r < len; r += 1024) s += x[r] * x[r];
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if (lane == 0) sv[w] = s;
+  __syncthreads();
+  if (tid == 0) {
+    double ss = 0.0;
+    for (int k = 0; k < 16; ++k) ss += sv[k];
+    const double alpha = x[0];
+    if (len <= 1 || ss == 0.0) {
+      tau[i] = 0.0;
+      s_scale = 0.0;
+    } else {
+      const double xn = sqrt(ss);
+      const double a = fabs(alpha), big = fmax(a, xn), sml = fmin(a, xn);
+      const double h = (sml == 0.0) ? big : big * sqrt(1.0 + (sml / big) * (sml / big));
+      const double beta = (alpha >= 0.0) ? -h : h;
+      tau[i] = (beta - alpha) / beta;
+      s_scale = 1.0 / (alpha - beta);
+      x[0] = beta;
+    }
+  }
+  __syncthreads();
+  const double sc = s_scale;
+  if (sc != 0.0)
+    for (int64_t r = 1 + tid; r < len; r += 1024) x[r] *= sc;
+}
+
+// Step i, part 2: columns c > i get H_i applied (rows i..m-1) and their
+// partial norms downdated (dlaqp2's rule, recomputed from the column when the
+// downdate cancelled); one wave per column.
+__global__ void __launch_bounds__(256)
+pqr_update_kernel(int64_t m, int64_t n, double* __restrict__ A, int64_t lda, int64_t i,
+                  double* __restrict__ vn1, double* __restrict__ vn2,
+                  const double* __restrict__ tau) {
+  const int lane = threadIdx.x & 63;
+  const int64_t c = i + 1 + (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (c >= n) return;
+  const double t = tau[i];
+  const double* v = A + i * lda;  // v_i = 1, v_r = A(r, i) below
+  double* y = A + c * lda;
+  double yi = y[i];
+  if (t != 0.0) {
+    double s = 0.0;
+    for (int64_t r = i + lane; r < m; r += 64) s += (r == i ? 1.0 : v[r]) * y[r];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    const double wv = t * s;
+    for (int64_t r = i + lane; r < m; r += 64) y[r] -= (r == i ? 1.0 : v[r]) * wv;
+    yi -= wv;
+  }
+  const double n1 = vn1[c];
+  if (n1 != 0.0) {
+    double temp = fabs(yi) / n1;
+    temp = fmax(1.0 - temp * temp, 0.0);
+    const double r2 = n1 / vn2[c];
+    if (temp * r2 * r2 <= kTol3z) {
+      double s = 0.0;
+      for (int64_t r = i + 1 + lane; r < m; r += 64) s += y[r] * y[r];
+      for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+      if (lane == 0) {
+        const double nv = (i + 1 < m) ? sqrt(s) : 0.0;
+        vn1[c] = nv;
+        vn2[c] = nv;
+      }
+    } else if (lane == 0) {
+      vn1[c] = n1 * sqrt(temp);
+    }
+  }
+}
+
 // Inverse of each 64 x 64 diagonal block of an upper triangular R (k x k):
 // thread j solves R_bb x = e_j by back substitution.
 __global__ void __launch_bounds__(64)
@@ -317,11 +445,46 @@ int grid_for(int64_t total) {
 
 }  // namespace
 
+constexpr int64_t kPqrOneLaunchCols = 3584, kPqrOneLaunchSize = int64_t(1) << 25;
+
+static int pivoted_qr_in_place(Context* c, int64_t m, int64_t n, double* A, int64_t lda, int* perm,
+                               double* tau) {
+  DBuf<double> vn1, vn2;
+  RSVD_TRY(vn1.alloc((size_t)n));
+  RSVD_TRY(vn2.alloc((size_t)n));
+  KTimer kt(c, "pivoted_qr");
+  hipLaunchKernelGGL(pqr_init_kernel, dim3((unsigned)((n + 3) / 4)), dim3(256), 0, c->stream, m,
+                     n, (const double*)A, lda, vn1.p, vn2.p, perm);
+  RSVD_LAUNCH_CHECK();
+  const int64_t kmax = m < n ? m : n;
+  for (int64_t i = 0; i < kmax; ++i) {
+    hipLaunchKernelGGL(pqr_pivot_kernel, dim3(1), dim3(1024), 0, c->stream, m, n, A, lda, i,
+                       vn1.p, vn2.p, perm, tau);
+    RSVD_LAUNCH_CHECK();
+    const int64_t rest = n - i - 1;
+    if (rest > 0) {
+      hipLaunchKernelGGL(pqr_update_kernel, dim3((unsigned)((rest + 3) / 4)), dim3(256), 0,
+                         c->stream, m, n, A, lda, i, vn1.p, vn2.p, (const double*)tau);
+      RSVD_LAUNCH_CHECK();
+    }
+  }
+  return 0;
+}
+
 int pivoted_qr_f64(Context* c, int64_t m, int64_t n, double* A, int64_t lda, int* perm,
                    double* tau) {
   if (m <= 0 || n <= 0) return 0;
   if (lda < m) return set_error("pivoted_qr: lda %lld < m %lld", (long long)lda, (long long)m);
   const int64_t kmax = m < n ? m : n;
+  // One launch a step where its latency counts.  Its scan of all norms in every
+  // workgroup is 3 n^2 bytes a step, and past 4 n_cu workgroups of four columns
+  // they no longer run at once: against the two launches 384 x 1200 took 0.65 of
+  // the time, 384 x 3600 0.90, 1000 x 3600 0.82, 64 x 3600 as long, 1000 x 4400 1.3,
+  // 384 x 20000 4.1 times as long.  With the rows the step comes to be bound by its
+  // traffic (6000 x 3000 0.92, 100000 x 300 0.93, 400000 x 100 and 40000 x 1000 0.98),
+  // and its copies of the matrix are not worth their memory: up to 2^25 entries.
+  if (n > kPqrOneLaunchCols || m * n > kPqrOneLaunchSize)
+    return pivoted_qr_in_place(c, m, n, A, lda, perm, tau);
   DBuf<double> vn1, vn2, V, betas, W;
   DBuf<int> pos;
   RSVD_TRY(vn1.alloc((size_t)(2 * n)));
