@@ -506,9 +506,12 @@ struct GemmPlan {
 // a wave's MFMAs (64 cycles each in FP64, 32 in FP32) plus half a microsecond;
 // k slices add a launch and their traffic.  Against the best of all cuts,
 // measured on 25 shapes (26 to 50000 rows, 20 to 1792 columns), its choice was
-// within 8% of the fastest.  In an allocation-free call the slices are no more
-// than the largest free range of the scratch array holds: a call never needs more
-// than its panels for the sake of a slice.
+// within 8% of the fastest.  The slices hold at most kMaxSliceElems elements: what
+// they save on a larger output, part of a last round of workgroups, is not worth
+// the memory.  In an allocation-free call they are also no more than the largest
+// free range of the scratch array holds: a call never needs more than its panels
+// for the sake of a slice.
+constexpr int64_t kMaxSliceElems = int64_t(1) << 28;
 template <typename T>
 static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice,
                           int split = 0) {
@@ -523,7 +526,8 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
                                       : 250.0) / 2400.0;
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
-  const int64_t room = c->scratch_mode ? (int64_t)(scratch_room(c) / sizeof(T)) / (M * N) : kblocks;
+  int64_t room = kMaxSliceElems / (M * N);
+  if (c->scratch_mode) room = std::min(room, (int64_t)(scratch_room(c) / sizeof(T)) / (M * N));
   GemmPlan best{};
   double best_cost = 1e300;
   for (int t = 0; t < 3; ++t) {
