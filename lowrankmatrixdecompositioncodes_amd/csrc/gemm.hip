@@ -37,6 +37,7 @@
 // serves the smaller products of gemm_lp.hip.
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <type_traits>
 
 #include <rocblas/rocblas.h>
@@ -501,29 +502,46 @@ struct GemmPlan {
   int64_t gx, gy, tiles, kchunk;
 };
 
-// The cheapest cut by a model of the kernel's time in microseconds: the
-// workgroups run in rounds of one a CU (one wave on every SIMD), each as long as
-// a wave's MFMAs (64 cycles each in FP64, 32 in FP32) plus half a microsecond;
-// k slices add a launch and their traffic.  Against the best of all cuts,
-// measured on 25 shapes (26 to 50000 rows, 20 to 1792 columns), its choice was
-// within 8% of the fastest.  The slices hold at most kMaxSliceElems elements: what
-// they save on a larger output, part of a last round of workgroups, is not worth
-// the memory.  In an allocation-free call they are also no more than the largest
-// free range of the scratch array holds: a call never needs more than its panels
-// for the sake of a slice.
+// The model's constants of a precision, in microseconds: a k block of a 16 x 16 block
+// of C on one wave; the time of each tile over that, with op(A) row-contiguous and
+// k-contiguous; the workgroups a CU that a lone one takes the time of (its waves wait
+// for their operands with nothing else to run); a workgroup's start and end; what
+// slices add, once and an element; what a long k loop adds.
+struct CutCost {
+  double block, slow[2][3], alone[3], group[3], launch, elem, drift;
+};
+
+// The cheapest cut by a model of the kernel's time: rounds of one workgroup a CU (one
+// wave on every SIMD), each as long as a wave's k blocks -- its MFMAs, 64 cycles each
+// in FP64 and 32 in FP32; the split modes (16 each) wait for their operands far
+// longer.  In FP64 workgroups that share operands drift apart in a long k loop and
+// fetch them again: past 96 blocks a wave the time grows, by `drift` at 192.
+// Fitted to a grid of cuts of 1750 FP64 and 870 FP32 and split products and Grams (16
+// to 90000 rows, even and odd sizes, every transposition): its choice is 2.2% (FP64)
+// and 2.5% (FP32) slower than the fastest of them in the geometric mean.  With rounds
+// and MFMAs alone it chose one workgroup a CU with a long loop too often, above all
+// for odd sizes, whose rows straddle cache lines: A^T B at 4013 x 50 x 18712 373 us,
+// now 235, at 2271 x 110 x 14730 279 and 205 us, at 100 x 4073 x 43721 1478 and 998 us.
+// The slices hold at most kMaxSliceElems elements: what they save on a larger output,
+// part of a last round of workgroups, is not worth the memory.  In an allocation-free
+// call they are also no more than the largest free range of the scratch array holds: a
+// call never needs more than its panels for the sake of a slice.
 constexpr int64_t kMaxSliceElems = int64_t(1) << 28;
 template <typename T>
-static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym, bool one_slice,
-                          int split = 0) {
+static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, bool sym,
+                          bool one_slice, int split = 0) {
   static const struct {
-    int bm, bn, ks, mfma;
-    double slow;  // measured time over the MFMAs' (operand loads a wave does not share)
-  } kTiles[3] = {{128, 64, 1, 8, 1.0}, {64, 32, 4, 8, 1.05}, {32, 32, 4, 4, 1.05}};
+    int bm, bn, ks, blocks;  // blocks of C a wave owns
+  } kTiles[3] = {{128, 64, 1, 8}, {64, 32, 4, 8}, {32, 32, 4, 4}};
+  static const CutCost
+      kF64 = {256.0 / 2400, {{1.1, 1.1, 1.13}, {1.26, 1.26, 1.1}}, {1.3, 2.0, 1.1},
+              {0.5, 0.8, 0.8}, 2.0, 1.5e-6, 0.4},
+      kF32 = {256.0 / 2400, {{1.1, 1.1, 1.0}, {1.1, 1.1, 1.0}}, {1.6, 1.4, 1.0},
+              {0.3, 0.3, 0.3}, 2.0, 5e-7, 0.0},
+      kSplit = {0.13, {{1.0, 1.1, 1.0}, {1.0, 1.1, 1.0}}, {1.2, 2.0, 1.2},
+                {0.3, 0.3, 0.3}, 2.0, 1e-6, 0.0};
+  const CutCost& m = sizeof(T) == 8 ? kF64 : (split == 0 ? kF32 : kSplit);
   constexpr int64_t depth = KBlock<T>::kDepth;
-  // cycles of a 16 x 16 block of C and a k block; the split modes wait for their
-  // operands (1.5 to 2 KB a block) far longer than for their MFMAs (16 each)
-  const double block_us = (split == 0 ? (sizeof(T) == 8 ? 64.0 : 32.0) * KBlock<T>::kSteps
-                                      : 250.0) / 2400.0;
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
   int64_t room = kMaxSliceElems / (M * N);
@@ -552,9 +570,12 @@ static GemmPlan gemm_plan(Context* c, int64_t M, int64_t N, int64_t K, bool sym,
     for (int64_t s = smin; s <= smax; ++s) {
       const int64_t kb = (kblocks + s - 1) / s;
       if ((kblocks + kb - 1) / kb != s && s > smin) continue;  // as with a smaller s
-      const double wave = (double)((kb + d.ks - 1) / d.ks) * d.mfma * block_us;
-      double cost = (double)((tiles * s + cus - 1) / cus) * (wave * d.slow + 0.5);
-      if (s > 1) cost += 2.0 + 2e-6 * (double)s * (double)M * (double)N * sizeof(T) / 8;
+      const double rounds = (double)((tiles * s + cus - 1) / cus);
+      const double blocks = (double)((kb + d.ks - 1) / d.ks);
+      double wave = blocks * d.blocks * m.block * m.slow[ka][t];
+      if (blocks > 96) wave *= 1.0 + m.drift * std::min(1.0, std::log2(blocks / 96.0));
+      double cost = std::max(rounds, m.alone[t]) * wave + rounds * m.group[t];
+      if (s > 1) cost += m.launch + m.elem * (double)s * (double)M * (double)N;
       if (cost < best_cost) {
         best_cost = cost;
         best = GemmPlan{t, (int)((kblocks + kb - 1) / kb), gx, gy, tiles, kb * depth};
@@ -700,7 +721,7 @@ static int gemm_any(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t 
   // formed and stored on both sides of it
   const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == T(0);
-  return launch_gemm<T>(c, gemm_plan<T>(c, M, N, K, sym, false), ta, tb, M, N, K, alpha, A, lda, B,
+  return launch_gemm<T>(c, gemm_plan<T>(c, tA, M, N, K, sym, false), ta, tb, M, N, K, alpha, A, lda, B,
                         ldb, beta, C, ldc, nullptr, sym, tag);
 }
 
@@ -709,7 +730,7 @@ int gemm_split(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t
                float* C, int64_t ldc, int split) {
   const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == 0.0f;
-  const GemmPlan pl = gemm_plan<float>(c, M, N, K, sym, false, split);
+  const GemmPlan pl = gemm_plan<float>(c, tA, M, N, K, sym, false, split);
   return split == 1 ? launch_gemm<float, 1>(c, pl, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C,
                                             ldc, nullptr, sym, tag)
                     : launch_gemm<float, 3>(c, pl, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C,
@@ -743,7 +764,7 @@ int gemm_f64_deflate(Context* c, int64_t M, int64_t N, int64_t K, const double* 
     return 0;
   }
   const int64_t k = K > 0 ? K : 1;
-  const GemmPlan pl = gemm_plan<double>(c, M, N, k, false, true);
+  const GemmPlan pl = gemm_plan<double>(c, false, M, N, k, false, true);
   const int64_t nparts = pl.gx * pl.gy;
   DBuf<double> part;
   RSVD_TRY(part.alloc((size_t)nparts));
