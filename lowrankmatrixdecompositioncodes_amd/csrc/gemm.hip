@@ -546,6 +546,26 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
   const int64_t kblocks = (K + depth - 1) / depth;
   int64_t room = kMaxSliceElems / (M * N);
   if (c->scratch_mode) room = std::min(room, (int64_t)(scratch_room(c) / sizeof(T)) / (M * N));
+  // FP32: a wave's running sum takes at most `longest` products as far as 64 slices
+  // allow (its rounding grows with the length).  512 where the output is small: at
+  // 65536 rows the Gram behind the last CholeskyQR step needs it.  For larger ones what
+  // 128 x 64 tiles sliced for two workgroups a CU take, 256 products a slice or more;
+  // of two such tiles a CU or more the sums are not cut.
+  int64_t longest = 0;
+  if (sizeof(T) == 4 && !one_slice) {
+    longest = 512;
+    if (M * N > (int64_t(1) << 20)) {
+      const int64_t gx = (M + 127) / 128, gy = (N + 63) / 64;
+      int64_t tiles = gx * gy;
+      if (sym) {
+        tiles = 0;
+        for (int64_t y = 0; y < gy; ++y) tiles += sym_tiles(y, gx, 128, 64);
+      }
+      const int64_t most = tiles < 2 * cus ? std::min<int64_t>(64, K / 256) : 1;
+      const int64_t slices = most > 1 ? pick_k_slices(tiles, 2 * cus, most) : 1;
+      longest = std::max<int64_t>(longest, (K + slices - 1) / slices);
+    }
+  }
   GemmPlan best{};
   double best_cost = 1e300;
   for (int t = 0; t < 3; ++t) {
@@ -559,12 +579,9 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
     int64_t smax = one_slice ? 1 : kblocks / (2 * d.ks);
     smax = smax > room ? room : smax;
     smax = smax < 1 ? 1 : (smax > 64 ? 64 : smax);
-    // FP32: a wave's running sum takes at most 512 products where the output
-    // is small enough to be sliced (its rounding grows with the length: at
-    // 65536 rows the Gram behind the last CholeskyQR step needs it)
     int64_t smin = 1;
-    if (sizeof(T) == 4 && !one_slice && M * N <= (int64_t(1) << 20)) {
-      smin = (K + 512 * d.ks - 1) / (512 * d.ks);
+    if (longest > 0) {
+      smin = (K + longest * d.ks - 1) / (longest * d.ks);
       smin = smin < smax ? smin : smax;
     }
     for (int64_t s = smin; s <= smax; ++s) {

@@ -61,3 +61,22 @@ def test_gram_is_symmetric(gpu_lib, n, k, dtype):
         Y = X.astype(np.float64) if ta == "T" else X.T.astype(np.float64)
         assert np.array_equal(G, G.T)
         assert np.all(np.abs(G - Y.T @ Y) <= (k + 4) * eps * (np.abs(Y).T @ np.abs(Y)))
+
+
+def test_fp32_sums_stay_short(gpu_lib):
+    """An FP32 product with a long k and an output past 2^20 entries: its running sums take at most
+    K / 35 = 1728 products.  With positive terms each rounding errs by u / sqrt(3) of the sum so far
+    (u = 2^-24): u sqrt(1728) / 3 of a sum, over sqrt(35) independent ones 1.4e-7 in the root mean
+    square, and u / sqrt(3) for the last rounding; a single sum a quarter of K long reaches 1.2e-6."""
+    rp = gpu_lib
+    m = n = 1200
+    k = 60000
+    rng = np.random.default_rng(4)
+    A = rng.uniform(0.5, 1.5, (m, k)).astype(np.float32)
+    B = rng.uniform(0.5, 1.5, (k, n)).astype(np.float32)
+    dA, dB = rp.DeviceMatrix.from_host(A), rp.DeviceMatrix.from_host(B)
+    dC = rp.DeviceMatrix(m, n, np.float32)
+    rc = rp.load().rsvd_dev_gemm(1, b"N", b"N", m, n, k, 1.0, dA.ptr, m, dB.ptr, k, 0.0, dC.ptr, m)
+    assert rc == 0, rp.last_error()
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    assert np.sqrt(np.mean((dC.to_host() / want - 1.0) ** 2)) <= 3e-7
