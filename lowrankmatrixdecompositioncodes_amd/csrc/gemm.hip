@@ -456,6 +456,96 @@ gemm_kernel(const GemmArgs<T> g) {
   }
 }
 
+// FP32 with the operands staged: 128 x BN tiles of C, 16 elements of k at a time in LDS,
+// for the products that gemm_staged chooses.  An FP32 MFMA takes half the cycles of an
+// FP64 one for the same element count, and a wave of gemm_kernel that reads two
+// row-contiguous operands off the cache lines' boundaries fetches five lines where three
+// hold its data; here a workgroup fetches each once.
+template <bool TA, bool TB, int BN>
+__global__ void __launch_bounds__(kThreads, 2)
+gemm_staged_kernel(const GemmArgs<float> g) {
+  constexpr int BM = 128, BK = 16, PAD = 4;
+  constexpr int TM = 4, TN = BN / 32;  // 16 x 16 blocks of a wave (two waves along each side)
+  constexpr int EA = BM * BK / kThreads, EB = BN * BK / kThreads;
+  __shared__ float As[BK][BM + PAD], Bs[BK][BN + PAD];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lk = lane >> 4;
+  // the tile order of gemm_kernel
+  const int64_t gx = g.gx, gy = g.gy, nt = gridDim.x;
+  const int64_t xcd = blockIdx.x & 7, q = nt >> 3, r = nt & 7;
+  const int64_t t = xcd * q + (xcd < r ? xcd : r) + (blockIdx.x >> 3);
+  const int64_t m0 = (gy <= gx ? t / gy : t % gx) * BM, n0 = (gy <= gx ? t % gy : t / gx) * BN;
+  const int64_t kbeg = (int64_t)blockIdx.y * g.kchunk;
+  const int64_t kend = (kbeg + g.kchunk < g.K) ? kbeg + g.kchunk : g.K;
+  float* C = g.C + (int64_t)blockIdx.y * g.zstride;
+  // this thread's elements of a stage: row ma and k ka of A (and of B), the e-th one
+  // sa elements further along the other dimension
+  const int ma = TA ? tid / BK : tid % BM, ka = TA ? tid % BK : tid / BM;
+  const int nb = TB ? tid % BN : tid / BK, kb = TB ? tid / BN : tid % BK;
+  constexpr int RA = TA ? kThreads / BK : 0, KA = TA ? 0 : kThreads / BM;
+  constexpr int RB = TB ? 0 : kThreads / BK, KB = TB ? kThreads / BN : 0;
+  const float* pa = g.A + (TA ? kbeg + ka + (m0 + ma) * g.lda : m0 + ma + (kbeg + ka) * g.lda);
+  const float* pb = g.B + (TB ? n0 + nb + (kbeg + kb) * g.ldb : kbeg + kb + (n0 + nb) * g.ldb);
+  const int64_t sa = (TA ? RA : KA) * g.lda, sb = (TB ? KB : RB) * g.ldb;
+  const int64_t na = TA ? BK : BK * g.lda, nbs = TB ? BK * g.ldb : BK;  // to the next stage
+  const int mleft = (int)(g.M - m0 < BM ? g.M - m0 : BM);
+  const int nleft = (int)(g.N - n0 < BN ? g.N - n0 : BN);
+  float ra[EA], rb[EB];
+  auto load = [&](int64_t k0) {
+    const int kleft = (int)(kend - k0 < BK ? kend - k0 : BK);
+#pragma unroll
+    for (int e = 0; e < EA; ++e)
+      ra[e] = (ma + RA * e < mleft && ka + KA * e < kleft) ? pa[e * sa] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < EB; ++e)
+      rb[e] = (nb + RB * e < nleft && kb + KB * e < kleft) ? pb[e * sb] : 0.0f;
+    pa += na;
+    pb += nbs;
+  };
+  f4_t acc[TN][TM];
+#pragma unroll
+  for (int a = 0; a < TN; ++a)
+#pragma unroll
+    for (int b = 0; b < TM; ++b) acc[a][b] = f4_t{0, 0, 0, 0};
+  const int wm0 = (wave & 1) * 64, wn0 = (wave >> 1) * (BN / 2);
+  load(kbeg);
+  for (int64_t k0 = kbeg; k0 < kend; k0 += BK) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < EA; ++e) As[ka + KA * e][ma + RA * e] = ra[e];
+#pragma unroll
+    for (int e = 0; e < EB; ++e) Bs[kb + KB * e][nb + RB * e] = rb[e];
+    __syncthreads();
+    if (k0 + BK < kend) load(k0 + BK);
+#pragma unroll
+    for (int s = 0; s < BK / 4; ++s) {
+      float av[TM], bv[TN];
+#pragma unroll
+      for (int a = 0; a < TN; ++a) bv[a] = Bs[4 * s + lk][wn0 + 16 * a + li];
+#pragma unroll
+      for (int b = 0; b < TM; ++b) av[b] = As[4 * s + lk][wm0 + 16 * b + li];
+#pragma unroll
+      for (int a = 0; a < TN; ++a)
+#pragma unroll
+        for (int b = 0; b < TM; ++b) acc[a][b] = Mfma<float>::mma(bv[a], av[b], acc[a][b]);
+    }
+  }
+#pragma unroll
+  for (int a = 0; a < TN; ++a)
+#pragma unroll
+    for (int b = 0; b < TM; ++b) {
+      const int64_t gm = m0 + wm0 + 16 * b + li;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t gn = n0 + wn0 + 16 * a + Mfma<float>::row(lk, e);
+        if (gm >= g.M || gn >= g.N) continue;
+        float* cp = C + gm + gn * g.ldc;
+        const float v = g.alpha * acc[a][b][e];
+        *cp = g.beta != 0.0f ? v + g.beta * *cp : v;
+      }
+    }
+}
+
 // C = sum_z W[z] (+ beta*C), W[z] is M x N with leading dimension M, added in
 // double.  sym: the
 // entries on and above the diagonal, each stored on both sides of it.
@@ -615,6 +705,16 @@ static void gemm_launch_tile(Context* c, int tile, dim3 grid, const GemmArgs<T>&
                        c->stream, g);
 }
 
+template <typename T>
+static int launch_splitk_reduce(Context* c, int64_t M, int64_t N, int splits, const T* work, T beta,
+                                T* C, int64_t ldc, bool sym) {
+  const int64_t blocks = std::min<int64_t>((M * N + 255) / 256, 4096);
+  hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, c->stream, M, N,
+                     splits, work, beta, C, ldc, sym ? 1 : 0);
+  RSVD_LAUNCH_CHECK();
+  return 0;
+}
+
 template <typename T, int SPLIT = 0>
 static int launch_gemm(Context* c, const GemmPlan& pl, char ta, char tb, int64_t M, int64_t N,
                        int64_t K, T alpha, const T* A, int64_t lda, const T* B, int64_t ldb, T beta,
@@ -640,15 +740,65 @@ static int launch_gemm(Context* c, const GemmPlan& pl, char ta, char tb, int64_t
     else gemm_launch_tile<T, true, true, SPLIT>(c, pl.tile, grid, g);
     RSVD_LAUNCH_CHECK();
   }
-  if (pl.splits > 1) {
-    int64_t total = M * N;
-    int blocks = (int)((total + 255) / 256);
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks), dim3(256), 0, c->stream, M, N,
-                       pl.splits, (const T*)work.p, beta, C, ldc, sym ? 1 : 0);
+  return pl.splits > 1 ? launch_splitk_reduce<T>(c, M, N, pl.splits, work.p, beta, C, ldc, sym) : 0;
+}
+
+// The FP32 products of gemm_staged_kernel.  Over 500 products of 0.1 to 200 GFLOP
+// gemm_kernel takes 0.65 to 0.9 of its time below 1 GFLOP and for outputs of few rows, and
+// 0.8 to 0.95 above, but 1.1 to 1.5 times as long where both operands are row-contiguous
+// off the 128-byte lines (N T, odd sizes), or one is in a long k loop, or k is so short
+// that the tail of its 32-deep blocks weighs (46256 x 1611 x 89 290 us, here 230).
+static bool gemm_staged(bool tA, bool tB, int64_t M, int64_t N, int64_t K, int64_t lda,
+                        int64_t ldb) {
+  const int off = (!tA && lda % 32 != 0) + (tB && ldb % 32 != 0);
+  const double flops = 2.0 * (double)M * (double)N * (double)K;
+  if (M < (off == 2 ? 96 : 192) || flops < (K < 100 ? 5e8 : 1e9)) return false;
+  return off == 2 || (off == 1 && K > 10000) || K < 300;
+}
+
+static int launch_gemm_staged(Context* c, const char* tag, bool tA, bool tB, int64_t M, int64_t N,
+                              int64_t K, float alpha, const float* A, int64_t lda, const float* B,
+                              int64_t ldb, float beta, float* C, int64_t ldc) {
+  const int bn = N <= 32 ? 32 : 64;
+  const int64_t gx = (M + 127) / 128, gy = (N + bn - 1) / bn, tiles = gx * gy;
+  // slices for two workgroups a CU, 256 products or more each
+  const int64_t target = 2LL * (c->num_cus > 0 ? c->num_cus : 256);
+  int64_t splits = 1;
+  if (tiles < target && K >= 4 * 256)
+    splits = pick_k_slices(tiles, target, std::min<int64_t>(K / 256, bn == 32 ? 128 : 64));
+  const int64_t kchunk = ((K + splits - 1) / splits + 15) / 16 * 16;
+  splits = (K + kchunk - 1) / kchunk;
+  DBuf<float> work;
+  GemmArgs<float> g{M, N, K, kchunk, alpha, A, lda, B, ldb, beta, C, ldc, 0, nullptr, 0, 0,
+                    (int)gx, (int)gy};
+  if (splits > 1) {
+    RSVD_TRY(work.alloc((size_t)(M * N * splits)));
+    g.C = work.p;
+    g.ldc = M;
+    g.zstride = M * N;
+    g.beta = 0.0f;
+  }
+  {
+    KTimer kt(c, tag);
+    const dim3 grid((unsigned)tiles, (unsigned)splits);
+#define RSVD_STAGED(TA_, TB_)                                                                   \
+  do {                                                                                          \
+    if (bn == 32)                                                                               \
+      hipLaunchKernelGGL((gemm_staged_kernel<TA_, TB_, 32>), grid, dim3(kThreads), 0, c->stream, \
+                         g);                                                                    \
+    else                                                                                        \
+      hipLaunchKernelGGL((gemm_staged_kernel<TA_, TB_, 64>), grid, dim3(kThreads), 0, c->stream, \
+                         g);                                                                    \
+  } while (0)
+    if (!tA && !tB) RSVD_STAGED(false, false);
+    else if (tA && !tB) RSVD_STAGED(true, false);
+    else if (!tA && tB) RSVD_STAGED(false, true);
+    else RSVD_STAGED(true, true);
+#undef RSVD_STAGED
     RSVD_LAUNCH_CHECK();
   }
-  return 0;
+  return splits > 1 ? launch_splitk_reduce<float>(c, M, N, (int)splits, work.p, beta, C, ldc, false)
+                    : 0;
 }
 
 static int check_dims(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
@@ -738,6 +888,10 @@ static int gemm_any(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t 
   // formed and stored on both sides of it
   const bool tA = (ta == 'T' || ta == 't'), tB = (tb == 'T' || tb == 't');
   const bool sym = A == B && lda == ldb && tA != tB && M == N && beta == T(0);
+  if constexpr (sizeof(T) == 4) {
+    if (!sym && gemm_staged(tA, tB, M, N, K, lda, ldb))
+      return launch_gemm_staged(c, tag, tA, tB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  }
   return launch_gemm<T>(c, gemm_plan<T>(c, tA, M, N, K, sym, false), ta, tb, M, N, K, alpha, A, lda, B,
                         ldb, beta, C, ldc, nullptr, sym, tag);
 }

@@ -80,3 +80,28 @@ def test_fp32_sums_stay_short(gpu_lib):
     assert rc == 0, rp.last_error()
     want = A.astype(np.float64) @ B.astype(np.float64)
     assert np.sqrt(np.mean((dC.to_host() / want - 1.0) ** 2)) <= 3e-7
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k,pad", [(4099, 513, 255, 1), (2561, 1000, 257, 3), (70001, 31, 297, 0),
+                                       (9999, 32, 2001, 3), (193, 33, 80011, 1), (97, 200, 30011, 1),
+                                       (7777, 900, 41, 0), (1025, 129, 4099, 1)])
+def test_fp32_staged_products(gpu_lib, m, n, k, pad, ta, tb):
+    """FP32 products of a GFLOP and more: the sizes that stage their operands in LDS (short k, odd
+    row-contiguous operands, long k) and, in the other transpositions, those that do not; edges of
+    the 128-row and 32 / 64-column tiles, of the 16-deep stages and of the k slices."""
+    rp = gpu_lib
+    rng = np.random.default_rng(m)
+    fa, A = _padded(rng, *((m, k) if ta == "N" else (k, m)), pad, np.float32)
+    fb, B = _padded(rng, *((k, n) if tb == "N" else (n, k)), pad, np.float32)
+    fc, C0 = _padded(rng, m, n, pad, np.float32)
+    dA, dB, dC = (rp.DeviceMatrix.from_host(x) for x in (fa, fb, fc))
+    rc = rp.load().rsvd_dev_gemm(1, ta.encode(), tb.encode(), m, n, k, 2.0, dA.ptr, fa.shape[0],
+                                 dB.ptr, fb.shape[0], -0.5, dC.ptr, fc.shape[0])
+    assert rc == 0, rp.last_error()
+    oA, oB = (A if ta == "N" else A.T), (B if tb == "N" else B.T)
+    got = dC.to_host()
+    bound = (k + 4) * np.finfo(np.float32).eps * (2.0 * np.abs(oA) @ np.abs(oB) + np.abs(C0))
+    err = np.abs(got[:m] - (2.0 * oA @ oB - 0.5 * C0))
+    assert np.all(err <= bound), float((err / bound).max())
+    assert np.all(np.isnan(got[m:]))
