@@ -1,30 +1,41 @@
-"""FP64 products of the fixed-rank SVD at odd sizes: matrix rows that straddle cache lines and a
-narrow output, where a cut into one long workgroup a CU waits for its operands.  The rate of the
-fastest of ten calls lies above what such a cut reaches (20 to 26 TFLOP/s) and below what the
-present ones do (32 to 36)."""
+"""Rates of products at odd sizes, whose matrix rows straddle cache lines; the fastest of ten calls."""
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n,k,least", [(4013, 50, 18712, 27.0), (2271, 110, 14730, 30.0),
-                                         (100, 4073, 43721, 29.0)])
-def test_transposed_product_rate(gpu_lib, m, n, k, least):
-    rp = gpu_lib
+def _rate(rp, tag, dtype, ta, tb, m, n, k):
     lib = rp.load()
-    dA, dB, dC = rp.DeviceMatrix(k, m), rp.DeviceMatrix(k, n), rp.DeviceMatrix(m, n)
-    assert lib.rsvd_dev_gaussian(1, k, m, dA.ptr, k) == 0
-    assert lib.rsvd_dev_gaussian(2, k, n, dB.ptr, k) == 0
+    ar, ac = (m, k) if ta == b"N" else (k, m)
+    br, bc = (k, n) if tb == b"N" else (n, k)
+    rng = np.random.default_rng(1)
+    dA = rp.DeviceMatrix.from_host(rng.random((ar, ac), dtype=dtype))
+    dB, dC = rp.DeviceMatrix.from_host(rng.random((br, bc), dtype=dtype)), rp.DeviceMatrix(m, n, dtype)
     best = np.inf
     try:
         for _ in range(10):
             lib.rsvd_kstats_reset()
             lib.rsvd_kstats_enable(1)
-            rc = lib.rsvd_dev_gemm(0, b"T", b"N", m, n, k, 1.0, dA.ptr, k, dB.ptr, k, 0.0, dC.ptr, m)
+            rc = lib.rsvd_dev_gemm(0 if dtype == np.float64 else 1, ta, tb, m, n, k, 1.0, dA.ptr, ar,
+                                   dB.ptr, br, 0.0, dC.ptr, m)
             assert rc == 0, rp.last_error()
-            best = min(best, rp.kstats("gemm_f64")[0])
+            best = min(best, rp.kstats(tag)[0])
     finally:
         lib.rsvd_kstats_enable(0)
         lib.rsvd_kstats_reset()
-    assert 2e-9 * m * n * k / best >= least
+    return 2e-9 * m * n * k / best
+
+
+@pytest.mark.parametrize("m,n,k,least", [(4013, 50, 18712, 27.0), (2271, 110, 14730, 30.0),
+                                         (100, 4073, 43721, 29.0)])
+def test_transposed_product_rate(gpu_lib, m, n, k, least):
+    """FP64 A^T B with a narrow output: a cut into one long workgroup a CU waits for its operands (20
+    to 26 TFLOP/s); the present ones reach 32 to 36."""
+    assert _rate(gpu_lib, "gemm_f64", np.float64, b"T", b"N", m, n, k) >= least
+
+
+@pytest.mark.parametrize("m,n,k", [(50001, 301, 3005), (5001, 2003, 1005)])
+def test_fp32_row_contiguous_rate(gpu_lib, m, n, k):
+    """FP32 A B^T: staged operands reach 80 TFLOP/s and more, fed to registers by each wave 46."""
+    assert _rate(gpu_lib, "gemm_f32", np.float32, b"N", b"T", m, n, k) >= 62.0
