@@ -628,8 +628,8 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
               {0.5, 0.8, 0.8}, 2.0, 1.5e-6, 0.4},
       kF32 = {256.0 / 2400, {{1.1, 1.1, 1.0}, {1.1, 1.1, 1.0}}, {1.6, 1.4, 1.0},
               {0.3, 0.3, 0.3}, 2.0, 5e-7, 0.0},
-      kSplit = {0.13, {{1.0, 1.1, 1.0}, {1.0, 1.1, 1.0}}, {1.2, 2.0, 1.2},
-                {0.3, 0.3, 0.3}, 2.0, 1e-6, 0.0};
+      kSplit = {0.1, {{1.2, 1.05, 1.0}, {0.88, 0.9, 1.0}}, {1.4, 1.3, 1.2},
+                {0.1, 0.1, 0.1}, 2.0, 1e-6, 0.0};
   const CutCost& m = sizeof(T) == 8 ? kF64 : (split == 0 ? kF32 : kSplit);
   constexpr int64_t depth = KBlock<T>::kDepth;
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;

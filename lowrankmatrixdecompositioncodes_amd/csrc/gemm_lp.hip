@@ -390,17 +390,26 @@ __global__ void splitk_reduce_f32_kernel(int64_t M, int64_t N, int splits,
 
 // Products that leave the 128 x 128 tiles and the A-streaming kernel short of
 // workgroups: the small-tile kernel of gemm.hip, which rounds its operands in
-// registers.  Measured before and here, split-bf16: Grams up to 1024 columns
-// always (101 columns of 5003 rows 47 and 9 us, 544 of 65536 194 and 162 us, 256 of
-// 50000 78 and 45 us); others up to 4 GFLOP (1024 x 64 x 512 39 and 6 us, 2000 x 64 x
-// 2000 134 and 14 us, 5003 x 101 x 3001 54 and 47 us).  Past it the operands that
-// the staged tiles share win: 3000 x 3000 x 300 53 us there, 80 us here.
+// registers.  Over 260 products of 0.1 to 4 GFLOP it takes, in split-bf16, 0.6 of the
+// time in the geometric mean and at most 1.03 of it, but for C = A B^T and for wide
+// outputs with a short k (20705 x 249 x 249 N T 79 us against 62, 649 x 6113 x 130 60
+// against 52).  Past 4 GFLOP the operands that the staged tiles share win: 3000 x 3000 x
+// 300 53 us there, 80 us here.  Grams: up to 1024 columns, except where the staged tiles are whole
+// and loaded 16 bytes wide (split-bf16: 512 columns of 65536 rows 150 us here, 141
+// there, 640 220 and 145, 640 of 16384 79 and 74; others 0.5 to 0.9 of the time: 576 of
+// 131072 374 and 530, 1000 of 65536 360 and 574).  A single bf16 product moves the line:
+// 384 columns of 65536 rows 0.9, 512 0.8 of the staged tiles' speed.
 static bool lp_direct(bool tA, bool tB, int64_t M, int64_t N, int64_t K, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float beta, int split) {
   if (split == 6 || M == 0 || N == 0 || K == 0) return false;
   if (M > 65535LL * LBM || N > 65535LL * LBN) return false;  // as the tiled kernel's grid
-  const bool gram = A == B && lda == ldb && tA && !tB && M == N && beta == 0.0f && N <= 1024;
-  return gram || 2.0 * (double)M * (double)N * (double)K <= 4e9;
+  const double flops = 2.0 * (double)M * (double)N * (double)K;
+  if (A == B && lda == ldb && tA && !tB && M == N && beta == 0.0f && N <= 1024) {
+    const bool whole = N % LBN == 0 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0;
+    return !(whole && N >= (split == 1 ? 384 : 512) && flops > (split == 1 ? 1e10 : 2e10));
+  }
+  if (!tA && K <= 320 && flops > 5e8 && (tB || (N > M && K > 64))) return false;
+  return flops <= 4e9;
 }
 
 int gemm_bf16(Context* c, const char* tag, char ta, char tb, int64_t M, int64_t N, int64_t K,

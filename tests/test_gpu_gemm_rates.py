@@ -39,3 +39,25 @@ def test_transposed_product_rate(gpu_lib, m, n, k, least):
 def test_fp32_row_contiguous_rate(gpu_lib, m, n, k):
     """FP32 A B^T: staged operands reach 80 TFLOP/s and more, fed to registers by each wave 46."""
     assert _rate(gpu_lib, "gemm_f32", np.float32, b"N", b"T", m, n, k) >= 62.0
+
+
+@pytest.mark.parametrize("n,k,least", [(640, 65536, 340.0), (512, 131072, 270.0)])
+def test_split_bf16_gram_of_whole_tiles(gpu_lib, n, k, least):
+    """A long split-bf16 Gram whose columns fill the 128-column staged tiles, in TFLOP/s of the full
+    product: 435 and 297 there, 252 and 243 with operands that each wave fetches for itself."""
+    rp = gpu_lib
+    lib = rp.load()
+    A = np.random.default_rng(1).standard_normal((k, n), dtype=np.float32)
+    dA, dG = rp.DeviceMatrix.from_host(A), rp.DeviceMatrix(n, n, np.float32)
+    best = np.inf
+    try:
+        for _ in range(10):
+            lib.rsvd_kstats_reset()
+            lib.rsvd_kstats_enable(1)
+            rc = lib.rsvd_dev_gemm(3, b"T", b"N", n, n, k, 1.0, dA.ptr, k, dA.ptr, k, 0.0, dG.ptr, n)
+            assert rc == 0, rp.last_error()
+            best = min(best, rp.kstats("gemm_bf16")[0])
+    finally:
+        lib.rsvd_kstats_enable(0)
+        lib.rsvd_kstats_reset()
+    assert 2e-9 * n * n * k / best >= least
