@@ -61,6 +61,31 @@ def test_edges(gpu_lib, ta, tb, split):
 
 
 @pytest.mark.parametrize("split", [1, 3])
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k", [(1925, 961, 137), (4489, 323, 144), (559, 910, 2068),
+                                   (723, 1125, 99), (1311, 582, 107), (1113, 109, 1770),
+                                   (1367, 68, 1775)])
+def test_larger_tiles(gpu_lib, m, n, k, ta, tb, split):
+    """The sizes that the small-tile kernel's plan cuts into 128 x 64 (the first three, the third
+    of them in 6 slices: 5, 9 and 47 rows in the last tile) and 64 x 32 tiles (the last two in 7)."""
+    rp = gpu_lib
+    rng = np.random.default_rng(m)
+    fa = _padded(rng, *((m, k) if ta == "N" else (k, m)), 3)
+    fb = _padded(rng, *((k, n) if tb == "N" else (n, k)), 1)
+    fc = _padded(rng, m, n, 1)
+    dA, dB, dC = (rp.DeviceMatrix.from_host(x) for x in (fa, fb, fc))
+    rc = rp.load().rsvd_dev_gemm(2 if split == 1 else 3, ta.encode(), tb.encode(), m, n, k, 2.0,
+                                 dA.ptr, fa.shape[0], dB.ptr, fb.shape[0], -0.5, dC.ptr,
+                                 fc.shape[0])
+    assert rc == 0, rp.last_error()
+    A, B = fa[:-3].astype(np.float64), fb[:-1].astype(np.float64)
+    got = dC.to_host()
+    assert np.all(np.isnan(got[m:]))
+    _check(got[:m], 2.0 * (A if ta == "N" else A.T), B if tb == "N" else B.T,
+           -0.5 * fc[:m].astype(np.float64), split)
+
+
+@pytest.mark.parametrize("split", [1, 3])
 @pytest.mark.parametrize("n", [1000, 1001])
 def test_both_sides_of_the_rule(gpu_lib, n, split):
     rp = gpu_lib

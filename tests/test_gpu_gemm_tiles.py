@@ -1,6 +1,9 @@
-"""FP64 / FP32 products at the edges of the GEMM's tiles (32 and 128 rows, 32 and 64 columns), of
-its k blocks (16 FP64, 32 FP32 elements) and of its k slices, every transposition, Grams
-(A^T A and B B^T, one operand passed twice), and leading dimensions beyond the rows."""
+"""FP64 / FP32 products at the edges of the GEMM's tiles, of its k blocks (16 FP64, 32 FP32
+elements) and of its k slices, every transposition, Grams (A^T A and B B^T, one operand passed
+twice), and leading dimensions beyond the rows.  SHAPES and the Grams are cut into 32 x 32 tiles
+(a few workgroups); LARGE are the sizes that the cut's model gives 128 x 64 and 64 x 32 tiles."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -8,6 +11,23 @@ pytestmark = pytest.mark.gpu
 
 SHAPES = [(1, 1, 1), (31, 33, 15), (32, 32, 16), (33, 31, 17), (127, 64, 31), (128, 65, 32),
           (129, 63, 33), (64, 1, 4097), (1, 64, 700), (400, 26, 200), (257, 300, 1000)]
+
+# (m, n, k) and what the plan cuts it into, with A not transposed where A^T is not named
+LARGE = [(945, 1223, 68),     # FP64 128 x 64: a last tile of 49 rows leaves two of its waves idle
+         (949, 1242, 68),     # FP64 128 x 64, A^T
+         (659, 786, 1818),    # FP64 128 x 64 in 6 slices: one wave of the last tile has 19 rows
+         (4129, 46, 2988),    # FP64 128 x 64, A^T, 15 slices: less than a tile's columns
+         (2435, 202, 53),     # FP64 64 x 32: a last tile of 3 rows and 10 columns
+         (2843, 176, 49),     # FP64 64 x 32, A^T: 1 of a k block's 16 left over
+         (2059, 37, 1256),    # FP64 64 x 32 in 7 slices
+         (2253, 41, 1734),    # FP64 64 x 32, A^T, 7 slices
+         (2181, 714, 138),    # FP32 128 x 64: a last tile of 5 rows
+         (2739, 605, 136),    # FP32 128 x 64, A^T
+         (118, 2061, 2388),   # FP32 128 x 64 in 15 slices: less than a tile's rows
+         (723, 1125, 99),     # FP32 64 x 32
+         (1669, 497, 105),    # FP32 64 x 32, A^T
+         (4683, 35, 1775),    # FP32 64 x 32 in 5 slices
+         (4571, 41, 1251)]    # FP32 64 x 32, A^T, 5 slices
 
 
 def _padded(rng, rows, cols, pad, dtype):
@@ -41,6 +61,52 @@ def test_gemm_edges(gpu_lib, ta, tb, dtype):
         err = np.abs(got[:m] - (2.0 * oA @ oB + beta * C0))
         assert np.all(err <= bound), (m, n, k, float((err / bound).max()))
         assert np.all(np.isnan(got[m:]))
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("T", "N"), ("N", "T"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k", LARGE)
+def test_larger_tiles(gpu_lib, m, n, k, ta, tb, dtype):
+    rp = gpu_lib
+    rng = np.random.default_rng(m)
+    fa, A = _padded(rng, *((m, k) if ta == "N" else (k, m)), 3, dtype)
+    fb, B = _padded(rng, *((k, n) if tb == "N" else (n, k)), 1, dtype)
+    fc, C0 = _padded(rng, m, n, 1, dtype)
+    dA, dB, dC = (rp.DeviceMatrix.from_host(x) for x in (fa, fb, fc))
+    rc = rp.load().rsvd_dev_gemm(0 if dtype == np.float64 else 1, ta.encode(), tb.encode(), m, n, k,
+                                 2.0, dA.ptr, fa.shape[0], dB.ptr, fb.shape[0], -0.5, dC.ptr,
+                                 fc.shape[0])
+    assert rc == 0, rp.last_error()
+    oA, oB = (A if ta == "N" else A.T), (B if tb == "N" else B.T)
+    got = dC.to_host()
+    bound = (k + 4) * np.finfo(dtype).eps * (2.0 * np.abs(oA) @ np.abs(oB) + np.abs(C0))
+    err = np.abs(got[:m] - (2.0 * oA @ oB - 0.5 * C0))
+    assert np.all(err <= bound), float((err / bound).max())
+    assert np.all(np.isnan(got[m:]))
+
+
+@pytest.mark.parametrize("m,n,kstep", [(1937, 1999, 67), (1300, 331, 20)])
+def test_deflation_norm(gpu_lib, m, n, kstep):
+    """A <- A - Q B with the sum of squares of the result taken in the same launch, in 128 x 64
+    (first size: a last tile of 17 rows and 15 columns, three of its waves idle) and 32 x 32 tiles.
+    A tolerance that the first block meets ends the adaptive QB there and returns that norm."""
+    rp = gpu_lib
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((m, n))
+    nstep = -(-min(m, n) // kstep)
+    dA = rp.DeviceMatrix.from_host(A)
+    dQ, dB = rp.DeviceMatrix(m, kstep * nstep), rp.DeviceMatrix(kstep * nstep, n)
+    fr, norm = C.c_int(0), C.c_double(0)
+    rc = rp.load().rsvd_dev_randqb(dA.ptr, m, n, m, kstep, 0, 1e9, 0, 1, 1, 5, None, dQ.ptr, m,
+                                   dB.ptr, kstep * nstep, C.byref(fr), C.byref(norm))
+    assert rc == 0, rp.last_error()
+    assert fr.value == kstep
+    Q, B = dQ.to_host()[:, :kstep], dB.to_host()[:kstep]
+    eps = np.finfo(np.float64).eps
+    # an entry's error, here and there, and 4096 roundings in any one chain of the sum of squares
+    each = 2.0 * (kstep + 4) * eps * (np.abs(Q) @ np.abs(B) + np.abs(A))
+    want = np.linalg.norm(A - Q @ B)
+    assert abs(norm.value - want) <= np.linalg.norm(each) + 4096 * eps * want
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
