@@ -3,9 +3,10 @@
 // low_rank_svd_rand_decomp_fixed_rank, rra.c:73-234, vnum = 2: the reference
 // would loop over the matrices one call at a time).
 //
-// Every stage of the algorithm is one launch over the whole batch; a call is
-// a fixed sequence of about a dozen launches, captured once into a hipGraph
-// per batch layout and replayed:
+// Every step of the algorithm is one launch over the whole batch; a call is
+// a fixed sequence of 14 + 12 (q - 1) launches (26 at q = 2: an
+// orthonormalisation takes five, the final stage four), captured once into a
+// hipGraph per batch layout and replayed:
 //   bomega   Omega_i (n_i x l_i) from the seeded stream, seed + i, into Z_i
 //   btile    the skinny operand (Omega / Z / Q, K x 48) rounded to split bf16
 //            (hi, lo) in MFMA fragment order (as in apass.hip)
@@ -1178,7 +1179,7 @@ int fixed_rank_batched(Context* c, int count, const int* m, const int* n, const 
     snprintf(buf, sizeof buf,
              "rt_nn=%d rt_tn=%d (NN ms %.3f/%.3f/%.3f/%.3f, TN ms %.3f/%.3f/%.3f/%.3f for RT "
              "1/2/4/4 with k split over 4 waves (%d)); "
-             "one launch each: orth Y %.3f ms, orth Z %.3f ms, final %.3f ms, tile %.3f ms",
+             "each stage once: orth Y %.3f ms, orth Z %.3f ms, final %.3f ms, tile %.3f ms",
              P->rt_nn, P->rt_tn, P->tuned_ms[0][0], P->tuned_ms[0][1], P->tuned_ms[0][2],
              P->tuned_ms[0][3], P->tuned_ms[1][0], P->tuned_ms[1][1], P->tuned_ms[1][2],
              P->tuned_ms[1][3], kRtSplitK, P->stage_ms[0],

@@ -882,6 +882,8 @@ static int gemm_any(Context* c, char ta, char tb, int64_t M, int64_t N, int64_t 
     RSVD_LAUNCH_CHECK();
     return 0;
   }
+  // no limit of the grid's (its x counts every tile, under 2^24 of them for any matrix that
+  // fits the memory); more columns have always been refused
   if (N > 32 && (N + 63) / 64 > 65535)
     return set_error("gemm: N=%lld too large for the grid", (long long)N);
   // A^T A or B B^T with beta = 0: the entries on and above the diagonal are

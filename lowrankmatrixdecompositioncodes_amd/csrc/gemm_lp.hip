@@ -402,7 +402,8 @@ __global__ void splitk_reduce_f32_kernel(int64_t M, int64_t N, int splits,
 static bool lp_direct(bool tA, bool tB, int64_t M, int64_t N, int64_t K, const float* A,
                       int64_t lda, const float* B, int64_t ldb, float beta, int split) {
   if (split == 6 || M == 0 || N == 0 || K == 0) return false;
-  if (M > 65535LL * LBM || N > 65535LL * LBN) return false;  // as the tiled kernel's grid
+  // left to the staged tiles, whose grid.y refuses the longer side past 65535 tiles
+  if (M > 65535LL * LBM || N > 65535LL * LBN) return false;
   const double flops = 2.0 * (double)M * (double)N * (double)K;
   if (A == B && lda == ldb && tA && !tB && M == N && beta == 0.0f && N <= 1024) {
     const bool whole = N % LBN == 0 && lda % 4 == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0;

@@ -106,6 +106,8 @@ int svd_from_Q_f64(Context* c, const double* A, int64_t m, int64_t n, int64_t ld
   RSVD_TRY(sig.alloc((size_t)l));
   RSVD_TRY(gemm_f64_tag(c, "apass_f64", 'T', 'N', l, n, m, 1.0, Q, ldq, A, lda, 0.0, B.p, l));
   RSVD_TRY(gemm_f64(c, 'N', 'T', l, l, n, 1.0, B.p, l, B.p, l, 0.0, G.p, l));
+  // gemm_kernel's B B^T is symmetric as it is; the vendor product that a large one takes
+  // under rsvd_set_fp64_vendor_gemm is not
   hipLaunchKernelGGL(symmetrize_upper_kernel, dim3(grid1(l * l)), dim3(256), 0, c->stream, l, G.p);
   RSVD_LAUNCH_CHECK();
   int sw = 0;

@@ -855,6 +855,8 @@ symtri_values_kernel(int n, const double* __restrict__ G, int64_t ldg, double* _
     double s = 1.0;
 #pragma unroll 4
     for (int i = 0; i < n; ++i) {
+      // one Newton step: the quotient's error (about 2^-48 of it) shifts the eigenvalues as
+      // the same change of e2 would, by 4e-15 of the norm
       double r = __builtin_amdgcn_rcp(s);
       r = fma(r, fma(-s, r, 1.0), r);
       s = fma(-e2[i], r, dd[i] - x);
