@@ -632,6 +632,15 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
                 {0.1, 0.1, 0.1}, 2.0, 1e-6, 0.0};
   const CutCost& m = sizeof(T) == 8 ? kF64 : (split == 0 ? kF32 : kSplit);
   constexpr int64_t depth = KBlock<T>::kDepth;
+  // Large tall A^T B: 32 x 32 tiles fetch half as much again as 64 x 32 ones, and their
+  // reads reach what the memory gives (16384 x 544 x 65536: 7.5 TB/s).  From 40 GFLOP on 36
+  // products take 0.88 of the time that way in the geometric mean (0.68 to 1.2; 16384 x 544 x
+  // 65536 22.1 ms, now 19.4, 4987 x 576 x 18539 2.64 and 1.80).  Not with one narrow ragged
+  // column of tiles (12001 x 101 x 40003 2.48 and 2.88 ms) nor fewer rows than columns.
+  static const double kTallSlow[3] = {1.0, 1.04, 1.08};
+  const bool tall = sizeof(T) == 8 && ka && !sym && M >= N && (N % 32 == 0 || N >= 288) &&
+                    2.0 * (double)M * (double)N * (double)K > 4e10;
+  const double* slow = tall ? kTallSlow : m.slow[ka];
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
   int64_t room = kMaxSliceElems / (M * N);
@@ -679,7 +688,7 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
       if ((kblocks + kb - 1) / kb != s && s > smin) continue;  // as with a smaller s
       const double rounds = (double)((tiles * s + cus - 1) / cus);
       const double blocks = (double)((kb + d.ks - 1) / d.ks);
-      double wave = blocks * d.blocks * m.block * m.slow[ka][t];
+      double wave = blocks * d.blocks * m.block * slow[t];
       if (blocks > 96) wave *= 1.0 + m.drift * std::min(1.0, std::log2(blocks / 96.0));
       double cost = std::max(rounds, m.alone[t]) * wave + rounds * m.group[t];
       if (s > 1) cost += m.launch + m.elem * (double)s * (double)M * (double)N;

@@ -35,6 +35,13 @@ def test_transposed_product_rate(gpu_lib, m, n, k, least):
     assert _rate(gpu_lib, "gemm_f64", np.float64, b"T", b"N", m, n, k) >= least
 
 
+@pytest.mark.parametrize("m,n,k,least", [(4987, 576, 18539, 49.0), (36655, 384, 3765, 51.0)])
+def test_large_transposed_product_rate(gpu_lib, m, n, k, least):
+    """FP64 A^T B past 40 GFLOP with a tall output: 32 x 32 tiles reach 40 and 47 TFLOP/s (their
+    reads take all that the memory gives), 64 x 32 ones 57 and 58."""
+    assert _rate(gpu_lib, "gemm_f64", np.float64, b"T", b"N", m, n, k) >= least
+
+
 @pytest.mark.parametrize("m,n,k", [(50001, 301, 3005), (5001, 2003, 1005)])
 def test_fp32_row_contiguous_rate(gpu_lib, m, n, k):
     """FP32 A B^T: staged operands reach 80 TFLOP/s and more, fed to registers by each wave 46."""
