@@ -612,6 +612,8 @@ struct CutCost {
 // and MFMAs alone it chose one workgroup a CU with a long loop too often, above all
 // for odd sizes, whose rows straddle cache lines: A^T B at 4013 x 50 x 18712 373 us,
 // now 235, at 2271 x 110 x 14730 279 and 205 us, at 100 x 4073 x 43721 1478 and 998 us.
+// Slices cost their second launch: 4 us in a chain of small FP64 products (three slices
+// for 26 x 26 x 400 and 200 x 26 x 400 saved 2 us of their kernels' 7).
 // The slices hold at most kMaxSliceElems elements: what they save on a larger output,
 // part of a last round of workgroups, is not worth the memory.  In an allocation-free
 // call they are also no more than the largest free range of the scratch array holds: a
@@ -625,7 +627,7 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
   } kTiles[3] = {{128, 64, 1, 8}, {64, 32, 4, 8}, {32, 32, 4, 4}};
   static const CutCost
       kF64 = {256.0 / 2400, {{1.1, 1.1, 1.13}, {1.26, 1.26, 1.1}}, {1.3, 2.0, 1.1},
-              {0.5, 0.8, 0.8}, 2.0, 1.5e-6, 0.4},
+              {0.5, 0.8, 0.8}, 4.0, 1.5e-6, 0.4},
       kF32 = {256.0 / 2400, {{1.1, 1.1, 1.0}, {1.1, 1.1, 1.0}}, {1.6, 1.4, 1.0},
               {0.3, 0.3, 0.3}, 2.0, 5e-7, 0.0},
       kSplit = {0.1, {{1.2, 1.05, 1.0}, {0.88, 0.9, 1.0}}, {1.4, 1.3, 1.2},

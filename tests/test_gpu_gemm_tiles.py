@@ -15,11 +15,11 @@ SHAPES = [(1, 1, 1), (31, 33, 15), (32, 32, 16), (33, 31, 17), (127, 64, 31), (1
 # (m, n, k) and what the plan cuts it into, with A not transposed where A^T is not named
 LARGE = [(945, 1223, 68),     # FP64 128 x 64: a last tile of 49 rows leaves two of its waves idle
          (949, 1242, 68),     # FP64 128 x 64, A^T
-         (659, 786, 1818),    # FP64 128 x 64 in 6 slices: one wave of the last tile has 19 rows
+         (4247, 34, 1881),    # FP64 128 x 64 in 15 slices: one wave of the last tile has 23 rows
          (4129, 46, 2988),    # FP64 128 x 64, A^T, 15 slices: less than a tile's columns
          (2435, 202, 53),     # FP64 64 x 32: a last tile of 3 rows and 10 columns
          (2843, 176, 49),     # FP64 64 x 32, A^T: 1 of a k block's 16 left over
-         (2059, 37, 1256),    # FP64 64 x 32 in 7 slices
+         (1785, 40, 1669),    # FP64 64 x 32 in 9 slices
          (2253, 41, 1734),    # FP64 64 x 32, A^T, 7 slices
          (2181, 714, 138),    # FP32 128 x 64: a last tile of 5 rows
          (2739, 605, 136),    # FP32 128 x 64, A^T
