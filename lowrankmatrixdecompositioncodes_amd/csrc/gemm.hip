@@ -18,12 +18,14 @@
 //  * An operand stored k-contiguous is loaded eight full lines a time and
 //    transposed to lane order through a region of LDS of the wave's own
 //    (loaded in lane order it would take 16 half lines a load: 50 TF against
-//    61 TF for A^T B at 6000 x 288 x 16384).
-// Measured (FP64, best cut; the former kernel staged 128 x 64 tiles through one
-// LDS buffer with two barriers a slice): 16384 x 288 x 6000 N N 49 -> 67 TF,
-// A^T B as above 35 -> 61 TF, 2000 x 110 x 1000 39 -> 15 us, a 110 x 110 Gram of
-// 2000 rows 40 -> 9 us.  The large ones are bound by the MFMAs (71 TF at the
-// clock a large product reaches), the small ones by latency.
+//    60 TF for A^T B at 6000 x 288 x 16384).
+// Measured (FP64, the kernel's own time; the former kernel staged 128 x 64 tiles
+// through one LDS buffer with two barriers a slice): 16384 x 288 x 6000 N N 29 ->
+// 60 TF, A^T B as above 40 -> 60 TF, 2000 x 110 x 1000 112 -> 17 us, a 110 x 110
+// Gram of 2000 rows 38 -> 8 us.  The large ones are bound by the MFMAs (71 TF at
+// the clock a large product reaches) and, where A outgrows the caches, by reading
+// it again (gemm_plan); the small ones by latency.  FP32 products that read too
+// much this way take a staged kernel (gemm_staged).
 // Operand lane layout of the 16x16x4 MFMAs (per 64-lane wave):
 //   srcA: lane l holds X[i = l%16][k = l/16]
 //   srcB: lane l holds Y[k = l/16][j = l%16]
