@@ -638,7 +638,7 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
   constexpr int64_t depth = KBlock<T>::kDepth;
   // Large tall A^T B: 32 x 32 tiles fetch half as much again as 64 x 32 ones, and their
   // reads reach what the memory gives (16384 x 544 x 65536: 7.5 TB/s).  From 40 GFLOP on 36
-  // products take 0.88 of the time that way in the geometric mean (0.68 to 1.2; 16384 x 544 x
+  // products take 0.89 of the time that way in the geometric mean (0.68 to 1.2; 16384 x 544 x
   // 65536 22.1 ms, now 19.4, 4987 x 576 x 18539 2.64 and 1.80).  Not with one narrow ragged
   // column of tiles (12001 x 101 x 40003 2.48 and 2.88 ms) nor fewer rows than columns.
   static const double kTallSlow[3] = {1.0, 1.04, 1.08};
