@@ -636,15 +636,19 @@ static GemmPlan gemm_plan(Context* c, bool ka, int64_t M, int64_t N, int64_t K, 
                 {0.1, 0.1, 0.1}, 2.0, 1e-6, 0.0};
   const CutCost& m = sizeof(T) == 8 ? kF64 : (split == 0 ? kF32 : kSplit);
   constexpr int64_t depth = KBlock<T>::kDepth;
-  // Large tall A^T B: 32 x 32 tiles fetch half as much again as 64 x 32 ones, and their
-  // reads reach what the memory gives (16384 x 544 x 65536: 7.5 TB/s).  From 40 GFLOP on 36
-  // products take 0.89 of the time that way in the geometric mean (0.68 to 1.2; 16384 x 544 x
-  // 65536 22.1 ms, now 19.4, 4987 x 576 x 18539 2.64 and 1.80).  Not with one narrow ragged
-  // column of tiles (12001 x 101 x 40003 2.48 and 2.88 ms) nor fewer rows than columns.
-  static const double kTallSlow[3] = {1.0, 1.04, 1.08};
-  const bool tall = sizeof(T) == 8 && ka && !sym && M >= N && (N % 32 == 0 || N >= 288) &&
-                    2.0 * (double)M * (double)N * (double)K > 4e10;
-  const double* slow = tall ? kTallSlow : m.slow[ka];
+  // Large A^T B: 32 x 32 tiles fetch half as much again as 64 x 32 ones, and their reads
+  // reach what the memory gives (16384 x 544 x 65536 in FP64: 7.5 TB/s).  With constants
+  // of their own, FP64 from 40 GFLOP on: 36 products take 0.89 of the time in the geometric
+  // mean (0.68 to 1.2; 16384 x 544 x 65536 22.1 ms, now 19.4, 4987 x 576 x 18539 2.64 and
+  // 1.80).  Not with one narrow ragged column of tiles (12001 x 101 x 40003 2.48 and 2.88 ms)
+  // nor fewer rows than columns.  FP32 from 20 GFLOP on: 40 products 0.5 to 1.02 of the time
+  // (256 x 10180 x 85045 8.96 and 4.92 ms, 65867 x 760 x 10522 15.8 and 10.9).
+  static const double kLargeSlow[3] = {1.0, 1.04, 1.08};
+  const double flops = 2.0 * (double)M * (double)N * (double)K;
+  const bool large = ka && !sym && split == 0 &&
+                    (sizeof(T) == 8 ? flops > 4e10 && M >= N && (N % 32 == 0 || N >= 288)
+                                    : flops > 2e10);
+  const double* slow = large ? kLargeSlow : m.slow[ka];
   const int64_t cus = c->num_cus > 0 ? c->num_cus : 256;
   const int64_t kblocks = (K + depth - 1) / depth;
   int64_t room = kMaxSliceElems / (M * N);
